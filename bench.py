@@ -9,7 +9,7 @@ Prints ONE JSON line (rank 0).  `value` = primary probe rays per second of whole
 Mrays/s, over `--steps` updates enqueued back to back (no timing events, no host wait between
 them); `phases_ms` come from a second pass over the same updates with per-phase HIP events.
 `roofline` describes the kernel with the largest share of the step: its algorithmic bytes come from
-the traversal's own fetch counters (128-byte 4-wide nodes, 48-byte triangles) of an untimed
+the traversal's own fetch counters (80-byte 4-wide nodes, 48-byte triangles) of an untimed
 counting update, set against the HBM peak; `traffic` (bytes leaving L2 per launch, from the
 committed rocprofv3 counter summary) shows how few of them reach HBM, and `cache_ceiling` is the
 fastest device copy that stays in L2 / the Infinity Cache, measured in the same run.
@@ -569,7 +569,7 @@ def main():
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "traffic_source": os.path.relpath(PROFILE_SUMMARY, ROOT),
                 "algorithmic_bytes_per_launch": int(dk["algorithmic_bytes"]), "avg_ms": round(dk["ms"], 4),
-                "algorithmic_bytes_definition": "per primary ray: 128 B per 4-wide node fetched + 48 B per triangle "
+                "algorithmic_bytes_definition": "per primary ray: 80 B per 4-wide node fetched + 48 B per triangle "
                                                 "fetched (the traversal's own fetch counters) + the 16 B hit record"}
     for k, v in kernels.items():
         v["algorithmic_GB/s"] = round(v["algorithmic_bytes"] / (v["ms"] * 1e-3) / 1e9, 1)
@@ -588,8 +588,8 @@ def main():
         roofline["traffic_frac_of_peak"] = round(tr_gbs / HBM_PEAK_GBS, 4)
         roofline["fetched_bytes_beyond_L2"] = round(traffic / dk["algorithmic_bytes"], 4)
     if dom == "trace_primary":
-        roofline["limiter"] = ("latency of dependent node fetches under lane divergence: a wavefront runs until its "
-                               "longest ray ends (VALU lane utilisation in the profile summary), not HBM bandwidth")
+        roofline["limiter"] = ("vector instruction issue under lane divergence: a wavefront runs until its longest ray "
+                               "ends (VALU lane utilisation in the profile summary), not HBM bandwidth")
         roofline["frac_note"] = ("achieved counts every lane's node and triangle fetches, most of them served by L1, L2 "
                                  "and the Infinity Cache, so frac can pass 1; traffic_frac_of_peak is the HBM share")
     if peaks:

@@ -678,13 +678,15 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	std::vector<float> mats(material_count * 12);
 	for(size_t k = 0; k < material_count; ++k) std::memcpy(&mats[k * 12], &materials[k], 48);
 	const float4* nodes = nullptr;
+	const float4* boxes = nullptr;
 	const float4* tris = nullptr;
 	const InstanceDev* ip = nullptr;
 	const uint32_t* op = nullptr;
 	const uint32_t* ixp = nullptr;
 	const float4* vp = nullptr;
 	const float* mp = nullptr;
-	if((st = upload(h, reinterpret_cast<const float4*>(bvh.nodes.data()), bvh.nodes.size() / 4, &nodes)) != DDGI_OK ||
+	if((st = upload(h, reinterpret_cast<const float4*>(bvh.nodes.data()), bvh.nodes.size() / 4, &boxes)) != DDGI_OK ||
+	   (st = upload<float4>(h, nullptr, size_t(bvh.node_count) * (kPackedNodeBytes / 16), &nodes)) != DDGI_OK ||
 	   (st = upload(h, reinterpret_cast<const float4*>(bvh.tris.data()), bvh.tris.size() / 4, &tris)) != DDGI_OK ||
 	   (st = upload(h, inst.data(), inst.size(), &ip)) != DDGI_OK ||
 	   (st = upload(h, reinterpret_cast<const uint32_t*>(offsets), offset_count * 3, &op)) != DDGI_OK ||
@@ -714,7 +716,16 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	h->instances.assign(instances, instances + instance_count);
 	h->build_xf.resize(instance_count * 12);
 	for(size_t k = 0; k < instance_count; ++k) std::memcpy(&h->build_xf[k * 12], instances[k].transform, 48);
+	{  // the traversal's nodes, ready for any stream
+		hipError_t e = launch_pack_nodes(boxes, const_cast<float4*>(nodes), bvh.node_count, nullptr);
+		if(e == hipSuccess) e = hipStreamSynchronize(nullptr);
+		if(e != hipSuccess) {
+			free_scene(h);
+			return fail(h, DDGI_ERROR_HIP, std::string("packing the BVH nodes: ") + hipGetErrorString(e));
+		}
+	}
 	sd.nodes = nodes;
+	sd.boxes = const_cast<float4*>(boxes);
 	sd.tris = tris;
 	sd.inst = ip;
 	sd.offsets = op;
@@ -780,11 +791,12 @@ ddgi_status ddgi_update_instances(void* handle, uint32_t first, uint32_t count, 
 							  hipMemcpyHostToDevice, s));
 	HIP_TRY(h, hipMemcpyAsync(h->rel_xf + size_t(first) * 12, rel, size_t(count) * 48, hipMemcpyHostToDevice, s));
 	float4* tris = const_cast<float4*>(h->sd.tris);
-	float4* nodes = const_cast<float4*>(h->sd.nodes);
+	float4* nodes = h->sd.boxes;
 	HIP_TRY(h, launch_retransform(tris, h->obj_tris, h->sd.tri_count, h->move_xf, h->move_meta, first, count, s));
 	const std::vector<uint32_t>& lv = h->bvh_meta.level_offsets;
 	for(size_t d = lv.size() - 1; d >= 1; --d)
 		HIP_TRY(h, launch_refit_level(nodes, tris, h->slot_box, h->rel_xf, h->level_nodes + lv[d - 1], lv[d] - lv[d - 1], s));
+	HIP_TRY(h, launch_pack_nodes(nodes, const_cast<float4*>(h->sd.nodes), h->sd.node_count, s));
 	// the staging area and move_xf / move_meta are reused once this has run
 	HIP_TRY(h, hipEventRecord(h->move_done, s));
 	h->move_pending = true;

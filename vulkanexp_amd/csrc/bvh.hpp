@@ -2,7 +2,7 @@
 // (src/Renderer.cpp:272-449, :525-642).  Instances are flattened into world space at build time,
 // so traversal is single-level.
 //
-// Device layout (all float4 / 16-byte aligned, read with 128-bit loads):
+// Device layout (all float4 / 16-byte aligned, accessed 16 bytes at a time):
 //   node k  : kNodeFloats floats, a kWide-wide node collapsed from the binary SAH tree, holding the
 //             boxes of its (up to) kWide children side by side so that one node fetch tests all of
 //             them, in rows of kWide floats (one float4 per 4 children):
@@ -16,6 +16,8 @@
 //               [0] = (v0.xyz, global triangle id)   global id = instance-major flattened index
 //               [1] = (v1.xyz, instance index)
 //               [2] = (v2.xyz, mask | flip_facing << 8)
+// The traversal reads the nodes in a packed form made on the device (k_pack_nodes, kPackedNodeBytes each,
+// the same node indices and child codes); these full-precision ones are what a refit updates.
 // Node boxes are inflated by a few ulps so that FP32 slab tests stay conservative; an empty child
 // slot has the code kEmptyChild and a point box far outside any scene.
 #pragma once
@@ -37,6 +39,7 @@ constexpr uint32_t kNodeFloats = kWide == 4 ? 32 : 64;  // 6 box rows + 1 code r
 constexpr uint32_t kCodeRow = 6 * kWide;               // float offset of the child codes
 constexpr uint32_t kMaxWideDepth = 32;   // traversal stack: kWide - 1 entries per level
 static_assert(kWide == 4 || kWide == 8, "nodes are 4- or 8-wide");
+constexpr uint32_t kPackedNodeBytes = 80;  // the traversal's form of a 4-wide node (trace.hip, k_pack_nodes)
 
 struct BvhHost {
 	std::vector<float> nodes;     // kNodeFloats per node

@@ -112,22 +112,6 @@ __device__ __forceinline__ bool tri_intersect(const RayPrep& r, float4 a, float4
 	return t >= tmin && t <= tmax;
 }
 
-// Conservative slab test of one child box: [tn, tf] clipped to [tmin, tmax], far end widened by
-// a few ulps (robust traversal, Ize 2013); boxes are also inflated at build time.  The planes come
-// as the near and far plane of each axis for this ray (lo where 1/d is positive, hi where it is
-// negative): (p - o) / d rounds monotonically in p, so the near plane's distance is the smaller of
-// the two and no min / max pair per axis is needed.  With d = +-0 the distances are infinite and
-// the test keeps the box whenever the origin lies within its slab.
-__device__ __forceinline__ bool slab(const RayPrep& r, float nx, float fx, float ny, float fy, float nz, float fz,
-									 float tmin, float tmax, float& tn) {
-	const float xn = (nx - r.o[0]) * r.inv[0], xf = (fx - r.o[0]) * r.inv[0];
-	const float yn = (ny - r.o[1]) * r.inv[1], yf = (fy - r.o[1]) * r.inv[1];
-	const float zn = (nz - r.o[2]) * r.inv[2], zf = (fz - r.o[2]) * r.inv[2];
-	tn = fmaxf(fmaxf(xn, yn), fmaxf(zn, tmin));
-	const float tf = fminf(fminf(xf, yf), fminf(zf, tmax));
-	return tn <= tf * 1.000001f;
-}
-
 struct HitResult {
 	float t;
 	uint32_t slot;  // triangle position in the BVH triangle array, 0xFFFFFFFF = miss
@@ -138,29 +122,43 @@ struct HitResult {
 
 // Closest-hit (ANY = false; ties -> lowest global id) or any-hit traversal of the BVH.
 //
-// Nodes are 4-wide (bvh.hpp): one 128-byte fetch tests four child boxes.  The children the ray
-// enters are sorted by entry distance (a five-comparator network on registers); the nearest is
-// visited next and the others are pushed farthest first, so the next pop is the nearest remaining.
-// The result does not depend on the visiting order: closest hit is the minimum of (t, global id)
-// over every triangle the conservative box tests let through.
+// Nodes are 4-wide, in the packed form of k_pack_nodes: five 16-byte loads test four child boxes.  A
+// wavefront runs until its longest ray ends with about a third of its lanes active, so what bounds the
+// traversal is what a visit costs per wavefront: vector instructions (79 % of the SIMDs' issue cycles
+// with FP32 boxes) and vector loads, whose data return costs about 22 cycles per load of the CU however
+// few lanes are active (75 % of its cycles with the seven loads of an FP32 node).  Cutting one of them
+// alone moved nothing; the packed node cuts both: a plane's distance is one v_fma_mix_f32 on the FP16
+// plane (distance = q * (scale / d) + (origin - o) / d), and two loads fewer are returned.  The near and
+// far plane rows are chosen by the sign of 1/d (which is the smaller distance, since the distance is
+// monotonic in the plane), so no min / max pair is needed, and the far end is widened by a few ulps
+// (robust traversal, Ize 2013).  With d = +-0 the distances are infinite or NaN; maxima and minima drop
+// the NaNs, so such a box is kept.
 //
-// Stack: the newest STACK entries live in an LDS ring laid out [entry][thread] (conflict-free;
-// `stack` points at this thread's column, `stride` is the block size); when the ring is full its
-// oldest entry moves to a private spill array, and pops drain the ring first, then the spill, so
-// the order stays LIFO.  At most kWide - 1 entries per level of the wide tree are pending, and
-// STACK + kSpill covers the deepest tree accepted (kMaxWideDepth levels), while the LDS footprint
-// stays small enough for full occupancy.
+// The children the ray enters are sorted by entry distance (a five-comparator network on registers;
+// sorting only the nearest, or leaving the middle pair, visits more and took 0.64 / 0.66 ms against
+// 0.58 in the large workload's primary pass); the nearest is visited next and the others are pushed
+// farthest first, so the next pop is the nearest remaining.  The result does not depend on the visiting
+// order: closest hit is the minimum of (t, global id) over every triangle the conservative box tests
+// let through.
+//
+// Stack: entries 0 .. STACK - 1 live in LDS laid out [entry][thread] (conflict-free; `stack` points at
+// this thread's column, STRIDE is the block size), later ones in a private array.  Entry 0 is a
+// sentinel, so that a pop needs no test for an empty stack; with three entries free in the LDS part
+// the three pushes of a visit are unconditional stores with a conditional advance.  At most kWide - 1
+// entries per level of the wide tree are pending.  12 LDS entries measured fastest (8 / 12 / 16 / 22:
+// 0.605 / 0.574 / 0.580 / 0.629 ms): more LDS per workgroup keeps fewer of them on a CU.
+//
+// Large workload (4.2 M rays), primary pass: FP32 nodes with a ring stack 0.674 ms; packed nodes and
+// this stack 0.575 ms at 7 waves per SIMD, 0.555 ms at 8, which its 64 registers now allow.
 //
 // Leaves are tested two triangles at a time, each triangle's 48 bytes loaded in one go, so that
 // two loads are in flight and the mask word costs no extra round trip.
 //
-// With COUNT, n_nodes / n_tris receive the number of node (kNodeFloats * 4 bytes) and 48-byte
-// triangle fetches
-// (the algorithmic bytes of the traversal).
-constexpr int kLdsStack = 16;  // LDS ring entries per thread
-// private spill entries: kLdsStack + kSpill = (kWide - 1) * kMaxWideDepth
-constexpr int kSpill = (int(kWide) - 1) * int(kMaxWideDepth) - kLdsStack;
-static_assert(kLdsStack + kSpill >= (int(kWide) - 1) * int(kMaxWideDepth), "traversal stack too small for the deepest tree");
+// With COUNT, n_nodes / n_tris receive the number of node (kPackedNodeBytes) and 48-byte triangle
+// fetches (the algorithmic bytes of the traversal).
+constexpr int kLdsStack = 12;  // LDS entries per thread
+// entries beyond them, in a private array; one entry is the bottom's sentinel
+constexpr int kStackMax = (int(kWide) - 1) * int(kMaxWideDepth) + 1;
 
 // CULL: back-facing triangles are ignored (rasterizer back-face culling).
 template <bool ANY, bool CULL>
@@ -182,40 +180,26 @@ __device__ __forceinline__ bool test_triangle(const RayPrep& r, float tmin, uint
 	return true;
 }
 
-template <bool ANY, int STACK, bool COUNT = false, bool CULL = false>
+template <bool ANY, int STACK, int STRIDE, bool COUNT = false, bool CULL = false>
 __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, const float4* __restrict__ tris,
 											  const RayPrep& r, float tmin, float tmax, uint32_t mask,
-											  uint32_t* stack, int stride, uint32_t& n_nodes_out, uint32_t& n_tris_out) {
-	static_assert((STACK & (STACK - 1)) == 0, "the LDS ring size must be a power of two");
+											  uint32_t* stack, uint32_t& n_nodes_out, uint32_t& n_tris_out) {
+	static_assert(kWide == 4, "packed nodes are 4-wide");
 	HitResult best;
 	best.t = tmax;
 	best.slot = 0xFFFFFFFFu;
 	best.gid = 0xFFFFFFFFu;
 	best.meta = 0u;
 	best.V = best.W = best.det = 0.0f;
-	uint32_t spill[kSpill];
-	int head = 0, count = 0, nspill = 0;  // ring write position, ring entries, spilled entries
-// pop into `v`, or run `on_empty` when ring and spill are both empty
-#define DDGI_STACK_POP(v, on_empty)                    \
-	if(count > 0) {                                    \
-		head = (head - 1) & (STACK - 1);               \
-		--count;                                       \
-		v = stack[head * stride];                      \
-	} else if(nspill > 0) {                            \
-		v = spill[--nspill];                           \
-	} else {                                           \
-		on_empty;                                      \
-	}
-// push `v`; when the ring is full its oldest entry (at `head`) moves to the spill array first
-#define DDGI_STACK_PUSH(v)                             \
-	{                                                  \
-		if(count == STACK) {                           \
-			spill[nspill++] = stack[head * stride];    \
-			--count;                                   \
-		}                                              \
-		stack[head * stride] = (v);                    \
-		head = (head + 1) & (STACK - 1);               \
-		++count;                                       \
+	uint32_t spill[kStackMax - STACK];
+	constexpr uint32_t kNone = 0xFFFFFFFFu;  // no node (the stack's bottom) / no postponed leaf
+	stack[0] = kNone;
+	int sp = 1;  // stack entries
+#define DDGI_STACK_POP(v)                                                        \
+	{                                                                            \
+		--sp;                                                                    \
+		if(sp < STACK) v = stack[sp * STRIDE];                                   \
+		else v = spill[sp - STACK];                                              \
 	}
 // order (key, code) pairs i, j by key
 #define DDGI_CSWAP(i, j)                               \
@@ -232,105 +216,76 @@ __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, 
 	// it in `leaf` and goes on descending from its stack until at least half of the active lanes of
 	// the wavefront hold a leaf (or it has run out of nodes); the wavefront then tests leaves
 	// together.  Waiting for every lane idles the lanes that hold one; testing at once idles the
-	// others; half measured fastest (the probe update's primary pass 0.92 ms when waiting for all,
-	// 0.86 ms at a half; an eighth 0.90, three quarters 0.89).  Closest hit is the minimum of
-	// (t, global id) over all triangles, so the order changes no result.
-	constexpr uint32_t kNone = 0xFFFFFFFFu;  // no node (empty stack) / no postponed leaf
+	// others; half measured fastest (three, five and six eighths: 0.587 / 0.590 / 0.597 ms against
+	// 0.580).
 	uint32_t node = 0;  // root (always an inner node)
 	uint32_t leaf = kNone;
 	uint32_t n_nodes = 0, n_tris = 0;
 	const float kInf = __int_as_float(0x7f800000);
-	// byte offset in a node of this ray's near plane row per axis (rows lo.x, hi.x, lo.y, hi.y, lo.z,
-	// hi.z): the near plane is lo where 1/d is positive (sign bit clear), hi where not; the far row
-	// is the other one of the pair, its offset the near one's with bit kRowBytes flipped (a node
-	// starts at a multiple of 4 rows)
-	constexpr uint32_t kRowBytes = 16u * (kWide / 4u);
-	uint32_t near_off[3];
-#pragma unroll
-	for(int a = 0; a < 3; ++a) near_off[a] = kRowBytes * (2u * uint32_t(a) + (__float_as_uint(r.inv[a]) >> 31));
+	const bool neg[3] = {(__float_as_uint(r.inv[0]) >> 31) != 0u, (__float_as_uint(r.inv[1]) >> 31) != 0u,
+						 (__float_as_uint(r.inv[2]) >> 31) != 0u};
 	const char* __restrict__ node_bytes = reinterpret_cast<const char*>(nodes);
+	typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 	for(;;) {
 		// descend through inner nodes
 		while(!(node & kLeafFlag)) {
 			// 32-bit offsets from the array's base (the node array stays far below 4 GiB)
-			const uint32_t node_off = node * uint32_t(kNodeFloats * 4);
-			constexpr int G = int(kWide) / 4;  // float4s per row
-			float bx[6][kWide];  // near x, far x, near y, far y, near z, far z
-			uint32_t code[kWide];
+			const float4* nd = reinterpret_cast<const float4*>(node_bytes + node * kPackedNodeBytes);
+			const float4 h = nd[0], px = nd[1], py = nd[2], pz = nd[3], cd = nd[4];
+			++n_nodes;
+			uint32_t code[4] = {__float_as_uint(cd.x), __float_as_uint(cd.y), __float_as_uint(cd.z), __float_as_uint(cd.w)};
+			float tn[4], tf[4];
 #pragma unroll
-			for(int row = 0; row < 6; ++row) {
-				const uint32_t near = node_off + near_off[row >> 1];
-				const uint32_t off = (row & 1) ? near ^ kRowBytes : near;
+			for(int ax = 0; ax < 3; ++ax) {
+				const float4 pl = ax == 0 ? px : (ax == 1 ? py : pz);
+				const float org = ax == 0 ? h.x : (ax == 1 ? h.y : h.z);
+				const float A = h.w * r.inv[ax], B = (org - r.o[ax]) * r.inv[ax];
+				const uint32_t n01 = __float_as_uint(neg[ax] ? pl.z : pl.x), n23 = __float_as_uint(neg[ax] ? pl.w : pl.y);
+				const uint32_t f01 = __float_as_uint(neg[ax] ? pl.x : pl.z), f23 = __float_as_uint(neg[ax] ? pl.y : pl.w);
+				const half2_t qn[2] = {__builtin_bit_cast(half2_t, n01), __builtin_bit_cast(half2_t, n23)};
+				const half2_t qf[2] = {__builtin_bit_cast(half2_t, f01), __builtin_bit_cast(half2_t, f23)};
 #pragma unroll
-				for(int g = 0; g < G; ++g) {
-					const float4 v = *reinterpret_cast<const float4*>(node_bytes + (off + 16u * uint32_t(g)));
-					bx[row][4 * g] = v.x;
-					bx[row][4 * g + 1] = v.y;
-					bx[row][4 * g + 2] = v.z;
-					bx[row][4 * g + 3] = v.w;
+				for(int k = 0; k < 4; ++k) {
+					const float en = __builtin_fmaf(float(qn[k >> 1][k & 1]), A, B), ef = __builtin_fmaf(float(qf[k >> 1][k & 1]), A, B);
+					tn[k] = ax == 0 ? en : fmaxf(tn[k], en);
+					tf[k] = ax == 0 ? ef : fminf(tf[k], ef);
 				}
 			}
+			// entry distance of each child the ray enters, infinity for the others
+			float key[4];
 #pragma unroll
-			for(int g = 0; g < G; ++g) {
-				const float4 v = *reinterpret_cast<const float4*>(node_bytes + (node_off + kRowBytes * 6u + 16u * uint32_t(g)));
-				code[4 * g] = __float_as_uint(v.x);
-				code[4 * g + 1] = __float_as_uint(v.y);
-				code[4 * g + 2] = __float_as_uint(v.z);
-				code[4 * g + 3] = __float_as_uint(v.w);
-			}
-			++n_nodes;
-			// entry distance of each child the ray enters, infinity for the others (slab distances are
-			// finite or clipped to [tmin, tmax], so a finite key is an entered child)
-			float key[kWide];
-#pragma unroll
-			for(int k = 0; k < int(kWide); ++k) {
-				float tn;
-				key[k] = (slab(r, bx[0][k], bx[1][k], bx[2][k], bx[3][k], bx[4][k], bx[5][k], tmin, best.t, tn) &&
-						  code[k] != kEmptyChild)
-							 ? tn
-							 : kInf;
+			for(int k = 0; k < 4; ++k) {
+				const float n = fmaxf(tn[k], tmin), f = fminf(tf[k], best.t);
+				key[k] = n <= f * 1.000001f ? n : kInf;
 			}
 			// sorted by key, the entered children come first
-			{
-				if constexpr(kWide == 4) {
-					DDGI_CSWAP(0, 1)
-					DDGI_CSWAP(2, 3)
-					DDGI_CSWAP(0, 2)
-					DDGI_CSWAP(1, 3)
-					DDGI_CSWAP(1, 2)
-				} else {  // Batcher's odd-even merge network for 8 keys (19 comparators)
-					DDGI_CSWAP(0, 1)
-					DDGI_CSWAP(2, 3)
-					DDGI_CSWAP(4, 5)
-					DDGI_CSWAP(6, 7)
-					DDGI_CSWAP(0, 2)
-					DDGI_CSWAP(1, 3)
-					DDGI_CSWAP(4, 6)
-					DDGI_CSWAP(5, 7)
-					DDGI_CSWAP(1, 2)
-					DDGI_CSWAP(5, 6)
-					DDGI_CSWAP(0, 4)
-					DDGI_CSWAP(1, 5)
-					DDGI_CSWAP(2, 6)
-					DDGI_CSWAP(3, 7)
-					DDGI_CSWAP(2, 4)
-					DDGI_CSWAP(3, 5)
-					DDGI_CSWAP(1, 2)
-					DDGI_CSWAP(3, 4)
-					DDGI_CSWAP(5, 6)
+			DDGI_CSWAP(0, 1)
+			DDGI_CSWAP(2, 3)
+			DDGI_CSWAP(0, 2)
+			DDGI_CSWAP(1, 3)
+			DDGI_CSWAP(1, 2)
+			// push the others, farthest first; within the LDS part every slot is written and the stack
+			// grows by those that were entered
+			if(sp <= STACK - 3) {
+#pragma unroll
+				for(int k = 3; k >= 1; --k) {
+					stack[sp * STRIDE] = code[k];
+					sp += key[k] != kInf ? 1 : 0;
+				}
+			} else {
+#pragma unroll
+				for(int k = 3; k >= 1; --k) {
+					if(key[k] == kInf) continue;
+					if(sp < STACK) stack[sp * STRIDE] = code[k];
+					else spill[sp - STACK] = code[k];
+					++sp;
 				}
 			}
-			if(key[0] == kInf) {
-				DDGI_STACK_POP(node, node = kNone)
-			} else {
-				node = code[0];
-#pragma unroll
-				for(int k = int(kWide) - 1; k >= 1; --k)
-					if(key[k] != kInf) DDGI_STACK_PUSH(code[k])
-			}
+			node = code[0];
+			if(key[0] == kInf) DDGI_STACK_POP(node)
 			if(leaf == kNone && node != kNone && (node & kLeafFlag)) {  // postpone the leaf
 				leaf = node;
-				DDGI_STACK_POP(node, node = kNone)
+				DDGI_STACK_POP(node)
 			}
 			// at least half of the active lanes hold a leaf
 			if(uint32_t(__popcll(__ballot(leaf != kNone))) * 2u >= uint32_t(__popcll(__ballot(true)))) break;
@@ -356,14 +311,13 @@ __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, 
 			leaf = kNone;
 			if(node != kNone && (node & kLeafFlag)) {
 				leaf = node;
-				DDGI_STACK_POP(node, node = kNone)
+				DDGI_STACK_POP(node)
 			}
 		}
 		if(node == kNone) break;
 	}
 done:
 #undef DDGI_STACK_POP
-#undef DDGI_STACK_PUSH
 #undef DDGI_CSWAP
 	if(COUNT) {
 		n_nodes_out = n_nodes;

@@ -56,7 +56,8 @@ struct InstanceDev {
 };
 
 struct SceneDev {
-	const float4* nodes;
+	const float4* nodes;       // the traversal's packed nodes (kPackedNodeBytes each)
+	float4* boxes;             // the same nodes with FP32 boxes (kNodeFloats each), which refits update
 	const float4* tris;
 	const InstanceDev* inst;
 	const uint32_t* offsets;   // 3 per entry (material, vertex offset, index offset)
@@ -246,6 +247,8 @@ hipError_t launch_trace_rays(const SceneDev& sc, const ddgi_ray* rays, ddgi_hit*
 // build, 3x4).
 hipError_t launch_retransform(float4* tris, const float* obj, uint32_t tri_count, const float* xf, const uint32_t* meta,
 							  uint32_t first, uint32_t count, hipStream_t s);
+// Traversal nodes (kPackedNodeBytes each) of `count` wide nodes.
+hipError_t launch_pack_nodes(const float4* nodes, float4* packed, uint32_t count, hipStream_t s);
 hipError_t launch_refit_level(float4* nodes, const float4* tris, const float* slot_box, const float* rel_xf,
 							  const uint32_t* level_nodes, uint32_t count, hipStream_t s);
 hipError_t launch_gbuffer(const SceneDev& sc, const ddgi_ray* rays, uint64_t count, ddgi_gbuffer_texel* out, hipStream_t s);

@@ -157,8 +157,8 @@ __device__ __forceinline__ void finish_primary_ray(const TraceFrameArgs& a, uint
 
 // Traversal thread `gtid` = slot * n + j traces ray perm[j] of the probe in `slot`; `stack` is the
 // thread's column of an LDS stack with `stride` columns.
-template <int STACK, bool COUNT>
-__device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint32_t gtid, uint32_t* stack, int stride) {
+template <int STACK, int STRIDE, bool COUNT>
+__device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint32_t gtid, uint32_t* stack) {
 	const uint32_t n = a.grid.n;
 	const uint32_t slot = gtid / n, j = gtid - slot * n;
 	if(slot >= *a.count) return;
@@ -169,8 +169,8 @@ __device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint3
 	RayPrep r;
 	ray_prepare(o[0], o[1], o[2], d.x, d.y, d.z, r);
 	uint32_t nn = 0, nt = 0;
-	const HitResult h = traverse<false, STACK, COUNT>(a.scene.nodes, a.scene.tris, r, 0.01f, a.grid.tmax_primary,
-													  DDGI_MASK_STATIC | DDGI_MASK_DYNAMIC, stack, stride, nn, nt);
+	const HitResult h = traverse<false, STACK, STRIDE, COUNT>(a.scene.nodes, a.scene.tris, r, 0.01f, a.grid.tmax_primary,
+															  DDGI_MASK_STATIC | DDGI_MASK_DYNAMIC, stack, nn, nt);
 	const uint32_t key = a.shade_keys ? cell_key(a.grid, o[0] + h.t * d.x, o[1] + h.t * d.y, o[2] + h.t * d.z, a.key_shift)
 									  : 0u;
 	finish_primary_ray(a, slot * n + j, h, key);  // thread order: coalesced stores
@@ -181,11 +181,11 @@ __device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint3
 }
 
 template <int STACK, bool COUNT>
-// seven waves per SIMD (72 VGPRs): the occupancy at which the traversal ran fastest, 5 to 8 measured
-__global__ __launch_bounds__(kPrimaryBlock) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_trace_primary(TraceFrameArgs a) {
+// eight waves per SIMD (64 VGPRs, no spills): 0.559 ms, against 0.580 at 7 and 0.617 at 6
+__global__ __launch_bounds__(kPrimaryBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_primary(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kPrimaryBlock];
-	trace_primary_ray<STACK, COUNT>(a, xcd_remap(blockIdx.x, gridDim.x) * kPrimaryBlock + threadIdx.x,
-									stack + threadIdx.x, kPrimaryBlock);
+	trace_primary_ray<STACK, kPrimaryBlock, COUNT>(a, xcd_remap(blockIdx.x, gridDim.x) * kPrimaryBlock + threadIdx.x,
+												   stack + threadIdx.x);
 }
 
 // ---- closest-hit shading + shadow ray (closesthit.glsl:143-289) ----
@@ -208,8 +208,7 @@ template <int STACK, bool COUNT>
 __device__ __forceinline__ SurfaceShade shade_surface(const SceneDev& sc, const GridConst& grid, const LightConst& light,
 													  const uint32_t* states, const float4* irr, const float2* dep,
 													  const float o[3], Vec3 d, float t, uint32_t tslot, float b1,
-													  float b2, uint32_t* stack, int stride,
-													  unsigned long long* visit_counters) {
+													  float b2, uint32_t* stack, unsigned long long* visit_counters) {
 	SurfaceShade r;
 	const float b0 = 1.0f - b1 - b2;
 	const Vec3 position = v3(d.x * t + o[0], d.y * t + o[1], d.z * t + o[2]);
@@ -219,7 +218,7 @@ __device__ __forceinline__ SurfaceShade shade_surface(const SceneDev& sc, const 
 	RayPrep sr;
 	ray_prepare(position.x, position.y, position.z, light.dir[0], light.dir[1], light.dir[2], sr);
 	uint32_t nn = 0, nt = 0;
-	const HitResult sh = traverse<true, STACK, COUNT>(sc.nodes, sc.tris, sr, 0.1f, 10000.0f, 0xFFu, stack, stride, nn, nt);
+	const HitResult sh = traverse<true, STACK, kShadeBlock, COUNT>(sc.nodes, sc.tris, sr, 0.1f, 10000.0f, 0xFFu, stack, nn, nt);
 	if(COUNT) {
 		atomicAdd(&visit_counters[2], (unsigned long long)nn);
 		atomicAdd(&visit_counters[3], (unsigned long long)nt);
@@ -500,7 +499,7 @@ __global__ __launch_bounds__(1024) void k_sort_fine(SortJobs J) {
 // every lane of a wave shades and casts a shadow ray.  Each ray's result depends only on its own
 // record: the order of the list does not change any output.
 template <int STACK, bool COUNT>
-__device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, uint32_t* stack, int stride) {
+__device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, uint32_t* stack) {
 	if(k >= a.shade_count[kShadeTotalSlot]) return;
 	const uint32_t n = a.grid.n;
 	const uint32_t ri = a.shade_list[k];  // hits and rays are stored in thread (ray_order) order
@@ -514,7 +513,7 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, u
 	const float4 d4 = a.dirs[i];
 	const SurfaceShade r = shade_surface<STACK, COUNT>(a.scene, a.grid, a.light, a.states, a.irr, a.dep, o,
 														v3(d4.x, d4.y, d4.z), t, code & 0x7FFFFFFFu, hit.z, hit.w, stack,
-														stride, a.visit_counters);
+														a.visit_counters);
 	a.rays[ri] = make_float4(r.color.x, r.color.y, r.color.z, t);
 	if(a.factors) {
 		// affine decomposition in (albedo, light radiance) for non-metallic materials
@@ -547,7 +546,7 @@ template <int STACK, bool COUNT>
 __global__ __launch_bounds__(kShadeBlock, 6) void k_shade(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
-	if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x, kShadeBlock);
+	if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x);
 }
 
 // ---- misses under the atmospheric sky (miss.rmiss:17-23 with sky.glsl:60-127) ----
@@ -601,9 +600,9 @@ __global__ __launch_bounds__(kMaxRays) void k_batch_begin(BatchLaunch b) {
 // Persistent primary traversal over the work items of all volumes: each workgroup takes the next
 // item (a run of consecutive traversal threads of one volume) from a queue until the queue is
 // empty.  Every workgroup leaves once the head passes the item count, so the grid always drains.
-// five waves per SIMD (96 VGPRs, no spills beyond the traversal's private stack)
+// seven waves per SIMD (72 VGPRs): 2.79 ms for 21.9 M rays of 20 volumes, against 2.88 at 5, 2.82 at 6, 2.90 at 8
 template <int STACK, int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 5))) void k_batch_trace(BatchLaunch b) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_batch_trace(BatchLaunch b) {
 	__shared__ uint32_t stack[STACK * BLOCK];
 	__shared__ uint32_t s_item;
 	uint32_t* head = &b.ctl->next[0];
@@ -619,7 +618,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5, 5))) v
 		const BatchVolume& v = b.vols[vol];
 		const uint32_t end = min(first + b.trace_item_threads, v.threads);
 		for(uint32_t g = first + threadIdx.x; g < end; g += BLOCK)
-			trace_primary_ray<STACK, false>(v.trace, g, stack + threadIdx.x, BLOCK);
+			trace_primary_ray<STACK, BLOCK, false>(v.trace, g, stack + threadIdx.x);
 	}
 }
 
@@ -631,7 +630,7 @@ __global__ __launch_bounds__(kShadeBlock, 6) void k_batch_shade(BatchLaunch b) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t vol = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].volume);
 	const uint32_t first = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].first);
-	shade_ray<STACK, false>(b.vols[vol].trace, first + threadIdx.x, stack + threadIdx.x, kShadeBlock);
+	shade_ray<STACK, false>(b.vols[vol].trace, first + threadIdx.x, stack + threadIdx.x);
 }
 
 // ---- arbitrary ray queries (public ddgi_hit records) ----
@@ -645,8 +644,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays(SceneDev sc, const d
 	RayPrep r;
 	ray_prepare(q.origin[0], q.origin[1], q.origin[2], q.direction[0], q.direction[1], q.direction[2], r);
 	uint32_t nn, nt;
-	const HitResult h = traverse<ANY, STACK, false, CULL>(sc.nodes, sc.tris, r, q.tmin, q.tmax, mask, stack + threadIdx.x,
-														   kTraceBlock, nn, nt);
+	const HitResult h = traverse<ANY, STACK, kTraceBlock, false, CULL>(sc.nodes, sc.tris, r, q.tmin, q.tmax, mask,
+																		stack + threadIdx.x, nn, nt);
 	ddgi_hit out;
 	if(h.slot == 0xFFFFFFFFu) {
 		out.t = -1.0f;
@@ -682,8 +681,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(7, 
 	RayPrep r;
 	ray_prepare(q.origin[0], q.origin[1], q.origin[2], q.direction[0], q.direction[1], q.direction[2], r);
 	uint32_t nn, nt;
-	const HitResult h = traverse<false, STACK, false, true>(sc.nodes, sc.tris, r, q.tmin, q.tmax, 0xFFu,
-															 stack + threadIdx.x, kTraceBlock, nn, nt);
+	const HitResult h = traverse<false, STACK, kTraceBlock, false, true>(sc.nodes, sc.tris, r, q.tmin, q.tmax, 0xFFu,
+																		  stack + threadIdx.x, nn, nt);
 	ddgi_gbuffer_texel g;
 	if(h.slot == 0xFFFFFFFFu) {  // depth 0; the normal slot carries the ray direction (for the sky)
 		for(int k = 0; k < 3; ++k) {
@@ -776,8 +775,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_gather(GatherArgs a) {
 			RayPrep sr;
 			ray_prepare(position.x, position.y, position.z, sd.x, sd.y, sd.z, sr);
 			uint32_t nn, nt;
-			const HitResult sh = traverse<true, STACK>(a.scene.nodes, a.scene.tris, sr, 0.01f, 10000.0f, 0xFFu,
-														stack + threadIdx.x, kTraceBlock, nn, nt);
+			const HitResult sh = traverse<true, STACK, kTraceBlock>(a.scene.nodes, a.scene.tris, sr, 0.01f, 10000.0f, 0xFFu,
+														stack + threadIdx.x, nn, nt);
 			if(sh.slot == 0xFFFFFFFFu) {
 				visible = 1.0f;
 				if(sd.y < 0.0f) visible *= 1.0f - fminf(fmaxf(-sd.y, 0.0f), 0.1f) / 0.1f;
@@ -828,8 +827,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_direct_light(DirectLightArgs a)
 			RayPrep sr;
 			ray_prepare(g.position[0], g.position[1], g.position[2], dir.x, dir.y, dir.z, sr);
 			uint32_t nn, nt;
-			const HitResult sh = traverse<true, STACK>(a.scene.nodes, a.scene.tris, sr, 0.01f, 10000.0f, 0xFFu,
-														stack + threadIdx.x, kTraceBlock, nn, nt);
+			const HitResult sh = traverse<true, STACK, kTraceBlock>(a.scene.nodes, a.scene.tris, sr, 0.01f, 10000.0f, 0xFFu,
+														stack + threadIdx.x, nn, nt);
 			float vis = 0.0f;
 			if(sh.slot == 0xFFFFFFFFu) {
 				vis = 1.0f;
@@ -896,8 +895,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_reflection_trace(ReflectionArgs
 		RayPrep r;
 		ray_prepare(o[0], o[1], o[2], dir.x, dir.y, dir.z, r);
 		uint32_t nn, nt;
-		const HitResult h = traverse<false, STACK>(a.scene.nodes, a.scene.tris, r, 0.1f, 10000.0f, 0xFFu,
-													stack + threadIdx.x, kTraceBlock, nn, nt);
+		const HitResult h = traverse<false, STACK, kTraceBlock>(a.scene.nodes, a.scene.tris, r, 0.1f, 10000.0f, 0xFFu,
+													stack + threadIdx.x, nn, nt);
 		const float4 hit = pack_hit(h);
 		const uint32_t code = __float_as_uint(hit.y);
 		Vec3 c = v3(0.0f, 0.0f, 0.0f);
@@ -937,11 +936,83 @@ __global__ __launch_bounds__(kShadeBlock, 5) void k_reflection_shade(ReflectionA
 		const float4 hit = a.hits[local];
 		const float o[3] = {g.position[0], g.position[1], g.position[2]};
 		const Vec3 c = shade_surface<STACK, false>(a.scene, a.grid, a.light, a.states, a.irr, a.dep, o, dir, hit.x,
-												   __float_as_uint(hit.y), hit.z, hit.w, stack + threadIdx.x, kShadeBlock,
-												   nullptr)
+												   __float_as_uint(hit.y), hit.z, hit.w, stack + threadIdx.x, nullptr)
 						   .color;
 		a.out[id] = compress_reflection(c, g.roughness);
 	}
+}
+
+// ---- traversal nodes ----
+// The traversal's 80-byte form of a wide node (one thread per node): the origin and scale of the
+// node's grid (scale a power of two), the children's planes as FP16 integers 0..2047 on it, rounded
+// outward, in rows x, y, z of (lo of 4 children, hi of 4 children), and the child codes (80 bytes where
+// FP32 boxes take 128; 11 bits keep the boxes tight enough that no more nodes are visited).  A plane is
+// origin + q * scale; the traversal's distance fma(q, scale / d, (origin - o) / d) is off by at most
+// about 2.4e-7 of the node's size (in position) beside the errors relative to the distance that the
+// far end's widening covers, so the boxes are first grown by 1e-6 of that size.  An empty child gets
+// an inverted box, which no ray enters; a node too large for the grid gets infinite ones.
+__global__ void k_pack_nodes(const float4* __restrict__ nodes, float4* __restrict__ packed, uint32_t count) {
+	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	if(i >= count) return;
+	const float4* src = nodes + size_t(i) * (kNodeFloats / 4);
+	float lo[3][4], hi[3][4];
+#pragma unroll
+	for(int a = 0; a < 3; ++a) {
+		const float4 l = src[2 * a], h = src[2 * a + 1];
+		lo[a][0] = l.x, lo[a][1] = l.y, lo[a][2] = l.z, lo[a][3] = l.w;
+		hi[a][0] = h.x, hi[a][1] = h.y, hi[a][2] = h.z, hi[a][3] = h.w;
+	}
+	const float4 cd = src[6];
+	const uint32_t code[4] = {__float_as_uint(cd.x), __float_as_uint(cd.y), __float_as_uint(cd.z), __float_as_uint(cd.w)};
+	double mn[3], mx[3], size = 0.0;
+#pragma unroll
+	for(int a = 0; a < 3; ++a) {
+		mn[a] = 1e300;
+		mx[a] = -1e300;
+#pragma unroll
+		for(int k = 0; k < 4; ++k) {
+			if(code[k] == kEmptyChild) continue;
+			mn[a] = fmin(mn[a], double(lo[a][k]));
+			mx[a] = fmax(mx[a], double(hi[a][k]));
+		}
+		size = fmax(size, mx[a] - mn[a]);
+	}
+	const double slack = size * 1e-6;
+	float org[3];
+	double ext = 0.0;
+#pragma unroll
+	for(int a = 0; a < 3; ++a) {
+		org[a] = float(mn[a] - slack);
+		if(double(org[a]) > mn[a] - slack) org[a] = nextafterf(org[a], -__int_as_float(0x7f800000));
+		ext = fmax(ext, mx[a] + slack - double(org[a]));
+	}
+	const bool fits = ext < 1e37;  // false for infinite extents too
+	// the smallest power of two with 2047 steps over the extent
+	uint32_t sb = __float_as_uint(float(ext * (1.000001 / 2047.0)));
+	sb = (sb + 0x007FFFFFu) & 0x7F800000u;
+	const float scale = fits ? __uint_as_float(sb) : 1.0f;
+	const double inv = 1.0 / double(scale);
+	float4* dst = reinterpret_cast<float4*>(reinterpret_cast<char*>(packed) + size_t(i) * kPackedNodeBytes);
+	dst[0] = fits ? make_float4(org[0], org[1], org[2], scale) : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
+	typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+	const _Float16 inf = __builtin_bit_cast(_Float16, (unsigned short)0x7C00);
+#pragma unroll
+	for(int a = 0; a < 3; ++a) {
+		half4_t q[2];
+#pragma unroll
+		for(int k = 0; k < 4; ++k) {
+			const double l = floor((double(lo[a][k]) - slack - double(org[a])) * inv);
+			const double h = ceil((double(hi[a][k]) + slack - double(org[a])) * inv);
+			const bool empty = code[k] == kEmptyChild;
+			q[0][k] = empty ? _Float16(65504.0f) : (fits ? _Float16(float(fmin(fmax(l, 0.0), 2047.0))) : _Float16(-inf));
+			q[1][k] = empty ? _Float16(-65504.0f) : (fits ? _Float16(float(fmin(fmax(h, 0.0), 2047.0))) : inf);
+		}
+		struct Row {
+			half4_t lo, hi;
+		} row{q[0], q[1]};
+		dst[1 + a] = __builtin_bit_cast(float4, row);
+	}
+	dst[4] = cd;
 }
 
 // ---- instance moves (the TLAS instance update + refit of src/Renderer.cpp:671-742) ----
@@ -1085,8 +1156,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_init_probes(SceneDev sc, GridCo
 		RayPrep r;
 		ray_prepare(o[0], o[1], o[2], d.x, d.y, d.z, r);
 		uint32_t nn, nt;
-		const HitResult h = traverse<false, STACK>(sc.nodes, sc.tris, r, 0.01f, tmax, DDGI_MASK_STATIC, stack + threadIdx.x,
-												   kTraceBlock, nn, nt);
+		const HitResult h = traverse<false, STACK, kTraceBlock>(sc.nodes, sc.tris, r, 0.01f, tmax, DDGI_MASK_STATIC, stack + threadIdx.x, nn, nt);
 		const float depth = (h.slot == 0xFFFFFFFFu) ? 3.402823466e+38f : h.t;
 		if(depth < max_distance) {
 			const bool is_back = (h.det < 0.0f) != ((h.meta & 0x100u) != 0u);
@@ -1309,6 +1379,12 @@ hipError_t launch_retransform(float4* tris, const float* obj, uint32_t tri_count
 	if(tri_count == 0 || count == 0) return hipSuccess;
 	hipLaunchKernelGGL(k_retransform, dim3(blocks_for(tri_count, 256)), dim3(256), 0, s, tris, obj, tri_count, xf, meta,
 					   first, count);
+	return hipGetLastError();
+}
+
+hipError_t launch_pack_nodes(const float4* nodes, float4* packed, uint32_t count, hipStream_t s) {
+	if(count == 0) return hipSuccess;
+	hipLaunchKernelGGL(k_pack_nodes, dim3(blocks_for(count, 128)), dim3(128), 0, s, nodes, packed, count);
 	return hipGetLastError();
 }
 
