@@ -1030,11 +1030,14 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	const uint32_t max_items = uint32_t(P + (N + kDiffChunk - 1) / kDiffChunk);
 	DiffArgs d{};
 	float4* factors = nullptr;
-	float *pos, *nrm, *toc, *out, *loss_part, *g_T;
-	uint32_t *gmat, *states, *indices, *cell_id, *cell_count, *cell_start, *cursor, *cell_item_start, *item_cell,
-		*item_begin, *item_count, *n_items, *sorted;
+	float *pos, *nrm, *toc, *loss_part, *g_T;
+	float4* rec = nullptr;
+	uint32_t *gmat, *states, *indices;
+	DiffBins bins{};
+	// texels of a cell ordered by their first colour tap, unless the keys' counters grow too large
+	bins.taps = P <= (uint64_t(1) << 18) ? 64u : 1u;
 	float2* dep;
-	long long *part_tile, *part_mat_pix, *part_mat_ray;
+	long long *part_tile, *part_mat_pix, *part_mat_ray, *part_rows;
 	hipError_t e = diff_alloc(h, &factors, rays * 4 * sizeof(float4));
 	if(e == hipSuccess) e = diff_alloc(h, &D.rad, rays * sizeof(float4));
 	if(e == hipSuccess) e = diff_alloc(h, &D.prev, P * 64 * sizeof(float4));
@@ -1050,23 +1053,23 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	if(e == hipSuccess) e = diff_alloc(h, &nrm, N * 12);
 	if(e == hipSuccess) e = diff_alloc(h, &toc, N * 12);
 	if(e == hipSuccess) e = diff_alloc(h, &gmat, N * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &out, N * 12);
+	if(e == hipSuccess && N <= kDiffRecords) e = diff_alloc(h, &rec, N * kDiffRecRows * sizeof(float4));
 	D.loss_parts = uint32_t((N + 255) / 256);
 	if(e == hipSuccess) e = diff_alloc(h, &loss_part, size_t(D.loss_parts) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &cell_id, N * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &cell_count, P * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &cell_start, (P + 1) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &cursor, P * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &cell_item_start, (P + 1) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &item_cell, size_t(max_items) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &item_begin, size_t(max_items) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &item_count, size_t(max_items) * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &n_items, 4);
-	if(e == hipSuccess) e = diff_alloc(h, &sorted, N * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.key_of, N * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.key_count, P * bins.taps * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.key_start, P * bins.taps * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.cursor, P * bins.taps * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.cell_item_start, (P + 1) * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.item_begin, size_t(max_items) * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.item_count, size_t(max_items) * 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.n_items, 4);
+	if(e == hipSuccess) e = diff_alloc(h, &bins.sorted, N * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &part_tile, size_t(max_items) * 8 * 192 * 8);
 	if(e == hipSuccess) e = diff_alloc(h, &part_mat_pix, size_t(max_items) * M * 3 * 8);
 	if(e == hipSuccess) e = diff_alloc(h, &g_T, P * 108 * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &part_mat_ray, P * (M * 3 + 3) * 8);
+	if(e == hipSuccess) e = diff_alloc(h, &part_rows, size_t(kDiffSumBlocks) * (M * 3 + 3) * 8);
 	if(e != hipSuccess) {
 		free_diff(h);
 		return fail(h, e == hipErrorOutOfMemory ? DDGI_ERROR_OUT_OF_MEMORY : DDGI_ERROR_HIP,
@@ -1111,22 +1114,25 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	d.gmat = gmat;
 	d.N = N;
 	d.M = uint32_t(M);
-	d.sorted = sorted;
-	d.cell_item_start = cell_item_start;
-	d.item_begin = item_begin;
-	d.item_count = item_count;
-	d.n_items = n_items;
+	d.sorted = bins.sorted;
+	d.cell_item_start = bins.cell_item_start;
+	d.item_begin = bins.item_begin;
+	d.item_count = bins.item_count;
+	d.n_items = bins.n_items;
 	d.max_items = max_items;
 	d.rad = D.rad;
 	d.irr = D.irr;
-	d.out = out;
 	d.loss_part = loss_part;
 	d.part_tile = part_tile;
 	d.part_mat_pix = part_mat_pix;
 	d.g_T = g_T;
 	d.part_mat_ray = part_mat_ray;
-	HIP_TRY(h, diff_bin(d, cell_id, cell_count, cell_start, cursor, cell_item_start, item_cell, item_begin, item_count,
-						n_items, sorted, s));
+	d.part_rows = part_rows;
+	HIP_TRY(h, diff_bin(d, bins, s));
+	if(rec) {
+		HIP_TRY(h, diff_records(d, rec, s));
+		d.rec = rec;
+	}
 	D.d = d;
 	D.ready = true;
 	h->last_stream = s;

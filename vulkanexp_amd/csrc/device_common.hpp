@@ -637,83 +637,6 @@ __device__ __forceinline__ Vec3 sample_probes(const GridConst& g, const uint32_t
 	return v3(fb.x * (1.0f - k) + fin.x * k, fb.y * (1.0f - k) + fin.y * k, fb.z * (1.0f - k) + fin.z * k);
 }
 
-// The irradiance-independent part of a sampleProbes call, split out for the adjoint: per cage
-// slot i (0..7) the probe, its weight and fallback weight; the colour tap footprint (the same
-// tile coordinates for all 8 probes: they depend on the normal only); the weight totals.
-struct SampleCollect {
-	uint32_t mask;  // bit i: cage probe i contributes
-	uint32_t lin[8];
-	float w[8], fw[8];
-	int cx0, cy0, cx1, cy1;
-	float cwx, cwy, tw, tfb;
-	bool outside;
-};
-
-__device__ __forceinline__ void sample_collect(const GridConst& g, const uint32_t* __restrict__ states,
-											   const float2* __restrict__ dep, Vec3 position, Vec3 normal,
-											   Vec3 to_camera, SampleCollect& c) {
-	c.mask = 0;
-	c.tw = c.tfb = 0.0f;
-	c.outside = true;
-	const Vec3 acell = v3(fabsf(g.cell[0]), fabsf(g.cell[1]), fabsf(g.cell[2]));
-	const Vec3 emin = v3(g.emin[0], g.emin[1], g.emin[2]);
-	const Vec3 gc = v3((position.x - emin.x) / acell.x, (position.y - emin.y) / acell.y, (position.z - emin.z) / acell.z);
-	if(gc.x < 0.0f || gc.y < 0.0f || gc.z < 0.0f) return;
-	c.outside = false;
-	const Vec3 biased = position + (normal + to_camera) * g.shadow_bias;
-	const int f0 = int(gc.x), f1 = int(gc.y), f2 = int(gc.z);
-	const Vec3 p0 = v3(float(f0) * g.cell[0] + emin.x, float(f1) * g.cell[1] + emin.y, float(f2) * g.cell[2] + emin.z);
-	Vec3 alpha = v3((position.x - p0.x) / acell.x, (position.y - p0.y) / acell.y, (position.z - p0.z) / acell.z);
-	alpha = v3(fminf(fmaxf(alpha.x, 0.0f), 1.0f), fminf(fmaxf(alpha.y, 0.0f), 1.0f), fminf(fmaxf(alpha.z, 0.0f), 1.0f));
-	float cu, cv;
-	oct_uv(normal.x, normal.y, normal.z, cu, cv);
-	tile_coords<8>(cu, cv, c.cx0, c.cy0, c.cx1, c.cy1, c.cwx, c.cwy);
-#pragma unroll
-	for(int i = 0; i < 8; ++i) {
-		c.lin[i] = 0;
-		c.w[i] = c.fw[i] = 0.0f;
-		uint32_t lin;
-		float w, fw;
-		if(!cage_probe(g, states, dep, position, normal, biased, emin, alpha, f0, f1, f2, i, lin, w, fw)) continue;
-		c.mask |= 1u << i;
-		c.lin[i] = lin;
-		c.w[i] = w;
-		c.fw[i] = fw;
-		c.tw += w;
-		c.tfb += fw;
-	}
-}
-
-__device__ __forceinline__ float tap3(const float4* __restrict__ irr, const SampleCollect& c, uint32_t lin, int ch) {
-	const float4* ct = irr + size_t(lin) * 64;
-	const float4 c00 = ct[c.cy0 * 8 + c.cx0], c10 = ct[c.cy0 * 8 + c.cx1], c01 = ct[c.cy1 * 8 + c.cx0],
-				 c11 = ct[c.cy1 * 8 + c.cx1];
-	const float a00 = ch == 0 ? c00.x : (ch == 1 ? c00.y : c00.z), a10 = ch == 0 ? c10.x : (ch == 1 ? c10.y : c10.z);
-	const float a01 = ch == 0 ? c01.x : (ch == 1 ? c01.y : c01.z), a11 = ch == 0 ? c11.x : (ch == 1 ? c11.y : c11.z);
-	return (a00 * (1.0f - c.cwx) + a10 * c.cwx) * (1.0f - c.cwy) + (a01 * (1.0f - c.cwx) + a11 * c.cwx) * c.cwy;
-}
-
-__device__ __forceinline__ Vec3 sample_eval(const SampleCollect& c, const float4* __restrict__ irr) {
-	if(c.outside) return v3(0.0f, 0.0f, 0.0f);
-	float out[3];
-#pragma unroll
-	for(int ch = 0; ch < 3; ++ch) {
-		float fin = 0.0f, fb = 0.0f;
-#pragma unroll
-		for(int i = 0; i < 8; ++i) {
-			if(!(c.mask & (1u << i))) continue;
-			const float s = sqrtf(tap3(irr, c, c.lin[i], ch));
-			fin += s * c.w[i];
-			fb += s * c.fw[i];
-		}
-		if(c.tw > 1e-3f) fin *= 1.0f / c.tw;
-		if(c.tfb > 1e-3f) fb *= 1.0f / c.tfb;
-		const float k = 8.0f * fminf(fmaxf(c.tw, 0.0f), 1.0f / 8.0f);
-		out[ch] = fb * fb * (1.0f - k) + fin * fin * k;
-	}
-	return v3(out[0], out[1], out[2]);
-}
-
 // Order-independent (hence deterministic) accumulation: contributions are added as 64-bit
 // fixed-point integers with 2^-50 resolution.
 constexpr double kFixScale = 1125899906842624.0;  // 2^50
@@ -721,47 +644,6 @@ __device__ __forceinline__ long long to_fixed(float x) {
 	const float s = x * 1125899906842624.0f;
 	const float lim = 9.0e18f;
 	return __float2ll_rn(fminf(fmaxf(s, -lim), lim));
-}
-
-// Adjoint of sample_eval with respect to the irradiance atlas.  acc[i*192 + texel*3 + ch] is the
-// fixed-point gradient accumulator of cage slot i's tile (64 texels x rgb).  sqrt'(x) is taken at
-// max(x, 1e-12).
-__device__ __forceinline__ void sample_adjoint(const SampleCollect& c, const float4* __restrict__ irr, Vec3 g_out,
-											   unsigned long long* acc) {
-	if(c.outside || c.mask == 0u) return;
-	const float k = 8.0f * fminf(fmaxf(c.tw, 0.0f), 1.0f / 8.0f);
-	const float inv_w = c.tw > 1e-3f ? 1.0f / c.tw : 1.0f;
-	const float inv_fb = c.tfb > 1e-3f ? 1.0f / c.tfb : 1.0f;
-	const float b00 = (1.0f - c.cwx) * (1.0f - c.cwy), b10 = c.cwx * (1.0f - c.cwy), b01 = (1.0f - c.cwx) * c.cwy,
-				b11 = c.cwx * c.cwy;
-	const int t00 = c.cy0 * 8 + c.cx0, t10 = c.cy0 * 8 + c.cx1, t01 = c.cy1 * 8 + c.cx0, t11 = c.cy1 * 8 + c.cx1;
-#pragma unroll
-	for(int ch = 0; ch < 3; ++ch) {
-		const float go = ch == 0 ? g_out.x : (ch == 1 ? g_out.y : g_out.z);
-		float s[8];
-		float fin = 0.0f, fb = 0.0f;
-#pragma unroll
-		for(int i = 0; i < 8; ++i) {
-			s[i] = 0.0f;
-			if(!(c.mask & (1u << i))) continue;
-			s[i] = sqrtf(tap3(irr, c, c.lin[i], ch));
-			fin += s[i] * c.w[i];
-			fb += s[i] * c.fw[i];
-		}
-		fin *= inv_w;
-		fb *= inv_fb;
-#pragma unroll
-		for(int i = 0; i < 8; ++i) {
-			if(!(c.mask & (1u << i))) continue;
-			const float dds = (1.0f - k) * 2.0f * fb * c.fw[i] * inv_fb + k * 2.0f * fin * c.w[i] * inv_w;
-			const float gcol = go * dds * 0.5f / sqrtf(fmaxf(s[i] * s[i], 1e-12f));
-			unsigned long long* a = acc + i * 192 + ch;
-			atomicAdd(a + t00 * 3, (unsigned long long)to_fixed(gcol * b00));
-			atomicAdd(a + t10 * 3, (unsigned long long)to_fixed(gcol * b10));
-			atomicAdd(a + t01 * 3, (unsigned long long)to_fixed(gcol * b01));
-			atomicAdd(a + t11 * 3, (unsigned long long)to_fixed(gcol * b11));
-		}
-	}
 }
 
 // pbrMetallicRoughness (src/shaders/pbrMetallicRoughness.glsl:43-84)

@@ -32,64 +32,248 @@ __device__ __forceinline__ bool cell_of(const GridConst& g, const float* pos, ui
 
 __device__ __forceinline__ Vec3 load3(const float* p, uint64_t i) { return v3(p[i * 3], p[i * 3 + 1], p[i * 3 + 2]); }
 
-// ---- prepare: bin texels by cell ----
-__global__ void k_cells(DiffArgs d, uint32_t* __restrict__ cell_id, uint32_t* __restrict__ cell_count) {
+// ---- the sampling of a texel ----
+// The irradiance-independent part of a sampleProbes call: per cage slot i (0..7) the weight and fallback
+// weight (0 when the probe does not contribute, bit i of mask), their totals, the probe of slot 0, and the
+// first colour tap (texel cy0 * 8 + cx0 of the tile) with the bilinear fractions, the same for the 8
+// probes (they depend on the normal only).
+struct TexelWeights {
+	float w[8], fw[8], cwx, cwy, tw, tfb;
+	uint32_t base, t00, mask;
+};
+
+__device__ __forceinline__ TexelWeights make_weights(const DiffArgs& d, uint64_t x) {
+	const GridConst& g = d.grid;
+	TexelWeights c;
+	c.mask = c.base = c.t00 = 0u;
+	c.cwx = c.cwy = c.tw = c.tfb = 0.0f;
+#pragma unroll
+	for(int i = 0; i < 8; ++i) c.w[i] = c.fw[i] = 0.0f;
+	const Vec3 position = load3(d.pos, x), normal = load3(d.nrm, x), to_camera = load3(d.tocam, x);
+	const Vec3 acell = v3(fabsf(g.cell[0]), fabsf(g.cell[1]), fabsf(g.cell[2]));
+	const Vec3 emin = v3(g.emin[0], g.emin[1], g.emin[2]);
+	const Vec3 gc = v3((position.x - emin.x) / acell.x, (position.y - emin.y) / acell.y, (position.z - emin.z) / acell.z);
+	if(gc.x < 0.0f || gc.y < 0.0f || gc.z < 0.0f) return c;
+	const Vec3 biased = position + (normal + to_camera) * g.shadow_bias;
+	const int f0 = int(gc.x), f1 = int(gc.y), f2 = int(gc.z);
+	const Vec3 p0 = v3(float(f0) * g.cell[0] + emin.x, float(f1) * g.cell[1] + emin.y, float(f2) * g.cell[2] + emin.z);
+	Vec3 alpha = v3((position.x - p0.x) / acell.x, (position.y - p0.y) / acell.y, (position.z - p0.z) / acell.z);
+	alpha = v3(fminf(fmaxf(alpha.x, 0.0f), 1.0f), fminf(fmaxf(alpha.y, 0.0f), 1.0f), fminf(fmaxf(alpha.z, 0.0f), 1.0f));
+	float cu, cv;
+	oct_uv(normal.x, normal.y, normal.z, cu, cv);
+	int cx0, cy0, cx1, cy1;
+	tile_coords<8>(cu, cv, cx0, cy0, cx1, cy1, c.cwx, c.cwy);
+	c.t00 = uint32_t(cy0 * 8 + cx0);
+	c.base = uint32_t(f0) + uint32_t(g.res[0]) * (uint32_t(f1) + uint32_t(g.res[1]) * uint32_t(f2));
+#pragma unroll
+	for(int i = 0; i < 8; ++i) {
+		uint32_t lin;
+		float w, fw;
+		if(!cage_probe(g, d.states, d.dep, position, normal, biased, emin, alpha, f0, f1, f2, i, lin, w, fw)) continue;
+		c.mask |= 1u << i;
+		c.w[i] = w;
+		c.fw[i] = fw;
+		c.tw += w;
+		c.tfb += fw;
+	}
+	return c;
+}
+
+// The weights of texel x from its record (w[8], fw[8], cwx, cwy, base, t00 | mask << 8), or recomputed.
+__device__ __forceinline__ TexelWeights texel_weights(const DiffArgs& d, uint64_t x) {
+	if(!d.rec) return make_weights(d, x);
+	const float4* r = d.rec + x * kDiffRecRows;
+	const float4 q[5] = {r[0], r[1], r[2], r[3], r[4]};
+	TexelWeights c;
+#pragma unroll
+	for(int i = 0; i < 2; ++i) {
+		c.w[4 * i] = q[i].x, c.w[4 * i + 1] = q[i].y, c.w[4 * i + 2] = q[i].z, c.w[4 * i + 3] = q[i].w;
+		c.fw[4 * i] = q[2 + i].x, c.fw[4 * i + 1] = q[2 + i].y, c.fw[4 * i + 2] = q[2 + i].z, c.fw[4 * i + 3] = q[2 + i].w;
+	}
+	c.cwx = q[4].x;
+	c.cwy = q[4].y;
+	c.base = __float_as_uint(q[4].z);
+	const uint32_t meta = __float_as_uint(q[4].w);
+	c.t00 = meta & 63u;
+	c.mask = meta >> 8;
+	c.tw = c.tfb = 0.0f;
+#pragma unroll
+	for(int i = 0; i < 8; ++i) {
+		c.tw += c.w[i];
+		c.tfb += c.fw[i];
+	}
+	return c;
+}
+
+// What sampleProbes makes of the weights: per channel the probes' square roots s and the normalised sums;
+// the irradiance is fb^2 (1 - k) + fin^2 k.
+struct TexelEval {
+	float s[8][3], fin[3], fb[3], k, inv_w, inv_fb;
+};
+
+__device__ __forceinline__ TexelEval texel_eval(const DiffArgs& d, const TexelWeights& c) {
+	TexelEval e;
+	const uint32_t x0 = c.t00 & 7u, y0 = c.t00 >> 3, x1 = min(x0 + 1u, 7u), y1 = min(y0 + 1u, 7u);
+	const uint32_t t10 = y0 * 8u + x1, t01 = y1 * 8u + x0, t11 = y1 * 8u + x1;
+	const uint32_t rx = uint32_t(d.grid.res[0]), ry = uint32_t(d.grid.res[1]);
+	e.inv_w = c.tw > 1e-3f ? 1.0f / c.tw : 1.0f;
+	e.inv_fb = c.tfb > 1e-3f ? 1.0f / c.tfb : 1.0f;
+	e.k = 8.0f * fminf(fmaxf(c.tw, 0.0f), 1.0f / 8.0f);
+#pragma unroll
+	for(int ch = 0; ch < 3; ++ch) e.fin[ch] = e.fb[ch] = 0.0f;
+#pragma unroll
+	for(int i = 0; i < 8; ++i) {
+		const bool on = (c.mask >> i) & 1u;
+		// slots that do not contribute read some tile and drop what they read
+		const uint32_t lin = on ? c.base + uint32_t(i & 1) + rx * (uint32_t((i >> 1) & 1) + ry * uint32_t(i >> 2)) : 0u;
+		const float4* ct = d.irr + size_t(lin) * 64;
+		const float4 c00 = ct[c.t00], c10 = ct[t10], c01 = ct[t01], c11 = ct[t11];
+		const float a[3][4] = {{c00.x, c10.x, c01.x, c11.x}, {c00.y, c10.y, c01.y, c11.y}, {c00.z, c10.z, c01.z, c11.z}};
+#pragma unroll
+		for(int ch = 0; ch < 3; ++ch) {
+			const float v = (a[ch][0] * (1.0f - c.cwx) + a[ch][1] * c.cwx) * (1.0f - c.cwy) +
+							(a[ch][2] * (1.0f - c.cwx) + a[ch][3] * c.cwx) * c.cwy;
+			e.s[i][ch] = on ? sqrtf(v) : 0.0f;
+			e.fin[ch] += e.s[i][ch] * c.w[i];
+			e.fb[ch] += e.s[i][ch] * c.fw[i];
+		}
+	}
+#pragma unroll
+	for(int ch = 0; ch < 3; ++ch) {
+		e.fin[ch] *= e.inv_w;
+		e.fb[ch] *= e.inv_fb;
+	}
+	return e;
+}
+
+// ---- prepare: sampling records, and texels binned by (cell, first colour tap) ----
+__global__ __launch_bounds__(kBlock) void k_records(DiffArgs d, float4* __restrict__ rec) {
+	const uint64_t x = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+	if(x >= d.N) return;
+	const TexelWeights c = make_weights(d, x);
+	float4* r = rec + x * kDiffRecRows;
+	r[0] = make_float4(c.w[0], c.w[1], c.w[2], c.w[3]);
+	r[1] = make_float4(c.w[4], c.w[5], c.w[6], c.w[7]);
+	r[2] = make_float4(c.fw[0], c.fw[1], c.fw[2], c.fw[3]);
+	r[3] = make_float4(c.fw[4], c.fw[5], c.fw[6], c.fw[7]);
+	r[4] = make_float4(c.cwx, c.cwy, __uint_as_float(c.base), __uint_as_float(c.t00 | (c.mask << 8)));
+}
+
+// Adds 1 to counter[key] for every active lane and returns the lane's own position, with one atomic per
+// distinct key of the wavefront (neighbouring texels mostly share theirs: one atomic per lane on a few
+// hundred hot counters took 4 ms for a full-HD view).
+__device__ __forceinline__ uint32_t wave_count(uint32_t* counter, uint32_t key) {
+	const uint32_t lane = __lane_id();
+	uint32_t pos = 0;
+	for(uint64_t left = __ballot(true); left != 0u;) {
+		const int leader = __ffsll((unsigned long long)left) - 1;
+		const uint32_t k = uint32_t(__builtin_amdgcn_readlane(int(key), leader));
+		const uint64_t same = __ballot(key == k) & left;
+		if(key == k) {
+			uint32_t base = 0;
+			if(int(lane) == leader) base = atomicAdd(&counter[k], uint32_t(__popcll(same)));
+			pos = uint32_t(__builtin_amdgcn_readlane(int(base), leader)) +
+				  uint32_t(__popcll(same & ((uint64_t(1) << lane) - 1u)));
+		}
+		left &= ~same;
+	}
+	return pos;
+}
+
+__global__ void k_cells(DiffArgs d, uint32_t taps, uint32_t* __restrict__ key_of, uint32_t* __restrict__ key_count) {
 	const uint64_t x = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if(x >= d.N) return;
 	uint32_t c;
-	if(cell_of(d.grid, d.pos, x, c)) {
-		cell_id[x] = c;
-		atomicAdd(&cell_count[c], 1u);
-	} else {
-		cell_id[x] = 0xFFFFFFFFu;
+	if(!cell_of(d.grid, d.pos, x, c)) {
+		key_of[x] = 0xFFFFFFFFu;
+		return;
 	}
+	if(taps == 64u) {
+		float cu, cv, wx, wy;
+		int x0, y0, x1, y1;
+		oct_uv(d.nrm[x * 3], d.nrm[x * 3 + 1], d.nrm[x * 3 + 2], cu, cv);
+		tile_coords<8>(cu, cv, x0, y0, x1, y1, wx, wy);
+		c = c * 64u + uint32_t(y0 * 8 + x0);
+	}
+	key_of[x] = c;
+	wave_count(key_count, c);
 }
 
-// single block: exclusive scans over cells -> pixel offsets and work items of <= kDiffChunk texels
-__global__ __launch_bounds__(1024) void k_items(DiffArgs d, const uint32_t* __restrict__ cell_count,
-												uint32_t* __restrict__ cell_start, uint32_t* __restrict__ cell_item_start,
-												uint32_t* __restrict__ item_cell, uint32_t* __restrict__ item_begin,
-												uint32_t* __restrict__ item_count, uint32_t* __restrict__ n_items) {
-	__shared__ uint32_t s_pix, s_items;
-	if(threadIdx.x == 0) {
-		s_pix = 0;
-		s_items = 0;
+// Sum over a workgroup of 1024 threads of (a, b), and this thread's exclusive prefix.
+__device__ __forceinline__ void block_scan2(uint32_t a, uint32_t b, uint32_t* s_a, uint32_t* s_b, uint32_t& pa, uint32_t& pb,
+											uint32_t& ta, uint32_t& tb) {
+	const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+	uint32_t ia = a, ib = b;
+	for(int o = 1; o < 64; o <<= 1) {
+		const uint32_t xa = uint32_t(__shfl_up(int(ia), o)), xb = uint32_t(__shfl_up(int(ib), o));
+		if(lane >= uint32_t(o)) {
+			ia += xa;
+			ib += xb;
+		}
+	}
+	if(lane == 63u) {
+		s_a[wave] = ia;
+		s_b[wave] = ib;
 	}
 	__syncthreads();
-	const uint32_t cells = d.grid.probe_count;
-	for(uint32_t base = 0; base < cells; base += 1024) {
-		// serial scan by thread 0 over this chunk (cells <= 2^24, a few thousand here)
-		if(threadIdx.x == 0) {
-			for(uint32_t c = base; c < min(cells, base + 1024u); ++c) {
-				const uint32_t cnt = cell_count[c];
-				cell_start[c] = s_pix;
-				cell_item_start[c] = s_items;
-				const uint32_t ni = (cnt + kDiffChunk - 1) / kDiffChunk;
-				for(uint32_t k = 0; k < ni; ++k) {
-					item_cell[s_items + k] = c;
-					item_begin[s_items + k] = s_pix + k * kDiffChunk;
-					item_count[s_items + k] = min(kDiffChunk, cnt - k * kDiffChunk);
-				}
-				s_pix += cnt;
-				s_items += ni;
+	pa = ia - a;
+	pb = ib - b;
+	ta = tb = 0;
+	for(uint32_t w = 0; w < 16u; ++w) {
+		pa += w < wave ? s_a[w] : 0u;
+		pb += w < wave ? s_b[w] : 0u;
+		ta += s_a[w];
+		tb += s_b[w];
+	}
+	__syncthreads();
+}
+
+// One workgroup: exclusive sums over the keys (texel offsets) and over the cells (work items of at most
+// kDiffChunk texels of a cell).
+__global__ __launch_bounds__(1024) void k_items(DiffArgs d, uint32_t taps, const uint32_t* __restrict__ key_count,
+												uint32_t* __restrict__ key_start, uint32_t* __restrict__ cell_item_start,
+												uint32_t* __restrict__ item_begin, uint32_t* __restrict__ item_count,
+												uint32_t* __restrict__ n_items) {
+	__shared__ uint32_t s_a[16], s_b[16];
+	const uint32_t cells = d.grid.probe_count, t = threadIdx.x;
+	uint32_t pix = 0, items = 0;
+	for(uint32_t base = 0; base < cells; base += 1024u) {
+		const uint32_t c = base + t;
+		uint32_t cnt = 0;
+		if(c < cells)
+			for(uint32_t k = 0; k < taps; ++k) cnt += key_count[size_t(c) * taps + k];
+		const uint32_t ni = (cnt + kDiffChunk - 1) / kDiffChunk;
+		uint32_t pc, pi, tc, ti;
+		block_scan2(cnt, ni, s_a, s_b, pc, pi, tc, ti);
+		if(c < cells) {
+			uint32_t at = pix + pc;
+			cell_item_start[c] = items + pi;
+			for(uint32_t k = 0; k < ni; ++k) {
+				item_begin[items + pi + k] = at + k * kDiffChunk;
+				item_count[items + pi + k] = min(kDiffChunk, cnt - k * kDiffChunk);
+			}
+			for(uint32_t k = 0; k < taps; ++k) {
+				key_start[size_t(c) * taps + k] = at;
+				at += key_count[size_t(c) * taps + k];
 			}
 		}
-		__syncthreads();
+		pix += tc;
+		items += ti;
 	}
-	if(threadIdx.x == 0) {
-		cell_start[cells] = s_pix;
-		cell_item_start[cells] = s_items;
-		*n_items = s_items;
+	if(t == 0) {
+		cell_item_start[cells] = items;
+		*n_items = items;
 	}
 }
 
-__global__ void k_scatter(DiffArgs d, const uint32_t* __restrict__ cell_id, const uint32_t* __restrict__ cell_start,
+__global__ void k_scatter(DiffArgs d, const uint32_t* __restrict__ key_of, const uint32_t* __restrict__ key_start,
 						  uint32_t* __restrict__ cursor, uint32_t* __restrict__ sorted) {
 	const uint64_t x = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if(x >= d.N) return;
-	const uint32_t c = cell_id[x];
+	const uint32_t c = key_of[x];
 	if(c == 0xFFFFFFFFu) return;
-	sorted[cell_start[c] + atomicAdd(&cursor[c], 1u)] = uint32_t(x);
+	const uint32_t pos = wave_count(cursor, c);
+	sorted[key_start[c] + pos] = uint32_t(x);
 }
 
 // ---- forward ----
@@ -110,68 +294,175 @@ __global__ void k_radiance(DiffArgs d) {
 	d.rad[r] = out;
 }
 
+// One thread per texel: 80 bytes of record, 16 of material and target in, 12 out, and 32 taps that
+// neighbouring texels share.  Memory-bound: 63 us for a full-HD view (250 MB in 50 us at a copy's rate),
+// against 128 us with the weights recomputed.
 __global__ __launch_bounds__(kBlock) void k_gather_fwd(DiffArgs d) {
-	__shared__ float red[kBlock];
+	__shared__ float red[kBlock / 64];
 	const uint64_t x = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
 	float l = 0.0f;
 	if(x < d.N) {
-		SampleCollect c;
-		sample_collect(d.grid, d.states, d.dep, load3(d.pos, x), load3(d.nrm, x), load3(d.tocam, x), c);
-		const Vec3 o = sample_eval(c, d.irr);
+		const TexelWeights c = texel_weights(d, x);
+		const TexelEval e = texel_eval(d, c);
 		const float* a = d.albedo + size_t(d.gmat[x]) * 3;
-		const float s[3] = {o.x * a[0] * 0.996f, o.y * a[1] * 0.996f, o.z * a[2] * 0.996f};
-		d.out[x * 3] = o.x;
-		d.out[x * 3 + 1] = o.y;
-		d.out[x * 3 + 2] = o.z;
+#pragma unroll
 		for(int ch = 0; ch < 3; ++ch) {
-			d.shade[x * 3 + ch] = s[ch];
-			const float e = s[ch] - d.target[x * 3 + ch];
-			l += e * e;
+			const float o = e.fb[ch] * e.fb[ch] * (1.0f - e.k) + e.fin[ch] * e.fin[ch] * e.k;
+			const float s = o * a[ch] * 0.996f;
+			d.shade[x * 3 + ch] = s;
+			const float err = s - d.target[x * 3 + ch];
+			l += err * err;
 		}
 	}
-	red[threadIdx.x] = l;
+	for(int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+	if(__lane_id() == 0) red[threadIdx.x >> 6] = l;
 	__syncthreads();
-	for(int o = kBlock / 2; o > 0; o >>= 1) {
-		if(int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
-		__syncthreads();
-	}
-	if(threadIdx.x == 0) d.loss_part[blockIdx.x] = red[0];
+	if(threadIdx.x == 0) d.loss_part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void k_loss(DiffArgs d, uint32_t parts) {
-	if(threadIdx.x != 0 || blockIdx.x != 0) return;
+// One workgroup; the partial sums added in double, in a fixed order (5 us; 329 us in one thread).
+__global__ __launch_bounds__(1024) void k_loss(DiffArgs d, uint32_t parts) {
+	__shared__ double red[1024];
 	double s = 0.0;
-	for(uint32_t i = 0; i < parts; ++i) s += double(d.loss_part[i]);
-	d.loss[0] = float(s / double(3ull * d.N));
+	for(uint32_t i = threadIdx.x; i < parts; i += 1024u) s += double(d.loss_part[i]);
+	red[threadIdx.x] = s;
+	__syncthreads();
+	for(uint32_t o = 512; o > 0; o >>= 1) {
+		if(threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+		__syncthreads();
+	}
+	if(threadIdx.x == 0) d.loss[0] = float(red[0] / double(3ull * d.N));
 }
 
 // ---- backward ----
-// One block per work item: the item's texels share one cage of 8 probes.
-__global__ __launch_bounds__(kBlock) void k_gather_bwd(DiffArgs d) {
+// Contributions are held in units of 2^-50, rounded to integers, in doubles: sums of these are exact,
+// hence independent of their order, while they stay below 2^53 units (8.0; the contributions of a mean
+// over the texels are far smaller), and are rounded to 53 bits above that.
+constexpr float kUnits = 1125899906842624.0f;  // 2^50
+__device__ __forceinline__ float to_units(float x) { return fminf(fmaxf(x * kUnits, -9.0e18f), 9.0e18f); }
+__device__ __forceinline__ void add_units(unsigned long long* a, double v) {
+	atomicAdd(a, (unsigned long long)(long long)(fmin(fmax(v, -9.0e18), 9.0e18)));
+}
+
+// One workgroup per work item: its texels share one cage of 8 probes, whose gradient tiles it sums in
+// LDS.  A wavefront evaluates 64 texels, one per lane, and then, for each channel, turns to eight texels at
+// a time with one lane per cage probe (through LDS).  As the texels are ordered by their first tap, the
+// eight nearly always share their four taps (and the 64 their material), so that a lane adds its
+// contributions to registers and goes to the LDS tiles only when the taps change.  Full-HD view: 531 us
+// with 96 LDS atomics per texel, most of them 64 lanes on one address; 233 us with eight lanes per texel
+// throughout, where the evaluation is done eight times over; 110 us so (178 with the texels ordered by
+// cell only, 124 with items of 2048 texels, 195 with 4096; 5 waves per SIMD spill: 157).  Bound by vector
+// instructions: the square roots, divisions and roundings of 96 contributions per texel.
+// four waves per SIMD: 128 VGPRs
+__global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 	extern __shared__ unsigned long long lds[];
 	unsigned long long* tile = lds;                  // [8][64][3]
 	unsigned long long* mat = lds + 8 * 192;         // [M][3]
+	__shared__ __attribute__((aligned(16))) float s_g[kBlock / 64][64 * 8];  // gradient per (texel, probe), one channel
+	__shared__ __attribute__((aligned(16))) float s_b[kBlock / 64][64 * 4];  // tap weights per texel
+	__shared__ uint32_t s_t[kBlock / 64][64];                                // first tap, kNo: no texel
 	const uint32_t item = blockIdx.x;
 	if(item >= *d.n_items) return;
 	for(uint32_t k = threadIdx.x; k < 8 * 192 + d.M * 3; k += kBlock) lds[k] = 0ull;
 	__syncthreads();
 	const uint32_t begin = d.item_begin[item], cnt = d.item_count[item];
 	const float inv3n = 2.0f / float(3ull * d.N);
-	for(uint32_t k = threadIdx.x; k < cnt; k += kBlock) {
-		const uint64_t x = d.sorted[begin + k];
-		SampleCollect c;
-		sample_collect(d.grid, d.states, d.dep, load3(d.pos, x), load3(d.nrm, x), load3(d.tocam, x), c);
+	const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, i = lane & 7u;
+	unsigned long long* my_tile = tile + i * 192;
+	constexpr uint32_t kNo = 0xFFFFFFFFu;
+	uint32_t cur_tap = kNo, cur_mat = kNo;  // wave-uniform: what the registers hold sums of
+	double acc[4][3], macc[3];
+#pragma unroll
+	for(int q = 0; q < 4; ++q) acc[q][0] = acc[q][1] = acc[q][2] = 0.0;
+	macc[0] = macc[1] = macc[2] = 0.0;
+	const auto tap_of = [](uint32_t t00, int q) {
+		const uint32_t x = min((t00 & 7u) + uint32_t(q & 1), 7u), y = min((t00 >> 3) + uint32_t(q >> 1), 7u);
+		return y * 8u + x;
+	};
+	const auto flush_taps = [&] {
+#pragma unroll
+		for(int q = 0; q < 4; ++q)
+#pragma unroll
+			for(int ch = 0; ch < 3; ++ch) {
+				if(acc[q][ch] != 0.0) add_units(my_tile + tap_of(cur_tap, q) * 3 + ch, acc[q][ch]);
+				acc[q][ch] = 0.0;
+			}
+	};
+	const auto flush_mat = [&] {
+#pragma unroll
+		for(int ch = 0; ch < 3; ++ch) {
+			double v = macc[ch];
+			for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+			if(lane == 0 && v != 0.0) add_units(mat + size_t(cur_mat) * 3 + ch, v);
+			macc[ch] = 0.0;
+		}
+	};
+	for(uint32_t k0 = wave * 64u; k0 < cnt; k0 += kBlock) {  // wave-uniform; no barrier inside
+		const bool on = k0 + lane < cnt;
+		const uint64_t x = d.sorted[begin + (on ? k0 + lane : k0)];
+		const TexelWeights c = texel_weights(d, x);
+		const TexelEval e = texel_eval(d, c);
 		const uint32_t m = d.gmat[x];
 		const float* a = d.albedo + size_t(m) * 3;
-		float go[3];
-		for(int ch = 0; ch < 3; ++ch) {
-			const float o = d.out[x * 3 + ch];
-			const float gs = (o * a[ch] * 0.996f - d.target[x * 3 + ch]) * inv3n;
-			atomicAdd(&mat[m * 3 + ch], (unsigned long long)to_fixed(gs * o * 0.996f));
-			go[ch] = gs * a[ch] * 0.996f;
+		const uint32_t mat0 = uint32_t(__builtin_amdgcn_readfirstlane(int(m)));
+		const bool one_mat = __ballot(on && m != mat0) == 0u;
+		if(one_mat && mat0 != cur_mat) {
+			flush_mat();
+			cur_mat = mat0;
 		}
-		sample_adjoint(c, d.irr, v3(go[0], go[1], go[2]), tile);
+		float go[3];
+#pragma unroll
+		for(int ch = 0; ch < 3; ++ch) {
+			const float o = e.fb[ch] * e.fb[ch] * (1.0f - e.k) + e.fin[ch] * e.fin[ch] * e.k;
+			const float gs = on ? (o * a[ch] * 0.996f - d.target[x * 3 + ch]) * inv3n : 0.0f;
+			go[ch] = gs * a[ch] * 0.996f;
+			const double gm = double(rintf(to_units(gs * o * 0.996f)));
+			if(one_mat) macc[ch] += gm;
+			else if(gm != 0.0) add_units(mat + size_t(m) * 3 + ch, gm);
+		}
+		*reinterpret_cast<float4*>(&s_b[wave][lane * 4]) = make_float4((1.0f - c.cwx) * (1.0f - c.cwy), c.cwx * (1.0f - c.cwy),
+																	  (1.0f - c.cwx) * c.cwy, c.cwx * c.cwy);
+		s_t[wave][lane] = on ? c.t00 : kNo;
+#pragma unroll
+		for(int ch = 0; ch < 3; ++ch) {
+			// d loss / d (the probe's bilinear irradiance); sqrt'(v) taken at s >= 1e-6
+			const float df = (1.0f - e.k) * 2.0f * e.fb[ch] * e.inv_fb, dw = e.k * 2.0f * e.fin[ch] * e.inv_w;
+			float g[8];
+#pragma unroll
+			for(int p = 0; p < 8; ++p)
+				g[p] = to_units(go[ch] * (df * c.fw[p] + dw * c.w[p]) * 0.5f / fmaxf(e.s[p][ch], 1e-6f));
+			float4* dst = reinterpret_cast<float4*>(&s_g[wave][lane * 8]);
+			dst[0] = make_float4(g[0], g[1], g[2], g[3]);
+			dst[1] = make_float4(g[4], g[5], g[6], g[7]);
+			// (the compiler orders these LDS accesses; a wavefront's LDS operations complete in order)
+			__builtin_amdgcn_wave_barrier();
+			for(uint32_t h = 0; h < 64u && k0 + h < cnt; h += 8u) {
+				const uint32_t texel = h + (lane >> 3);
+				const uint32_t t00 = s_t[wave][texel];
+				const uint32_t tap0 = uint32_t(__builtin_amdgcn_readfirstlane(int(t00)));  // the first texel exists
+				const float gv = s_g[wave][texel * 8 + i];
+				const float4 b4 = *reinterpret_cast<const float4*>(&s_b[wave][texel * 4]);
+				const float b[4] = {b4.x, b4.y, b4.z, b4.w};
+				if(__ballot(t00 != kNo && t00 != tap0) == 0u) {
+					if(tap0 != cur_tap) {
+						flush_taps();
+						cur_tap = tap0;
+					}
+#pragma unroll
+					for(int q = 0; q < 4; ++q) acc[q][ch] += double(rintf(gv * b[q]));  // no texel: gv is 0
+				} else if(t00 != kNo) {
+#pragma unroll
+					for(int q = 0; q < 4; ++q) {
+						const float v = rintf(gv * b[q]);
+						if(v != 0.0f) add_units(my_tile + tap_of(t00, q) * 3 + ch, double(v));
+					}
+				}
+			}
+			__builtin_amdgcn_wave_barrier();
+		}
 	}
+	flush_taps();
+	flush_mat();
 	__syncthreads();
 	long long* pt = d.part_tile + size_t(item) * 8 * 192;
 	for(uint32_t k = threadIdx.x; k < 8 * 192; k += kBlock) pt[k] = (long long)tile[k];
@@ -180,23 +471,30 @@ __global__ __launch_bounds__(kBlock) void k_gather_bwd(DiffArgs d) {
 }
 
 // One block per probe: sum the partial tiles of the (up to 8) cells whose cage contains the
-// probe, fold the border gradients onto the interior texels they copy, scale to float.
-__global__ __launch_bounds__(192) void k_probe_grad(DiffArgs d) {
+// probe, fold the border gradients onto the interior texels they copy, scale to float.  Four groups of
+// 192 threads share the items (integer sums: any order gives the same; 18 us, 70 us with one group).
+__global__ __launch_bounds__(768) void k_probe_grad(DiffArgs d) {
+	__shared__ long long part[4][64 * 3];
 	__shared__ long long g[64 * 3];
 	const uint32_t p = blockIdx.x;
 	const uint32_t rx = uint32_t(d.grid.res[0]), ry = uint32_t(d.grid.res[1]);
 	const int px = int(p % rx), py = int((p % (rx * ry)) / rx), pz = int(p / (rx * ry));
-	const uint32_t e = threadIdx.x;  // texel * 3 + channel
+	const uint32_t grp = threadIdx.x / 192u;
+	uint32_t e = threadIdx.x - grp * 192u;  // texel * 3 + channel
 	long long s = 0;
 	for(int o = 0; o < 8; ++o) {
 		const int cx = px - (o & 1), cy = py - ((o >> 1) & 1), cz = pz - ((o >> 2) & 1);
 		if(cx < 0 || cy < 0 || cz < 0) continue;
 		const uint32_t cell = uint32_t(cx) + rx * (uint32_t(cy) + ry * uint32_t(cz));
-		for(uint32_t it = d.cell_item_start[cell]; it < d.cell_item_start[cell + 1]; ++it)
-			s += d.part_tile[(size_t(it) * 8 + o) * 192 + e];
+		const uint32_t first = d.cell_item_start[cell], last = d.cell_item_start[cell + 1];
+#pragma unroll 4
+		for(uint32_t it = first + grp; it < last; it += 4u) s += d.part_tile[(size_t(it) * 8 + o) * 192 + e];
 	}
-	g[e] = s;
+	part[grp][e] = s;
 	__syncthreads();
+	if(grp == 0) g[e] = part[0][e] + part[1][e] + part[2][e] + part[3][e];
+	__syncthreads();
+	if(grp != 0) e = 192u;  // the rest is one group's
 	// border fold (adjoint of probesCopyBorders: dst <- src)
 	if(e < 3) {
 		const int R = 8;
@@ -243,6 +541,7 @@ __global__ __launch_bounds__(kBlock) void k_blend_bwd(DiffArgs d) {
 	}
 	__syncthreads();
 	const uint32_t n = d.grid.n;
+	double sun[3] = {0.0, 0.0, 0.0};  // every ray adds to these: summed in registers first
 	for(uint32_t j = threadIdx.x; j < n; j += kBlock) {
 		const float4 dr = d.dirs[d.perm[j]];
 		float gr[3] = {0.0f, 0.0f, 0.0f};
@@ -260,23 +559,43 @@ __global__ __launch_bounds__(kBlock) void k_blend_bwd(DiffArgs d) {
 		const float Av[3] = {A.x, A.y, A.z}, Bv[3] = {B.x, B.y, B.z}, Cv[3] = {C.x, C.y, C.z};
 		for(int ch = 0; ch < 3; ++ch) {
 			atomicAdd(&mat[m * 3 + ch], (unsigned long long)to_fixed(gr[ch] * (Av[ch] + Bv[ch] * d.sun[ch])));
-			atomicAdd(&mat[d.M * 3 + ch], (unsigned long long)to_fixed(gr[ch] * (Bv[ch] * a[ch] + Cv[ch])));
+			sun[ch] += double(rintf(to_units(gr[ch] * (Bv[ch] * a[ch] + Cv[ch]))));
 		}
+	}
+#pragma unroll
+	for(int ch = 0; ch < 3; ++ch) {
+		for(int o = 32; o > 0; o >>= 1) sun[ch] += __shfl_xor(sun[ch], o);
+		if(__lane_id() == 0) add_units(&mat[d.M * 3 + ch], sun[ch]);
 	}
 	__syncthreads();
 	long long* pr = d.part_mat_ray + size_t(slot) * (d.M * 3 + 3);
 	for(uint32_t k = threadIdx.x; k < d.M * 3 + 3; k += kBlock) pr[k] = (long long)mat[k];
 }
 
+// Columns (material channels, then the sun's) of the items' and slots' partial sums: workgroup b adds rows
+// b, b + kDiffSumBlocks, ... (one row after another, coalesced), then one thread per column adds the
+// workgroups' sums.  (One thread per column over every row: 214 us for a full-HD view.)
+__global__ __launch_bounds__(kBlock) void k_grad_rows(DiffArgs d) {
+	const uint32_t cols = d.M * 3 + 3, items = *d.n_items;
+	for(uint32_t k = threadIdx.x; k < cols; k += kBlock) {
+		long long s = 0;
+		if(k < d.M * 3) {
+#pragma unroll 8
+			for(uint32_t it = blockIdx.x; it < items; it += kDiffSumBlocks) s += d.part_mat_pix[size_t(it) * d.M * 3 + k];
+		}
+#pragma unroll 8
+		for(uint32_t sl = blockIdx.x; sl < d.slots; sl += kDiffSumBlocks) s += d.part_mat_ray[size_t(sl) * cols + k];
+		d.part_rows[size_t(blockIdx.x) * cols + k] = s;
+	}
+}
+
 __global__ void k_grad_final(DiffArgs d) {
 	const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-	if(k >= d.M * 3 + 3) return;
+	const uint32_t cols = d.M * 3 + 3;
+	if(k >= cols) return;
 	long long s = 0;
-	if(k < d.M * 3) {
-		const uint32_t items = *d.n_items;
-		for(uint32_t it = 0; it < items; ++it) s += d.part_mat_pix[size_t(it) * d.M * 3 + k];
-	}
-	for(uint32_t sl = 0; sl < d.slots; ++sl) s += d.part_mat_ray[size_t(sl) * (d.M * 3 + 3) + k];
+#pragma unroll 16
+	for(uint32_t b = 0; b < kDiffSumBlocks; ++b) s += d.part_rows[size_t(b) * cols + k];
 	const float v = float(double(s) / kFixScale) * d.grad_loss[0];
 	if(k < d.M * 3) d.g_albedo[k] = v;
 	else d.g_sun[k - d.M * 3] = v;
@@ -286,17 +605,20 @@ inline uint32_t nblocks(uint64_t n, uint32_t b) { return uint32_t((n + b - 1) / 
 
 }  // namespace
 
-hipError_t diff_bin(const DiffArgs& d, uint32_t* cell_id, uint32_t* cell_count, uint32_t* cell_start, uint32_t* cursor,
-					uint32_t* cell_item_start, uint32_t* item_cell, uint32_t* item_begin, uint32_t* item_count,
-					uint32_t* n_items, uint32_t* sorted, hipStream_t s) {
-	const uint32_t cells = d.grid.probe_count;
+hipError_t diff_bin(const DiffArgs& d, const DiffBins& b, hipStream_t s) {
+	const size_t keys = size_t(d.grid.probe_count) * b.taps;
 	hipError_t e;
-	if((e = hipMemsetAsync(cell_count, 0, cells * 4, s)) != hipSuccess) return e;
-	if((e = hipMemsetAsync(cursor, 0, cells * 4, s)) != hipSuccess) return e;
-	if(d.N) hipLaunchKernelGGL(k_cells, dim3(nblocks(d.N, 256)), dim3(256), 0, s, d, cell_id, cell_count);
-	hipLaunchKernelGGL(k_items, dim3(1), dim3(1024), 0, s, d, cell_count, cell_start, cell_item_start, item_cell, item_begin,
-					   item_count, n_items);
-	if(d.N) hipLaunchKernelGGL(k_scatter, dim3(nblocks(d.N, 256)), dim3(256), 0, s, d, cell_id, cell_start, cursor, sorted);
+	if((e = hipMemsetAsync(b.key_count, 0, keys * 4, s)) != hipSuccess) return e;
+	if((e = hipMemsetAsync(b.cursor, 0, keys * 4, s)) != hipSuccess) return e;
+	hipLaunchKernelGGL(k_cells, dim3(nblocks(d.N, 256)), dim3(256), 0, s, d, b.taps, b.key_of, b.key_count);
+	hipLaunchKernelGGL(k_items, dim3(1), dim3(1024), 0, s, d, b.taps, b.key_count, b.key_start, b.cell_item_start,
+					   b.item_begin, b.item_count, b.n_items);
+	hipLaunchKernelGGL(k_scatter, dim3(nblocks(d.N, 256)), dim3(256), 0, s, d, b.key_of, b.key_start, b.cursor, b.sorted);
+	return hipGetLastError();
+}
+
+hipError_t diff_records(const DiffArgs& d, float4* rec, hipStream_t s) {
+	hipLaunchKernelGGL(k_records, dim3(nblocks(d.N, kBlock)), dim3(kBlock), 0, s, d, rec);
 	return hipGetLastError();
 }
 
@@ -307,18 +629,19 @@ hipError_t diff_radiance(const DiffArgs& d, hipStream_t s) {
 
 hipError_t diff_gather_forward(const DiffArgs& d, hipStream_t s) {
 	const uint32_t parts = nblocks(d.N, kBlock);
-	if(d.N) hipLaunchKernelGGL(k_gather_fwd, dim3(parts), dim3(kBlock), 0, s, d);
-	hipLaunchKernelGGL(k_loss, dim3(1), dim3(64), 0, s, d, parts);
+	hipLaunchKernelGGL(k_gather_fwd, dim3(parts), dim3(kBlock), 0, s, d);
+	hipLaunchKernelGGL(k_loss, dim3(1), dim3(1024), 0, s, d, parts);
 	return hipGetLastError();
 }
 
 hipError_t diff_backward(const DiffArgs& d, hipStream_t s) {
 	const size_t lds1 = (8 * 192 + size_t(d.M) * 3) * sizeof(unsigned long long);
 	hipLaunchKernelGGL(k_gather_bwd, dim3(d.max_items), dim3(kBlock), lds1, s, d);
-	hipLaunchKernelGGL(k_probe_grad, dim3(d.grid.probe_count), dim3(192), 0, s, d);
+	hipLaunchKernelGGL(k_probe_grad, dim3(d.grid.probe_count), dim3(768), 0, s, d);
 	const size_t lds2 = (size_t(d.M) * 3 + 3) * sizeof(unsigned long long);
 	hipLaunchKernelGGL(k_blend_bwd, dim3(d.slots), dim3(kBlock), lds2, s, d);
-	hipLaunchKernelGGL(k_grad_final, dim3(nblocks(d.M * 3 + 3, 256)), dim3(256), 0, s, d);
+	hipLaunchKernelGGL(k_grad_rows, dim3(kDiffSumBlocks), dim3(kBlock), 0, s, d);
+	hipLaunchKernelGGL(k_grad_final, dim3(nblocks(d.M * 3 + 3, 64)), dim3(64), 0, s, d);
 	return hipGetLastError();
 }
 

@@ -5,7 +5,10 @@
 
 namespace ddgi {
 
-constexpr uint32_t kDiffChunk = 2048;  // G-buffer texels per backward work item (one cell)
+constexpr uint32_t kDiffChunk = 1024;  // G-buffer texels per backward work item (one cell)
+constexpr uint32_t kDiffRecRows = 5;  // float4s of a texel's sampling record
+constexpr uint64_t kDiffRecords = 12u << 20;  // most texels whose records are kept (1 GiB; a 4K view has 8.3 M)
+constexpr uint32_t kDiffSumBlocks = 64;  // workgroups that add up the material partial sums
 
 struct DiffArgs {
 	GridConst grid;
@@ -37,7 +40,7 @@ struct DiffArgs {
 	const float* target;            // [N][3]
 	float4* rad;                    // [rays]
 	const float4* irr;              // differentiated irradiance atlas (tiled)
-	float* out;                     // [N][3] sampled irradiance
+	const float4* rec;              // [N][kDiffRecRows] sampling records, nullptr: recomputed
 	float* shade;                   // [N][3]
 	float* loss_part;
 	float* loss;
@@ -45,14 +48,24 @@ struct DiffArgs {
 	long long* part_mat_pix;        // [max_items][M][3]
 	float* g_T;                     // [P][36][3]
 	long long* part_mat_ray;        // [slots][M * 3 + 3]
+	long long* part_rows;           // [kDiffSumBlocks][M * 3 + 3]
 	const float* grad_loss;         // [1]
 	float* g_albedo;                // [M][3]
 	float* g_sun;                   // [3]
 };
 
-hipError_t diff_bin(const DiffArgs& d, uint32_t* cell_id, uint32_t* cell_count, uint32_t* cell_start, uint32_t* cursor,
-					uint32_t* cell_item_start, uint32_t* item_cell, uint32_t* item_begin, uint32_t* item_count,
-					uint32_t* n_items, uint32_t* sorted, hipStream_t s);
+// Buffers of the texel binning; keys = cell * taps + first colour tap (taps = 64), or cells (taps = 1).
+struct DiffBins {
+	uint32_t taps;
+	uint32_t *key_of;                // [N]
+	uint32_t *key_count, *key_start, *cursor;  // [cells * taps]
+	uint32_t *cell_item_start;       // [cells + 1]
+	uint32_t *item_begin, *item_count, *n_items;
+	uint32_t* sorted;                // [N]
+};
+hipError_t diff_bin(const DiffArgs& d, const DiffBins& b, hipStream_t s);
+// The texels' sampling records (d.rec is set to them afterwards).
+hipError_t diff_records(const DiffArgs& d, float4* rec, hipStream_t s);
 hipError_t diff_radiance(const DiffArgs& d, hipStream_t s);
 hipError_t diff_gather_forward(const DiffArgs& d, hipStream_t s);
 hipError_t diff_backward(const DiffArgs& d, hipStream_t s);
