@@ -164,13 +164,10 @@ void free_scene(Handle* h) {
 	h->move_pending = false;
 	(void)hipHostFree(h->move_host);
 	h->move_host = nullptr;
-	h->move_xf = nullptr;
-	h->move_meta = nullptr;
-	h->obj_tris = nullptr;
-	h->slot_box = nullptr;
-	h->rel_xf = nullptr;
+	h->slots = SlotBoxArgs{};
+	h->node_range = nullptr;
+	h->node_codes = nullptr;
 	h->build_xf.clear();
-	h->level_nodes = nullptr;
 	h->instances.clear();
 	for(auto& b : h->scene_bufs) (void)hipFree(b.p);
 	h->scene_bufs.clear();
@@ -246,6 +243,55 @@ bool instance_dev(const ddgi_instance& in, const float* M, uint32_t prim_base, I
 	out.prim_base = prim_base;
 	out.mask = in.mask;
 	return true;
+}
+
+// The triangle slots (first, end) under every child of the wide tree's nodes, 4 per node (an empty child:
+// first >= end), and the nodes' child codes.  The slots are in the tree's leaf order, so a range holds
+// exactly its subtree's.
+void node_ranges(const BvhHost& bvh, std::vector<uint32_t>& range, std::vector<uint32_t>& codes) {
+	range.assign(size_t(bvh.node_count) * 8, 0u);
+	codes.resize(size_t(bvh.node_count) * 4);
+	for(size_t q = bvh.level_nodes.size(); q-- > 0;) {  // deepest level first
+		const size_t w = bvh.level_nodes[q];
+		for(uint32_t k = 0; k < kWide; ++k) {
+			uint32_t code;
+			std::memcpy(&code, &bvh.nodes[w * kNodeFloats + kCodeRow + k], 4);
+			codes[w * 4 + k] = code;
+			uint32_t first = 0xFFFFFFFFu, end = 0;
+			if(code == kEmptyChild) {
+				first = end = 0;
+			} else if(code & kLeafFlag) {
+				first = (code & ~kLeafFlag) >> 3;
+				end = first + (code & 7u) + 1u;
+			} else {
+				for(uint32_t c = 0; c < kWide; ++c) {
+					const uint32_t a = range[size_t(code) * 8 + 2 * c], b = range[size_t(code) * 8 + 2 * c + 1];
+					if(a >= b) continue;
+					first = std::min(first, a);
+					end = std::max(end, b);
+				}
+			}
+			range[w * 8 + 2 * k] = first;
+			range[w * 8 + 2 * k + 1] = end;
+		}
+	}
+}
+
+// Level sizes of the box tree over `slots` triangle slots, in steps of three levels; boxes in all.
+size_t box_tree_levels(uint32_t slots, BoxTree& tree) {
+	size_t total = 0;
+	uint32_t n = slots;
+	tree.levels = 0;
+	do {  // the slots and three levels, then three more as long as the last has many boxes
+		for(uint32_t end = tree.levels + (tree.levels == 0u ? 4u : 3u); tree.levels < end;) {
+			tree.first[tree.levels] = uint32_t(total);
+			tree.count[tree.levels] = n;
+			++tree.levels;
+			total += n;
+			n = (n + 7u) / 8u;
+		}
+	} while(tree.count[tree.levels - 1] > 8u);
+	return total;
 }
 
 ddgi_status make_rotation(const float* o, Rot& R) {
@@ -678,34 +724,41 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	std::vector<float> mats(material_count * 12);
 	for(size_t k = 0; k < material_count; ++k) std::memcpy(&mats[k * 12], &materials[k], 48);
 	const float4* nodes = nullptr;
-	const float4* boxes = nullptr;
 	const float4* tris = nullptr;
 	const InstanceDev* ip = nullptr;
 	const uint32_t* op = nullptr;
 	const uint32_t* ixp = nullptr;
 	const float4* vp = nullptr;
 	const float* mp = nullptr;
-	if((st = upload(h, reinterpret_cast<const float4*>(bvh.nodes.data()), bvh.nodes.size() / 4, &boxes)) != DDGI_OK ||
-	   (st = upload<float4>(h, nullptr, size_t(bvh.node_count) * (kPackedNodeBytes / 16), &nodes)) != DDGI_OK ||
+	std::vector<uint32_t> range, codes;
+	node_ranges(bvh, range, codes);
+	SlotBoxArgs sb{};
+	const size_t boxes = box_tree_levels(bvh.tri_count, sb.tree);
+	const float* box_mem = nullptr;
+	if((st = upload<float4>(h, nullptr, size_t(bvh.node_count) * (kPackedNodeBytes / 16), &nodes)) != DDGI_OK ||
 	   (st = upload(h, reinterpret_cast<const float4*>(bvh.tris.data()), bvh.tris.size() / 4, &tris)) != DDGI_OK ||
 	   (st = upload(h, inst.data(), inst.size(), &ip)) != DDGI_OK ||
 	   (st = upload(h, reinterpret_cast<const uint32_t*>(offsets), offset_count * 3, &op)) != DDGI_OK ||
 	   (st = upload(h, indices, index_count, &ixp)) != DDGI_OK ||
 	   (st = upload(h, reinterpret_cast<const float4*>(vertices), vertex_count * 4, &vp)) != DDGI_OK ||
 	   (st = upload(h, mats.data(), mats.size(), &mp)) != DDGI_OK ||
-	   (st = upload(h, bvh.obj_tris.data(), bvh.obj_tris.size(), &h->obj_tris)) != DDGI_OK ||
-	   (st = upload(h, bvh.slot_box.data(), bvh.slot_box.size(), &h->slot_box)) != DDGI_OK ||
-	   (st = upload(h, identity_xf(instance_count).data(), instance_count * 12, const_cast<const float**>(&h->rel_xf))) != DDGI_OK ||
-	   (st = upload(h, bvh.level_nodes.data(), bvh.level_nodes.size(), &h->level_nodes)) != DDGI_OK ||
-	   (st = upload<float>(h, nullptr, instance_count * 13, nullptr)) != DDGI_OK) {
+	   (st = upload(h, bvh.obj_tris.data(), bvh.obj_tris.size(), &sb.obj)) != DDGI_OK ||
+	   (st = upload(h, bvh.slot_box.data(), bvh.slot_box.size(), &sb.slot_box)) != DDGI_OK ||
+	   (st = upload(h, identity_xf(instance_count).data(), instance_count * 12, &sb.rel_xf)) != DDGI_OK ||
+	   (st = upload(h, reinterpret_cast<const uint2*>(range.data()), range.size() / 2, &h->node_range)) != DDGI_OK ||
+	   (st = upload(h, reinterpret_cast<const uint4*>(codes.data()), codes.size() / 4, &h->node_codes)) != DDGI_OK ||
+	   (st = upload<float>(h, nullptr, boxes * 6, &box_mem)) != DDGI_OK ||
+	   (st = upload<InstanceMove>(h, nullptr, instance_count, &sb.moves)) != DDGI_OK) {
 		free_scene(h);
 		return st;
 	}
-	h->move_xf = static_cast<float*>(h->scene_bufs.back().p);
-	h->move_meta = reinterpret_cast<uint32_t*>(h->move_xf + instance_count * 12);
+	sb.tris = const_cast<float4*>(tris);
+	sb.tri_count = bvh.tri_count;
+	sb.tree.boxes = const_cast<float*>(box_mem);
+	h->slots = sb;
 	if(!h->move_done) HIP_TRY(h, hipEventCreateWithFlags(&h->move_done, hipEventDisableTiming));
 	{
-		const hipError_t e = hipHostMalloc(&h->move_host, std::max<size_t>(instance_count * (25 * 4 + sizeof(InstanceDev)), 16),
+		const hipError_t e = hipHostMalloc(&h->move_host, std::max<size_t>(instance_count * sizeof(InstanceMove), 16),
 										   hipHostMallocDefault);
 		if(e != hipSuccess) {
 			h->move_host = nullptr;
@@ -717,15 +770,14 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	h->build_xf.resize(instance_count * 12);
 	for(size_t k = 0; k < instance_count; ++k) std::memcpy(&h->build_xf[k * 12], instances[k].transform, 48);
 	{  // the traversal's nodes, ready for any stream
-		hipError_t e = launch_pack_nodes(boxes, const_cast<float4*>(nodes), bvh.node_count, nullptr);
+		hipError_t e = launch_make_nodes(sb, h->node_range, h->node_codes, const_cast<float4*>(nodes), bvh.node_count, nullptr);
 		if(e == hipSuccess) e = hipStreamSynchronize(nullptr);
 		if(e != hipSuccess) {
 			free_scene(h);
-			return fail(h, DDGI_ERROR_HIP, std::string("packing the BVH nodes: ") + hipGetErrorString(e));
+			return fail(h, DDGI_ERROR_HIP, std::string("making the BVH nodes: ") + hipGetErrorString(e));
 		}
 	}
 	sd.nodes = nodes;
-	sd.boxes = const_cast<float4*>(boxes);
 	sd.tris = tris;
 	sd.inst = ip;
 	sd.offsets = op;
@@ -767,37 +819,29 @@ ddgi_status ddgi_update_instances(void* handle, uint32_t first, uint32_t count, 
 	if(st != DDGI_OK) return st;
 	if(h->move_pending) HIP_TRY(h, hipEventSynchronize(h->move_done));  // staging still read by the last call
 	h->move_pending = false;
-	float* xf = static_cast<float*>(h->move_host);
-	uint32_t* meta = reinterpret_cast<uint32_t*>(xf + n * 12);
-	InstanceDev* inst = reinterpret_cast<InstanceDev*>(meta + n);
-	float* rel = reinterpret_cast<float*>(inst + n);  // n * 12 floats
+	InstanceMove* mv = static_cast<InstanceMove*>(h->move_host);
 	for(uint32_t k = 0; k < count; ++k) {
 		const ddgi_instance& in = h->instances[first + k];
 		const float* M = transforms + size_t(k) * 12;
-		if(!instance_dev(in, M, h->bvh_meta.inst_prim_base[first + k], inst[k]))
+		if(!instance_dev(in, M, h->bvh_meta.inst_prim_base[first + k], mv[k].inst))
 			return fail(h, DDGI_ERROR_INVALID_ARGUMENT, "singular instance transform");
 		const double det = double(M[0]) * (double(M[5]) * M[10] - double(M[6]) * M[9]) -
 						   double(M[1]) * (double(M[4]) * M[10] - double(M[6]) * M[8]) +
 						   double(M[2]) * (double(M[4]) * M[9] - double(M[5]) * M[8]);
 		const bool flip = (det < 0.0) != ((in.flags & DDGI_INSTANCE_FLIP_FACING) != 0);
-		meta[k] = (in.mask & 0xFFu) | (flip ? 0x100u : 0u);
-		relative_transform(M, &h->build_xf[size_t(first + k) * 12], rel + size_t(k) * 12);
+		mv[k].meta = (in.mask & 0xFFu) | (flip ? 0x100u : 0u);
+		std::memcpy(mv[k].xf, M, 48);
+		relative_transform(M, &h->build_xf[size_t(first + k) * 12], mv[k].rel);
 	}
-	std::memcpy(xf, transforms, size_t(count) * 48);
 	hipStream_t s = static_cast<hipStream_t>(stream);
-	HIP_TRY(h, hipMemcpyAsync(h->move_xf, xf, size_t(count) * 48, hipMemcpyHostToDevice, s));
-	HIP_TRY(h, hipMemcpyAsync(h->move_meta, meta, size_t(count) * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-	HIP_TRY(h, hipMemcpyAsync(const_cast<InstanceDev*>(h->sd.inst) + first, inst, size_t(count) * sizeof(InstanceDev),
-							  hipMemcpyHostToDevice, s));
-	HIP_TRY(h, hipMemcpyAsync(h->rel_xf + size_t(first) * 12, rel, size_t(count) * 48, hipMemcpyHostToDevice, s));
-	float4* tris = const_cast<float4*>(h->sd.tris);
-	float4* nodes = h->sd.boxes;
-	HIP_TRY(h, launch_retransform(tris, h->obj_tris, h->sd.tri_count, h->move_xf, h->move_meta, first, count, s));
-	const std::vector<uint32_t>& lv = h->bvh_meta.level_offsets;
-	for(size_t d = lv.size() - 1; d >= 1; --d)
-		HIP_TRY(h, launch_refit_level(nodes, tris, h->slot_box, h->rel_xf, h->level_nodes + lv[d - 1], lv[d] - lv[d - 1], s));
-	HIP_TRY(h, launch_pack_nodes(nodes, const_cast<float4*>(h->sd.nodes), h->sd.node_count, s));
-	// the staging area and move_xf / move_meta are reused once this has run
+	SlotBoxArgs sb = h->slots;
+	sb.first = first;
+	sb.count = count;
+	// the kernel reads the staged moves from host memory: one launch in place of a copy per array
+	HIP_TRY(h, launch_apply_moves(mv, const_cast<InstanceMove*>(sb.moves), const_cast<InstanceDev*>(h->sd.inst),
+								  const_cast<float*>(sb.rel_xf), first, count, s));
+	HIP_TRY(h, launch_make_nodes(sb, h->node_range, h->node_codes, const_cast<float4*>(h->sd.nodes), h->sd.node_count, s));
+	// the staging area is reused once this has run
 	HIP_TRY(h, hipEventRecord(h->move_done, s));
 	h->move_pending = true;
 	for(uint32_t k = 0; k < count; ++k) std::memcpy(h->instances[first + k].transform, transforms + size_t(k) * 12, 48);

@@ -16,8 +16,8 @@
 //               [0] = (v0.xyz, global triangle id)   global id = instance-major flattened index
 //               [1] = (v1.xyz, instance index)
 //               [2] = (v2.xyz, mask | flip_facing << 8)
-// The traversal reads the nodes in a packed form made on the device (k_pack_nodes, kPackedNodeBytes each,
-// the same node indices and child codes); these full-precision ones are what a refit updates.
+// The traversal reads the nodes in a packed form made on the device from the slots' boxes (k_make_nodes,
+// kPackedNodeBytes each, the same node indices and child codes).
 // Node boxes are inflated by a few ulps so that FP32 slab tests stay conservative; an empty child
 // slot has the code kEmptyChild and a point box far outside any scene.
 #pragma once
@@ -39,7 +39,7 @@ constexpr uint32_t kNodeFloats = kWide == 4 ? 32 : 64;  // 6 box rows + 1 code r
 constexpr uint32_t kCodeRow = 6 * kWide;               // float offset of the child codes
 constexpr uint32_t kMaxWideDepth = 32;   // traversal stack: kWide - 1 entries per level
 static_assert(kWide == 4 || kWide == 8, "nodes are 4- or 8-wide");
-constexpr uint32_t kPackedNodeBytes = 80;  // the traversal's form of a 4-wide node (trace.hip, k_pack_nodes)
+constexpr uint32_t kPackedNodeBytes = 80;  // the traversal's form of a 4-wide node (trace.hip, k_make_nodes)
 
 struct BvhHost {
 	std::vector<float> nodes;     // kNodeFloats per node

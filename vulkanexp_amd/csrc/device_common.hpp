@@ -122,7 +122,7 @@ struct HitResult {
 
 // Closest-hit (ANY = false; ties -> lowest global id) or any-hit traversal of the BVH.
 //
-// Nodes are 4-wide, in the packed form of k_pack_nodes: five 16-byte loads test four child boxes.  A
+// Nodes are 4-wide, in the packed form of k_make_nodes: five 16-byte loads test four child boxes.  A
 // wavefront runs until its longest ray ends with about a third of its lanes active, so what bounds the
 // traversal is what a visit costs per wavefront: vector instructions (79 % of the SIMDs' issue cycles
 // with FP32 boxes) and vector loads, whose data return costs about 22 cycles per load of the CU however

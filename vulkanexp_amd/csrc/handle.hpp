@@ -69,18 +69,14 @@ struct Handle {
 	bool has_scene = false;
 	BvhHost bvh_meta;
 	size_t bvh_bytes = 0;
-	// instance moves (ddgi_update_instances): the scene's instance records, the triangles'
-	// object-space vertices in BVH slot order and the wide nodes by level; the moved instances'
-	// transforms (12 floats), triangle meta words and InstanceDev records pass through a pinned
-	// staging area (`move_host`, reused once `move_done` has fired) to `move_xf` / `move_meta`
+	// instance moves (ddgi_update_instances): the scene's instance records, what the boxes and nodes are
+	// made from (launch_make_nodes), and the moves, which pass through a pinned staging area
+	// (`move_host`, reused once `move_done` has fired)
 	std::vector<ddgi_instance> instances;
-	const float* obj_tris = nullptr;
-	const float* slot_box = nullptr;  // the builder's piece bounds per slot (BvhHost::slot_box)
-	float* rel_xf = nullptr;          // per instance: current transform after the inverse of the build's (3x4)
+	SlotBoxArgs slots{};              // moves: the device copy of the last moves
+	const uint2* node_range = nullptr;  // triangle slots under each child, 4 per node
+	const uint4* node_codes = nullptr;  // child codes per node
 	std::vector<float> build_xf;      // per instance: the transform the BVH was built with
-	const uint32_t* level_nodes = nullptr;
-	float* move_xf = nullptr;
-	uint32_t* move_meta = nullptr;
 	void* move_host = nullptr;
 	hipEvent_t move_done = nullptr;
 	bool move_pending = false;

@@ -57,7 +57,6 @@ struct InstanceDev {
 
 struct SceneDev {
 	const float4* nodes;       // the traversal's packed nodes (kPackedNodeBytes each)
-	float4* boxes;             // the same nodes with FP32 boxes (kNodeFloats each), which refits update
 	const float4* tris;
 	const InstanceDev* inst;
 	const uint32_t* offsets;   // 3 per entry (material, vertex offset, index offset)
@@ -68,6 +67,34 @@ struct SceneDev {
 	uint32_t node_count;
 	uint32_t instance_count;
 	uint32_t stack_depth;      // most stack entries a traversal needs (3 per level of the 4-wide tree)
+};
+
+// One moved instance: its transform, its motion since the BVH was built (both row-major 3x4), the triangle
+// records' meta word (mask | flip << 8) and its shading record.
+struct InstanceMove {
+	float xf[12];
+	float rel[12];
+	InstanceDev inst;
+	uint32_t meta;
+};
+
+// Boxes (6 floats: lo, hi) of the triangle slots (level 0) and of 8, 64, 512, ... consecutive ones: level
+// l has count[l] boxes from box first[l] on.
+constexpr uint32_t kBoxLevels = 12;
+struct BoxTree {
+	float* boxes;
+	uint32_t levels;
+	uint32_t first[kBoxLevels], count[kBoxLevels];
+};
+
+struct SlotBoxArgs {
+	float4* tris;
+	const float* obj;        // object-space vertices per slot (9 floats)
+	const float* slot_box;   // the builder's piece bounds per slot
+	const float* rel_xf;     // per instance its motion since the build (3x4)
+	const InstanceMove* moves;  // of instances first .. first + count - 1
+	uint32_t first, count, tri_count;
+	BoxTree tree;
 };
 
 // Internal hit record: (t, slot | back << 31, u, v); slot = triangle position in the BVH array,
@@ -241,16 +268,14 @@ hipError_t launch_shade(const TraceFrameArgs& a, hipStream_t s);
 hipError_t launch_sky(const TraceFrameArgs& a, hipStream_t s);
 hipError_t launch_trace_rays(const SceneDev& sc, const ddgi_ray* rays, ddgi_hit* hits, uint64_t count, uint32_t mask,
 							 bool any_hit, bool cull, hipStream_t s);
-// Instance moves: re-transform the triangles of instances [first, first + count) (xf: 12 floats,
-// meta: mask | flip << 8 per moved instance), then refit the wide tree level by level, deepest
-// first (slot_box: the builder's piece bounds per slot; rel_xf: per instance its motion since the
-// build, 3x4).
-hipError_t launch_retransform(float4* tris, const float* obj, uint32_t tri_count, const float* xf, const uint32_t* meta,
+// Traversal nodes (kPackedNodeBytes each) of `node_count` wide nodes whose children cover the slot ranges
+// `range` (4 per node, first >= second: empty), after re-transforming the triangles of moved instances.
+hipError_t launch_make_nodes(const SlotBoxArgs& a, const uint2* range, const uint4* codes, float4* packed,
+							 uint32_t node_count, hipStream_t s);
+// Copies `count` staged moves (host memory the device can read) to `moves`, and their records to the
+// instances' shading records and motions.
+hipError_t launch_apply_moves(const InstanceMove* staged, InstanceMove* moves, InstanceDev* inst, float* rel_xf,
 							  uint32_t first, uint32_t count, hipStream_t s);
-// Traversal nodes (kPackedNodeBytes each) of `count` wide nodes.
-hipError_t launch_pack_nodes(const float4* nodes, float4* packed, uint32_t count, hipStream_t s);
-hipError_t launch_refit_level(float4* nodes, const float4* tris, const float* slot_box, const float* rel_xf,
-							  const uint32_t* level_nodes, uint32_t count, hipStream_t s);
 hipError_t launch_gbuffer(const SceneDev& sc, const ddgi_ray* rays, uint64_t count, ddgi_gbuffer_texel* out, hipStream_t s);
 hipError_t launch_gather(const GatherArgs& a, hipStream_t s);
 hipError_t launch_direct_light(const DirectLightArgs& a, hipStream_t s);

@@ -6,6 +6,7 @@
 //
 // Built with -ffp-contract=off (see device_common.hpp).
 #include <algorithm>
+#include <cstddef>
 #include <type_traits>
 #include <vector>
 
@@ -942,39 +943,222 @@ __global__ __launch_bounds__(kShadeBlock, 5) void k_reflection_shade(ReflectionA
 	}
 }
 
-// ---- traversal nodes ----
-// The traversal's 80-byte form of a wide node (one thread per node): the origin and scale of the
-// node's grid (scale a power of two), the children's planes as FP16 integers 0..2047 on it, rounded
-// outward, in rows x, y, z of (lo of 4 children, hi of 4 children), and the child codes (80 bytes where
-// FP32 boxes take 128; 11 bits keep the boxes tight enough that no more nodes are visited).  A plane is
-// origin + q * scale; the traversal's distance fma(q, scale / d, (origin - o) / d) is off by at most
-// about 2.4e-7 of the node's size (in position) beside the errors relative to the distance that the
-// far end's widening covers, so the boxes are first grown by 1e-6 of that size.  An empty child gets
-// an inverted box, which no ray enters; a node too large for the grid gets infinite ones.
-__global__ void k_pack_nodes(const float4* __restrict__ nodes, float4* __restrict__ packed, uint32_t count) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if(i >= count) return;
-	const float4* src = nodes + size_t(i) * (kNodeFloats / 4);
-	float lo[3][4], hi[3][4];
+// ---- traversal nodes, and instance moves (the TLAS instance update + refit of
+// src/Renderer.cpp:671-742) ----
+// A child box of the wide tree bounds a contiguous range of triangle slots, so no box waits for another
+// one: every slot's box, then the boxes of 8, 64, 512, ... consecutive slots (BoxTree), and then every
+// child's box from the at most 14 boxes per level that its range takes.  Three launches whatever the
+// tree's depth (a launch per level, one thread per node, took 270 us for 22 k nodes on 13 levels; this
+// takes about 20).  Setting a scene makes its nodes the same way.
+__device__ __forceinline__ float pad_down_dev(float v) {
+	const double d = double(v) - (fabs(double(v)) * 1e-6 + 1e-6);
+	float f = float(d);
+	if(double(f) > d) f = nextafterf(f, -__int_as_float(0x7f800000));
+	return f;
+}
+__device__ __forceinline__ float pad_up_dev(float v) {
+	const double d = double(v) + (fabs(double(v)) * 1e-6 + 1e-6);
+	float f = float(d);
+	if(double(f) < d) f = nextafterf(f, __int_as_float(0x7f800000));
+	return f;
+}
+
+struct Box6 {
+	float lo[3], hi[3];
+};
+__device__ __forceinline__ Box6 empty_box() {
+	return {{3.402823466e+38f, 3.402823466e+38f, 3.402823466e+38f}, {-3.402823466e+38f, -3.402823466e+38f, -3.402823466e+38f}};
+}
+__device__ __forceinline__ void grow(Box6& b, const float* lo, const float* hi) {
 #pragma unroll
 	for(int a = 0; a < 3; ++a) {
-		const float4 l = src[2 * a], h = src[2 * a + 1];
-		lo[a][0] = l.x, lo[a][1] = l.y, lo[a][2] = l.z, lo[a][3] = l.w;
-		hi[a][0] = h.x, hi[a][1] = h.y, hi[a][2] = h.z, hi[a][3] = h.w;
+		b.lo[a] = fminf(b.lo[a], lo[a]);
+		b.hi[a] = fmaxf(b.hi[a], hi[a]);
 	}
-	const float4 cd = src[6];
-	const uint32_t code[4] = {__float_as_uint(cd.x), __float_as_uint(cd.y), __float_as_uint(cd.z), __float_as_uint(cd.w)};
+}
+// The union over groups of eight lanes, in each of them.
+__device__ __forceinline__ void union8(Box6& b) {
+#pragma unroll
+	for(int o = 1; o < 8; o <<= 1) {
+#pragma unroll
+		for(int a = 0; a < 3; ++a) {
+			b.lo[a] = fminf(b.lo[a], __shfl_xor(b.lo[a], o));
+			b.hi[a] = fmaxf(b.hi[a], __shfl_xor(b.hi[a], o));
+		}
+	}
+}
+__device__ __forceinline__ void store_box(float* dst, const Box6& b) {
+	for(int a = 0; a < 3; ++a) {
+		dst[a] = b.lo[a];
+		dst[3 + a] = b.hi[a];
+	}
+}
+
+// The three levels above level `level` from the boxes of a workgroup of 512 threads (thread t: box
+// blockIdx * 512 + t of that level): 64, 8 and 1 boxes per workgroup.
+__device__ __forceinline__ void build_levels(const BoxTree& tree, uint32_t level, Box6 b, float* s_box) {
+	const uint32_t t = threadIdx.x, i = blockIdx.x * 512u + t;
+	union8(b);
+	if((t & 7u) == 0u) {
+		store_box(s_box + (t >> 3) * 6, b);
+		if((i >> 3) < tree.count[level + 1]) store_box(tree.boxes + (size_t(tree.first[level + 1]) + (i >> 3)) * 6, b);
+	}
+	__syncthreads();
+	if(t < 64u) {
+		Box6 c = empty_box();
+		grow(c, s_box + t * 6, s_box + t * 6 + 3);
+		union8(c);
+		const uint32_t q = blockIdx.x * 8u + (t >> 3);
+		if((t & 7u) == 0u && q < tree.count[level + 2]) store_box(tree.boxes + (size_t(tree.first[level + 2]) + q) * 6, c);
+#pragma unroll
+		for(int o = 8; o < 64; o <<= 1)
+#pragma unroll
+			for(int a = 0; a < 3; ++a) {
+				c.lo[a] = fminf(c.lo[a], __shfl_xor(c.lo[a], o));
+				c.hi[a] = fmaxf(c.hi[a], __shfl_xor(c.hi[a], o));
+			}
+		if(t == 0u && blockIdx.x < tree.count[level + 3]) store_box(tree.boxes + (size_t(tree.first[level + 3]) + blockIdx.x) * 6, c);
+	}
+}
+
+// One thread per triangle slot.  A triangle of a moved instance gets its new world vertices: each row of
+// the row-major 3x4 transform evaluated in double left to right and rounded once to float, exactly as
+// the host flattening (bvh.cpp transform_point), so a moved scene traces like a freshly built one.  Then
+// the slot's box: the triangle's, clipped by the box of the piece that the slot holds (a spatial split may
+// have cut it; the piece's box at the build, carried by the instance's motion since as the box of its 8
+// moved corners, in double, rounded outward).
+__global__ __launch_bounds__(512) void k_slot_boxes(SlotBoxArgs a) {
+	__shared__ float s_box[64 * 6];
+	const uint32_t slot = blockIdx.x * 512u + threadIdx.x;
+	Box6 box = empty_box();
+	if(slot < a.tri_count) {
+		float4* t = a.tris + size_t(slot) * 3;
+		float4 v[3] = {t[0], t[1], t[2]};
+		const uint32_t inst = __float_as_uint(v[1].w), k = inst - a.first;  // wraps for instances below `first`
+		const float* rel = a.rel_xf + size_t(inst) * 12;
+		if(k < a.count) {
+			const float* M = a.moves[k].xf;
+			rel = a.moves[k].rel;
+			v[2].w = __uint_as_float(a.moves[k].meta);
+#pragma unroll
+			for(int q = 0; q < 3; ++q) {
+				const float* p = a.obj + size_t(slot) * 9 + q * 3;
+				float w[3];
+				for(int r = 0; r < 3; ++r) {
+					double acc = double(M[r * 4 + 0]) * double(p[0]);
+					acc = acc + double(M[r * 4 + 1]) * double(p[1]);
+					acc = acc + double(M[r * 4 + 2]) * double(p[2]);
+					acc = acc + double(M[r * 4 + 3]);
+					w[r] = float(acc);
+				}
+				v[q].x = w[0];
+				v[q].y = w[1];
+				v[q].z = w[2];
+				t[q] = v[q];
+			}
+		}
+#pragma unroll
+		for(int q = 0; q < 3; ++q) {
+			const float p[3] = {v[q].x, v[q].y, v[q].z};
+			grow(box, p, p);
+		}
+		const float* bx = a.slot_box + size_t(slot) * 6;
+		double mlo[3] = {1e300, 1e300, 1e300}, mhi[3] = {-1e300, -1e300, -1e300};
+		for(int c = 0; c < 8; ++c) {
+			const double p[3] = {bx[(c & 1) ? 3 : 0], bx[(c & 2) ? 4 : 1], bx[(c & 4) ? 5 : 2]};
+			for(int r = 0; r < 3; ++r) {
+				const double q = double(rel[r * 4 + 0]) * p[0] + double(rel[r * 4 + 1]) * p[1] + double(rel[r * 4 + 2]) * p[2] +
+								 double(rel[r * 4 + 3]);
+				mlo[r] = fmin(mlo[r], q);
+				mhi[r] = fmax(mhi[r], q);
+			}
+		}
+#pragma unroll
+		for(int r = 0; r < 3; ++r) {
+			float flo = float(mlo[r]), fhi = float(mhi[r]);
+			if(double(flo) > mlo[r]) flo = nextafterf(flo, -__int_as_float(0x7f800000));
+			if(double(fhi) < mhi[r]) fhi = nextafterf(fhi, __int_as_float(0x7f800000));
+			box.lo[r] = fmaxf(box.lo[r], flo);
+			box.hi[r] = fminf(box.hi[r], fhi);
+		}
+		store_box(a.tree.boxes + size_t(slot) * 6, box);
+	}
+	build_levels(a.tree, 0u, box, s_box);
+}
+
+// Levels level + 1 .. level + 3 of the box tree.
+__global__ __launch_bounds__(512) void k_box_levels(BoxTree tree, uint32_t level) {
+	__shared__ float s_box[64 * 6];
+	const uint32_t i = blockIdx.x * 512u + threadIdx.x;
+	Box6 b = empty_box();
+	if(i < tree.count[level]) {
+		const float* p = tree.boxes + (size_t(tree.first[level]) + i) * 6;
+		grow(b, p, p + 3);
+	}
+	build_levels(tree, level, b, s_box);
+}
+
+// The shading records and motions of the moved instances, from the moves staged in host memory.
+__global__ void k_apply_moves(const InstanceMove* __restrict__ staged, InstanceMove* __restrict__ moves,
+							  InstanceDev* __restrict__ inst, float* __restrict__ rel_xf, uint32_t first, uint32_t count) {
+	const uint32_t words = count * uint32_t(sizeof(InstanceMove) / 4);
+	for(uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < words; q += gridDim.x * blockDim.x) {
+		const uint32_t k = q / uint32_t(sizeof(InstanceMove) / 4), w = q - k * uint32_t(sizeof(InstanceMove) / 4);
+		const uint32_t v = reinterpret_cast<const uint32_t*>(staged)[q];
+		reinterpret_cast<uint32_t*>(moves)[q] = v;
+		constexpr uint32_t kRel = offsetof(InstanceMove, rel) / 4, kInst = offsetof(InstanceMove, inst) / 4;
+		if(w >= kRel && w < kRel + 12u) rel_xf[size_t(first + k) * 12 + (w - kRel)] = __uint_as_float(v);
+		if(w >= kInst && w < kInst + uint32_t(sizeof(InstanceDev) / 4))
+			reinterpret_cast<uint32_t*>(inst + first + k)[w - kInst] = v;
+	}
+}
+
+// The traversal's 80-byte form of a wide node: the origin and scale of the node's grid (scale a power of
+// two), the children's planes as FP16 integers 0..2047 on it, rounded outward, in rows x, y, z of (lo of 4
+// children, hi of 4 children), and the child codes (80 bytes where FP32 boxes take 128; 11 bits keep the
+// boxes tight enough that no more nodes are visited).  A plane is origin + q * scale; the traversal's
+// distance fma(q, scale / d, (origin - o) / d) is off by at most about 2.4e-7 of the node's size (in
+// position) beside the errors relative to the distance that the far end's widening covers, so the padded
+// boxes are first grown by 1e-6 of that size.  An empty child gets an inverted box, which no ray enters; a
+// node too large for the grid gets infinite ones.
+// 32 lanes per node, eight per child: `range` holds each child's triangle slots (first, end), and lane j of
+// a child takes the j-th box of either end of its range on every level.
+__global__ __launch_bounds__(256) void k_make_nodes(BoxTree tree, const uint2* __restrict__ range,
+													const uint4* __restrict__ codes, float4* __restrict__ packed, uint32_t count) {
+	const uint32_t node = blockIdx.x * 8u + (threadIdx.x >> 5);
+	if(node >= count) return;  // whole halves of a wavefront
+	const uint32_t lane = __lane_id(), j = lane & 7u, child = (lane >> 3) & 3u;
+	const uint2 r = range[size_t(node) * 4 + child];
+	const bool empty = r.x >= r.y;
+	Box6 b = empty_box();
+	uint32_t lo = r.x, hi = r.y;
+	for(uint32_t level = 0; lo < hi; ++level) {
+		const float* boxes = tree.boxes + size_t(tree.first[level]) * 6;
+		const uint32_t l8 = (lo + 7u) & ~7u, h8 = hi & ~7u;
+		if(l8 >= h8 || level + 1u >= tree.levels) {  // the rest on this level
+			for(uint32_t i = lo + j; i < hi; i += 8u) grow(b, boxes + size_t(i) * 6, boxes + size_t(i) * 6 + 3);
+			break;
+		}
+		if(lo + j < l8) grow(b, boxes + size_t(lo + j) * 6, boxes + size_t(lo + j) * 6 + 3);
+		if(h8 + j < hi) grow(b, boxes + size_t(h8 + j) * 6, boxes + size_t(h8 + j) * 6 + 3);
+		lo = l8 >> 3;
+		hi = h8 >> 3;
+	}
+	union8(b);
 	double mn[3], mx[3], size = 0.0;
 #pragma unroll
 	for(int a = 0; a < 3; ++a) {
-		mn[a] = 1e300;
-		mx[a] = -1e300;
-#pragma unroll
-		for(int k = 0; k < 4; ++k) {
-			if(code[k] == kEmptyChild) continue;
-			mn[a] = fmin(mn[a], double(lo[a][k]));
-			mx[a] = fmax(mx[a], double(hi[a][k]));
+		if(!empty) {
+			b.lo[a] = pad_down_dev(b.lo[a]);
+			b.hi[a] = pad_up_dev(b.hi[a]);
 		}
+		float l = b.lo[a], h = b.hi[a];  // over the node's four children
+		l = fminf(l, __shfl_xor(l, 8));
+		l = fminf(l, __shfl_xor(l, 16));
+		h = fmaxf(h, __shfl_xor(h, 8));
+		h = fmaxf(h, __shfl_xor(h, 16));
+		mn[a] = double(l);
+		mx[a] = double(h);
 		size = fmax(size, mx[a] - mn[a]);
 	}
 	const double slack = size * 1e-6;
@@ -992,145 +1176,30 @@ __global__ void k_pack_nodes(const float4* __restrict__ nodes, float4* __restric
 	sb = (sb + 0x007FFFFFu) & 0x7F800000u;
 	const float scale = fits ? __uint_as_float(sb) : 1.0f;
 	const double inv = 1.0 / double(scale);
-	float4* dst = reinterpret_cast<float4*>(reinterpret_cast<char*>(packed) + size_t(i) * kPackedNodeBytes);
-	dst[0] = fits ? make_float4(org[0], org[1], org[2], scale) : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
-	typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-	const _Float16 inf = __builtin_bit_cast(_Float16, (unsigned short)0x7C00);
+	float4* dst = reinterpret_cast<float4*>(reinterpret_cast<char*>(packed) + size_t(node) * kPackedNodeBytes);
+	const uint32_t base = lane & 32u;  // the node's first lane
 #pragma unroll
 	for(int a = 0; a < 3; ++a) {
-		half4_t q[2];
+		const double l = floor((double(b.lo[a]) - slack - double(org[a])) * inv);
+		const double h = ceil((double(b.hi[a]) + slack - double(org[a])) * inv);
+		// FP16 bits: the integers, 65504 / -65504 for an empty child, -inf / inf beyond the grid
+		const auto bits = [](double q) {
+			return uint32_t(__builtin_bit_cast(unsigned short, _Float16(float(fmin(fmax(q, 0.0), 2047.0)))));
+		};
+		const uint32_t ql = empty ? 0x7BFFu : (fits ? bits(l) : 0xFC00u), qh = empty ? 0xFBFFu : (fits ? bits(h) : 0x7C00u);
+		const int q = int(ql | (qh << 16));
+		uint32_t c[4];
 #pragma unroll
-		for(int k = 0; k < 4; ++k) {
-			const double l = floor((double(lo[a][k]) - slack - double(org[a])) * inv);
-			const double h = ceil((double(hi[a][k]) + slack - double(org[a])) * inv);
-			const bool empty = code[k] == kEmptyChild;
-			q[0][k] = empty ? _Float16(65504.0f) : (fits ? _Float16(float(fmin(fmax(l, 0.0), 2047.0))) : _Float16(-inf));
-			q[1][k] = empty ? _Float16(-65504.0f) : (fits ? _Float16(float(fmin(fmax(h, 0.0), 2047.0))) : inf);
-		}
-		struct Row {
-			half4_t lo, hi;
-		} row{q[0], q[1]};
-		dst[1 + a] = __builtin_bit_cast(float4, row);
+		for(int k = 0; k < 4; ++k) c[k] = uint32_t(__shfl(q, int(base) + 8 * k));
+		if((lane & 31u) == uint32_t(a))
+			dst[1 + a] = make_float4(__uint_as_float((c[0] & 0xFFFFu) | (c[1] << 16)), __uint_as_float((c[2] & 0xFFFFu) | (c[3] << 16)),
+									 __uint_as_float((c[0] >> 16) | (c[1] & 0xFFFF0000u)),
+									 __uint_as_float((c[2] >> 16) | (c[3] & 0xFFFF0000u)));
 	}
-	dst[4] = cd;
-}
-
-// ---- instance moves (the TLAS instance update + refit of src/Renderer.cpp:671-742) ----
-// World vertices of the triangles of instances [first, first + count): each row of the row-major
-// 3x4 transform evaluated in double left to right and rounded once to float, exactly as the host
-// flattening (bvh.cpp transform_point), so a moved scene traces like a freshly built one.  `meta`
-// holds mask | flip << 8 per moved instance.
-__global__ void k_retransform(float4* __restrict__ tris, const float* __restrict__ obj, uint32_t tri_count,
-							  const float* __restrict__ xf, const uint32_t* __restrict__ meta, uint32_t first,
-							  uint32_t count) {
-	const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-	if(slot >= tri_count) return;
-	float4* t = tris + size_t(slot) * 3;
-	const uint32_t k = __float_as_uint(t[1].w) - first;  // wraps for instances below `first`
-	if(k >= count) return;
-	const float* M = xf + size_t(k) * 12;
-	for(int v = 0; v < 3; ++v) {
-		const float* p = obj + size_t(slot) * 9 + v * 3;
-		float w[3];
-		for(int r = 0; r < 3; ++r) {
-			double acc = double(M[r * 4 + 0]) * double(p[0]);
-			acc = acc + double(M[r * 4 + 1]) * double(p[1]);
-			acc = acc + double(M[r * 4 + 2]) * double(p[2]);
-			acc = acc + double(M[r * 4 + 3]);
-			w[r] = float(acc);
-		}
-		const float4 old = t[v];
-		t[v] = make_float4(w[0], w[1], w[2], v == 2 ? __uint_as_float(meta[k]) : old.w);
-	}
-}
-
-__device__ __forceinline__ float pad_down_dev(float v) {
-	const double d = double(v) - (fabs(double(v)) * 1e-6 + 1e-6);
-	float f = float(d);
-	if(double(f) > d) f = nextafterf(f, -__int_as_float(0x7f800000));
-	return f;
-}
-__device__ __forceinline__ float pad_up_dev(float v) {
-	const double d = double(v) + (fabs(double(v)) * 1e-6 + 1e-6);
-	float f = float(d);
-	if(double(f) < d) f = nextafterf(f, __int_as_float(0x7f800000));
-	return f;
-}
-
-// Refit of one level of the wide tree (deeper levels already refitted): every child box of the
-// level's nodes becomes the padded bounds of its triangles (leaf) or of its child node's boxes.
-__global__ void k_refit_level(float4* __restrict__ nodes, const float4* __restrict__ tris,
-							  const float* __restrict__ slot_box, const float* __restrict__ rel_xf,
-							  const uint32_t* __restrict__ level_nodes, uint32_t count) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if(i >= count) return;
-	float* rec = reinterpret_cast<float*>(nodes + size_t(level_nodes[i]) * (kNodeFloats / 4));
-	for(int k = 0; k < int(kWide); ++k) {
-		const uint32_t code = __float_as_uint(rec[kCodeRow + k]);
-		if(code == kEmptyChild) continue;
-		float lo[3] = {3.402823466e+38f, 3.402823466e+38f, 3.402823466e+38f};
-		float hi[3] = {-3.402823466e+38f, -3.402823466e+38f, -3.402823466e+38f};
-		if(code & kLeafFlag) {
-			const uint32_t firstt = (code & ~kLeafFlag) >> 3, cnt = (code & 7u) + 1u;
-			for(uint32_t q = 0; q < cnt; ++q) {
-				const size_t slot = size_t(firstt + q);
-				float tlo[3] = {3.402823466e+38f, 3.402823466e+38f, 3.402823466e+38f};
-				float thi[3] = {-3.402823466e+38f, -3.402823466e+38f, -3.402823466e+38f};
-				for(int v = 0; v < 3; ++v) {
-					const float4 p = tris[slot * 3 + v];
-					const float c[3] = {p.x, p.y, p.z};
-					for(int a = 0; a < 3; ++a) {
-						tlo[a] = fminf(tlo[a], c[a]);
-						thi[a] = fmaxf(thi[a], c[a]);
-					}
-				}
-				// the slot bounds only its piece of the triangle (a spatial split may have cut it): the
-				// piece's box at the build, carried by the instance's motion since (the box of its 8
-				// moved corners, in double, rounded outward), clips the triangle's box
-				{
-					const float* M = rel_xf + size_t(__float_as_uint(tris[slot * 3 + 1].w)) * 12;
-					const float* bx = slot_box + slot * 6;
-					double mlo[3] = {1e300, 1e300, 1e300}, mhi[3] = {-1e300, -1e300, -1e300};
-					for(int c = 0; c < 8; ++c) {
-						const double p[3] = {bx[(c & 1) ? 3 : 0], bx[(c & 2) ? 4 : 1], bx[(c & 4) ? 5 : 2]};
-						for(int r = 0; r < 3; ++r) {
-							const double q = double(M[r * 4 + 0]) * p[0] + double(M[r * 4 + 1]) * p[1] +
-											 double(M[r * 4 + 2]) * p[2] + double(M[r * 4 + 3]);
-							mlo[r] = fmin(mlo[r], q);
-							mhi[r] = fmax(mhi[r], q);
-						}
-					}
-					for(int a = 0; a < 3; ++a) {
-						float flo = float(mlo[a]), fhi = float(mhi[a]);
-						if(double(flo) > mlo[a]) flo = nextafterf(flo, -__int_as_float(0x7f800000));
-						if(double(fhi) < mhi[a]) fhi = nextafterf(fhi, __int_as_float(0x7f800000));
-						tlo[a] = fmaxf(tlo[a], flo);
-						thi[a] = fminf(thi[a], fhi);
-					}
-				}
-				for(int a = 0; a < 3; ++a) {
-					lo[a] = fminf(lo[a], tlo[a]);
-					hi[a] = fmaxf(hi[a], thi[a]);
-				}
-			}
-			for(int a = 0; a < 3; ++a) {
-				lo[a] = pad_down_dev(lo[a]);
-				hi[a] = pad_up_dev(hi[a]);
-			}
-		} else {  // the child's padded boxes already bound it
-			const float* ch = reinterpret_cast<const float*>(nodes + size_t(code) * (kNodeFloats / 4));
-			for(int c = 0; c < int(kWide); ++c) {
-				if(__float_as_uint(ch[kCodeRow + c]) == kEmptyChild) continue;
-				for(int a = 0; a < 3; ++a) {
-					lo[a] = fminf(lo[a], ch[(2 * a) * kWide + c]);
-					hi[a] = fmaxf(hi[a], ch[(2 * a + 1) * kWide + c]);
-				}
-			}
-		}
-		for(int a = 0; a < 3; ++a) {
-			rec[(2 * a) * kWide + k] = lo[a];
-			rec[(2 * a + 1) * kWide + k] = hi[a];
-		}
+	if((lane & 31u) == 3u) dst[0] = fits ? make_float4(org[0], org[1], org[2], scale) : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
+	if((lane & 31u) == 4u) {
+		const uint4 c = codes[node];
+		dst[4] = make_float4(__uint_as_float(c.x), __uint_as_float(c.y), __uint_as_float(c.z), __uint_as_float(c.w));
 	}
 }
 
@@ -1374,25 +1443,22 @@ hipError_t launch_trace_rays(const SceneDev& sc, const ddgi_ray* rays, ddgi_hit*
 	return hipGetLastError();
 }
 
-hipError_t launch_retransform(float4* tris, const float* obj, uint32_t tri_count, const float* xf, const uint32_t* meta,
+hipError_t launch_make_nodes(const SlotBoxArgs& a, const uint2* range, const uint4* codes, float4* packed,
+							 uint32_t node_count, hipStream_t s) {
+	if(a.tri_count == 0 || node_count == 0) return hipSuccess;
+	hipLaunchKernelGGL(k_slot_boxes, dim3(blocks_for(a.tri_count, 512)), dim3(512), 0, s, a);
+	for(uint32_t level = 3; level + 3u < a.tree.levels; level += 3)
+		hipLaunchKernelGGL(k_box_levels, dim3(blocks_for(a.tree.count[level], 512)), dim3(512), 0, s, a.tree, level);
+	hipLaunchKernelGGL(k_make_nodes, dim3(blocks_for(node_count, 8)), dim3(256), 0, s, a.tree, range, codes, packed, node_count);
+	return hipGetLastError();
+}
+
+hipError_t launch_apply_moves(const InstanceMove* staged, InstanceMove* moves, InstanceDev* inst, float* rel_xf,
 							  uint32_t first, uint32_t count, hipStream_t s) {
-	if(tri_count == 0 || count == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_retransform, dim3(blocks_for(tri_count, 256)), dim3(256), 0, s, tris, obj, tri_count, xf, meta,
-					   first, count);
-	return hipGetLastError();
-}
-
-hipError_t launch_pack_nodes(const float4* nodes, float4* packed, uint32_t count, hipStream_t s) {
 	if(count == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_pack_nodes, dim3(blocks_for(count, 128)), dim3(128), 0, s, nodes, packed, count);
-	return hipGetLastError();
-}
-
-hipError_t launch_refit_level(float4* nodes, const float4* tris, const float* slot_box, const float* rel_xf,
-							  const uint32_t* level_nodes, uint32_t count, hipStream_t s) {
-	if(count == 0) return hipSuccess;
-	hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(count, 128)), dim3(128), 0, s, nodes, tris, slot_box, rel_xf,
-					   level_nodes, count);
+	const uint64_t words = uint64_t(count) * (sizeof(InstanceMove) / 4);
+	hipLaunchKernelGGL(k_apply_moves, dim3(uint32_t(std::min<uint64_t>((words + 255) / 256, 1024))), dim3(256), 0, s, staged,
+					   moves, inst, rel_xf, first, count);
 	return hipGetLastError();
 }
 
