@@ -50,26 +50,20 @@ __device__ __forceinline__ TexelWeights make_weights(const DiffArgs& d, uint64_t
 #pragma unroll
 	for(int i = 0; i < 8; ++i) c.w[i] = c.fw[i] = 0.0f;
 	const Vec3 position = load3(d.pos, x), normal = load3(d.nrm, x), to_camera = load3(d.tocam, x);
-	const Vec3 acell = v3(fabsf(g.cell[0]), fabsf(g.cell[1]), fabsf(g.cell[2]));
-	const Vec3 emin = v3(g.emin[0], g.emin[1], g.emin[2]);
-	const Vec3 gc = v3((position.x - emin.x) / acell.x, (position.y - emin.y) / acell.y, (position.z - emin.z) / acell.z);
-	if(gc.x < 0.0f || gc.y < 0.0f || gc.z < 0.0f) return c;
+	Cage cage;
+	if(!make_cage(g, position, cage)) return c;
 	const Vec3 biased = position + (normal + to_camera) * g.shadow_bias;
-	const int f0 = int(gc.x), f1 = int(gc.y), f2 = int(gc.z);
-	const Vec3 p0 = v3(float(f0) * g.cell[0] + emin.x, float(f1) * g.cell[1] + emin.y, float(f2) * g.cell[2] + emin.z);
-	Vec3 alpha = v3((position.x - p0.x) / acell.x, (position.y - p0.y) / acell.y, (position.z - p0.z) / acell.z);
-	alpha = v3(fminf(fmaxf(alpha.x, 0.0f), 1.0f), fminf(fmaxf(alpha.y, 0.0f), 1.0f), fminf(fmaxf(alpha.z, 0.0f), 1.0f));
 	float cu, cv;
 	oct_uv(normal.x, normal.y, normal.z, cu, cv);
-	int cx0, cy0, cx1, cy1;
-	tile_coords<8>(cu, cv, cx0, cy0, cx1, cy1, c.cwx, c.cwy);
-	c.t00 = uint32_t(cy0 * 8 + cx0);
-	c.base = uint32_t(f0) + uint32_t(g.res[0]) * (uint32_t(f1) + uint32_t(g.res[1]) * uint32_t(f2));
+	c.t00 = tile_coords<8>(cu, cv, c.cwx, c.cwy);
+	c.base = uint32_t(cage.f[0]) + uint32_t(g.res[0]) * (uint32_t(cage.f[1]) + uint32_t(g.res[1]) * uint32_t(cage.f[2]));
 #pragma unroll
 	for(int i = 0; i < 8; ++i) {
 		uint32_t lin;
-		float w, fw;
-		if(!cage_probe(g, d.states, d.dep, position, normal, biased, emin, alpha, f0, f1, f2, i, lin, w, fw)) continue;
+		Vec3 pp, dtp;
+		float trw, w, fw;
+		if(!cage_corner(g, d.states, cage, position, i, lin, pp, dtp, trw)) continue;
+		cage_weight(d.dep, lin, pp, dtp, trw, normal, biased, w, fw);
 		c.mask |= 1u << i;
 		c.w[i] = w;
 		c.fw[i] = fw;
@@ -113,8 +107,6 @@ struct TexelEval {
 
 __device__ __forceinline__ TexelEval texel_eval(const DiffArgs& d, const TexelWeights& c) {
 	TexelEval e;
-	const uint32_t x0 = c.t00 & 7u, y0 = c.t00 >> 3, x1 = min(x0 + 1u, 7u), y1 = min(y0 + 1u, 7u);
-	const uint32_t t10 = y0 * 8u + x1, t01 = y1 * 8u + x0, t11 = y1 * 8u + x1;
 	const uint32_t rx = uint32_t(d.grid.res[0]), ry = uint32_t(d.grid.res[1]);
 	e.inv_w = c.tw > 1e-3f ? 1.0f / c.tw : 1.0f;
 	e.inv_fb = c.tfb > 1e-3f ? 1.0f / c.tfb : 1.0f;
@@ -126,8 +118,8 @@ __device__ __forceinline__ TexelEval texel_eval(const DiffArgs& d, const TexelWe
 		const bool on = (c.mask >> i) & 1u;
 		// slots that do not contribute read some tile and drop what they read
 		const uint32_t lin = on ? c.base + uint32_t(i & 1) + rx * (uint32_t((i >> 1) & 1) + ry * uint32_t(i >> 2)) : 0u;
-		const float4* ct = d.irr + size_t(lin) * 64;
-		const float4 c00 = ct[c.t00], c10 = ct[t10], c01 = ct[t01], c11 = ct[t11];
+		const float4* ct = d.irr + size_t(lin) * 64 + c.t00;
+		const float4 c00 = ct[0], c10 = ct[1], c01 = ct[8], c11 = ct[9];
 		const float a[3][4] = {{c00.x, c10.x, c01.x, c11.x}, {c00.y, c10.y, c01.y, c11.y}, {c00.z, c10.z, c01.z, c11.z}};
 #pragma unroll
 		for(int ch = 0; ch < 3; ++ch) {
@@ -190,10 +182,8 @@ __global__ void k_cells(DiffArgs d, uint32_t taps, uint32_t* __restrict__ key_of
 	}
 	if(taps == 64u) {
 		float cu, cv, wx, wy;
-		int x0, y0, x1, y1;
 		oct_uv(d.nrm[x * 3], d.nrm[x * 3 + 1], d.nrm[x * 3 + 2], cu, cv);
-		tile_coords<8>(cu, cv, x0, y0, x1, y1, wx, wy);
-		c = c * 64u + uint32_t(y0 * 8 + x0);
+		c = c * 64u + tile_coords<8>(cu, cv, wx, wy);
 	}
 	key_of[x] = c;
 	wave_count(key_count, c);
@@ -375,10 +365,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 #pragma unroll
 	for(int q = 0; q < 4; ++q) acc[q][0] = acc[q][1] = acc[q][2] = 0.0;
 	macc[0] = macc[1] = macc[2] = 0.0;
-	const auto tap_of = [](uint32_t t00, int q) {
-		const uint32_t x = min((t00 & 7u) + uint32_t(q & 1), 7u), y = min((t00 >> 3) + uint32_t(q >> 1), 7u);
-		return y * 8u + x;
-	};
+	const auto tap_of = [](uint32_t t00, int q) { return t00 + uint32_t(q & 1) + 8u * uint32_t(q >> 1); };
 	const auto flush_taps = [&] {
 #pragma unroll
 		for(int q = 0; q < 4; ++q)

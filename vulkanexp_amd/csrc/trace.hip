@@ -214,8 +214,7 @@ __device__ __forceinline__ SurfaceShade shade_surface(const SceneDev& sc, const 
 	const float b0 = 1.0f - b1 - b2;
 	const Vec3 position = v3(d.x * t + o[0], d.y * t + o[1], d.z * t + o[2]);
 	// shadow ray toward the light: any hit, mask 0xFF, tmin 0.1, tmax 10000.  It goes first: it needs
-	// only the hit point, so few values stay live across the traversal (the shading terms, live
-	// across it when it came last, spilled 48 bytes per lane at 6 waves per SIMD).
+	// only the hit point, so few values stay live across the traversal.
 	RayPrep sr;
 	ray_prepare(position.x, position.y, position.z, light.dir[0], light.dir[1], light.dir[2], sr);
 	uint32_t nn = 0, nt = 0;
@@ -254,10 +253,12 @@ __device__ __forceinline__ SurfaceShade shade_surface(const SceneDev& sc, const 
 	const float ndd = dot3(normal, d);
 	const Vec3 refl = d - normal * (2.0f * ndd);
 	const Vec3 to_cam = v3(-d.x, -d.y, -d.z);
-	const Vec3 reflection = sample_probes(grid, states, irr, dep, position, refl, to_cam);
+	const Vec3 towards[2] = {refl, normal};
+	Vec3 sampled[2];
+	sample_probes<2>(grid, states, irr, dep, position, towards, to_cam, sampled);
+	const Vec3 reflection = sampled[0], indirect = sampled[1];
 	color = color + spec * reflection;
 	r.em_spec = color;
-	const Vec3 indirect = sample_probes(grid, states, irr, dep, position, normal, to_cam);
 	color = color + indirect * diffuse;
 	float fade = 1.0f;
 	if(lit) {
@@ -541,10 +542,12 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, u
 // One thread per entry of the ordered shade list, over a grid sized for the list's capacity (its
 // length is known only on the device; workgroups past it end at once).  The hardware refills a CU
 // as soon as one of its workgroups ends, so the CUs stay busy to the end of the list, which a
-// resident grid striding over the list does not do.  At least 6 waves per SIMD (80 registers): the
-// shadow traversal is latency-bound.
+// resident grid striding over the list does not do.  Bound by vector instructions (91 % of the SIMDs'
+// issue cycles) and the loads' data return (85 %).  Four waves per SIMD: sampling along two normals at
+// once takes 121 registers; at 5 and 6 waves it spills (0.406 and 0.437 ms against 0.374; two separate
+// calls with the compiler's divisions took 0.403 at any of these).
 template <int STACK, bool COUNT>
-__global__ __launch_bounds__(kShadeBlock, 6) void k_shade(TraceFrameArgs a) {
+__global__ __launch_bounds__(kShadeBlock, 4) void k_shade(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
 	if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x);
@@ -627,7 +630,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 7))) v
 // k_shade): workgroup i takes the kShadeBlock entries of shade item i; entries past a list's length
 // return at once.
 template <int STACK>
-__global__ __launch_bounds__(kShadeBlock, 6) void k_batch_shade(BatchLaunch b) {
+__global__ __launch_bounds__(kShadeBlock, 4) void k_batch_shade(BatchLaunch b) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t vol = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].volume);
 	const uint32_t first = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].first);
@@ -925,7 +928,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_reflection_trace(ReflectionArgs
 // One thread per entry of the key-ordered queue of front-face reflection hits, over a grid sized
 // for the chunk (as k_shade).
 template <int STACK>
-__global__ __launch_bounds__(kShadeBlock, 5) void k_reflection_shade(ReflectionArgs a) {
+__global__ __launch_bounds__(kShadeBlock, 4) void k_reflection_shade(ReflectionArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t count = *a.list_count;
 	for(uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x; k < count; k += gridDim.x * kShadeBlock) {
