@@ -568,11 +568,12 @@ ddgi_status ddgi_create(const ddgi_grid_params* params, const ddgi_options* opti
 	if(e == hipSuccess) e = dalloc(&h->sel, sizeof(SelectState));
 	if(e == hipSuccess) e = dalloc(&h->rays, P * R * sizeof(float4));
 	if(e == hipSuccess) e = dalloc(&h->hits, P * R * sizeof(float4));
-	// shade list and keys: the primary pass's segments hold up to kShadeSegments * kPrimaryBlock
-	// entries beyond P * R (each segment is sized for whole workgroups)
-	if(e == hipSuccess) e = dalloc(&h->shade_list, (P * R + kShadeSegments * kPrimaryBlock) * sizeof(uint32_t));
+	// shade list and keys: each of the primary pass's segments is sized for whole workgroups, or for
+	// whole work items in a batch
+	const size_t list = P * R + size_t(kShadeSegments) * kMaxItemThreads;
+	if(e == hipSuccess) e = dalloc(&h->shade_list, list * sizeof(uint32_t));
 	if(e == hipSuccess) e = dalloc(&h->shade_count, kListCounterBytes);
-	if(e == hipSuccess) e = dalloc(&h->shade_keys, (P * R + kShadeSegments * kPrimaryBlock) * sizeof(uint32_t));
+	if(e == hipSuccess) e = dalloc(&h->shade_keys, list * sizeof(uint32_t));
 	if(e == hipSuccess) e = dalloc(&h->sort_keys, P * R * sizeof(uint32_t));
 	if(e == hipSuccess) e = dalloc(&h->sort_list, P * R * sizeof(uint32_t));
 	if(e == hipSuccess) e = dalloc(&h->sort_counts, size_t(kShadeSortCounts) * sizeof(uint32_t));

@@ -47,7 +47,9 @@ struct Batch {
 	BatchItem* d_shade_items = nullptr;
 	size_t shade_cap = 0;
 	BatchItem* d_blend_items = nullptr;
+	BatchItem* d_sort_items = nullptr;
 	size_t blend_cap = 0;
+	size_t sort_cap = 0;
 	BatchControl* d_ctl = nullptr;
 	// graph of the current configuration
 	hipGraphExec_t exec = nullptr;
@@ -120,21 +122,24 @@ ddgi_status build_items(Batch* b, uint32_t mode, BatchLaunch& L) {
 	});
 	const uint32_t per_item = b->cfg.trace_block * b->cfg.trace_item_blocks;
 	const uint32_t probes = mode == kBlendFP32 ? b->cfg.blend_probes : kMfmaProbes;
-	std::vector<BatchItem> ti, si, bi;
+	std::vector<BatchItem> ti, si, bi, oi;
 	for(uint32_t v : order) {
 		const Handle* h = b->vols[v];
 		const uint64_t threads = uint64_t(h->P) * h->params.rays_per_probe;  // also the shade list's capacity
 		for(uint64_t f = 0; f < threads; f += per_item) ti.push_back(BatchItem{v, uint32_t(f)});
 		for(uint64_t f = 0; f < threads; f += kShadeBlock) si.push_back(BatchItem{v, uint32_t(f)});
 		for(uint32_t s = 0; s < h->P; s += probes) bi.push_back(BatchItem{v, s});
+		for(uint64_t f = 0; f < threads; f += kFineChunk) oi.push_back(BatchItem{v, uint32_t(f / kFineChunk)});
 	}
 	ddgi_status st = ensure_items(&b->d_trace_items, &b->trace_cap, ti.size());
 	if(st != DDGI_OK || (st = ensure_items(&b->d_shade_items, &b->shade_cap, si.size())) != DDGI_OK ||
-	   (st = ensure_items(&b->d_blend_items, &b->blend_cap, bi.size())) != DDGI_OK)
+	   (st = ensure_items(&b->d_blend_items, &b->blend_cap, bi.size())) != DDGI_OK ||
+	   (st = ensure_items(&b->d_sort_items, &b->sort_cap, oi.size())) != DDGI_OK)
 		return st;
 	BHIP_TRY(hipMemcpy(b->d_trace_items, ti.data(), ti.size() * sizeof(BatchItem), hipMemcpyHostToDevice));
 	BHIP_TRY(hipMemcpy(b->d_shade_items, si.data(), si.size() * sizeof(BatchItem), hipMemcpyHostToDevice));
 	BHIP_TRY(hipMemcpy(b->d_blend_items, bi.data(), bi.size() * sizeof(BatchItem), hipMemcpyHostToDevice));
+	BHIP_TRY(hipMemcpy(b->d_sort_items, oi.data(), oi.size() * sizeof(BatchItem), hipMemcpyHostToDevice));
 	L.vols = b->d_vols;
 	L.trace_items = b->d_trace_items;
 	L.blend_items = b->d_blend_items;
@@ -147,6 +152,8 @@ ddgi_status build_items(Batch* b, uint32_t mode, BatchLaunch& L) {
 	L.blend_mode = mode;
 	L.shade_items = b->d_shade_items;
 	L.shade_item_count = uint32_t(si.size());
+	L.sort_items = b->d_sort_items;
+	L.sort_item_count = uint32_t(oi.size());
 	return DDGI_OK;
 }
 
@@ -166,10 +173,8 @@ ddgi_status ensure_graph(Batch* b, uint32_t mode) {
 	BHIP_TRY(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
 	hipError_t e = launch_batch_begin(L, b->cap);
 	if(e == hipSuccess) e = launch_batch_weights(L, b->cap);
-	uint64_t max_list = 0;
-	for(const Handle* h : b->vols) max_list = std::max<uint64_t>(max_list, uint64_t(h->P) * h->params.rays_per_probe);
 	if(e == hipSuccess) e = launch_batch_trace(L, b->cfg.trace_block, std::min(g_primary, L.trace_item_count), b->cap);
-	if(e == hipSuccess) e = launch_batch_sort(L, max_list, b->cap);
+	if(e == hipSuccess) e = launch_batch_sort(L, b->cap);
 	if(e == hipSuccess) e = launch_batch_shade(L, b->cap);
 	if(e == hipSuccess) e = launch_batch_blend(L, b->cap);
 	hipGraph_t graph = nullptr;
@@ -190,7 +195,8 @@ ddgi_status ensure_graph(Batch* b, uint32_t mode) {
 	return DDGI_OK;
 }
 
-void fill_volume(const Handle& h, const Rot& R, BatchVolume& v) {
+// `per_item`: traversal threads of a work item.
+void fill_volume(const Handle& h, const Rot& R, uint32_t per_item, BatchVolume& v) {
 	const GridConst g = make_grid_const(h);
 	const int nxt = h.cur ^ 1;
 	v = BatchVolume{};
@@ -216,9 +222,11 @@ void fill_volume(const Handle& h, const Rot& R, BatchVolume& v) {
 	shade_key_layout(g, &key_shift, &key_bits);
 	a.shade_keys = h.shade_keys;
 	a.key_shift = key_shift;
-	a.seg_cap = 0;  // one shade list per volume
+	// segment s of the shade list takes the front-face hits of work items i with i % 8 == s
+	const uint32_t items = uint32_t((uint64_t(h.P) * g.n + per_item - 1) / per_item);
+	a.seg_cap = (items + kShadeSegments - 1) / kShadeSegments * per_item;
 	v.sort = SortJob{h.shade_keys, h.shade_list, h.shade_count, h.sort_counts, h.sort_keys, h.sort_list,
-					 h.shade_count + kShadeTotalSlot, sort_fine_bits(3 * key_bits), 1u, 0u, 0u};
+					 h.shade_count + kShadeTotalSlot, sort_fine_bits(3 * key_bits), kShadeSegments, a.seg_cap, 0u};
 	BlendArgs& bl = v.blend;
 	bl.grid = g;
 	bl.indices = h.indices;
@@ -254,6 +262,7 @@ void destroy_batch(Batch* b) {
 	(void)hipFree(b->d_trace_items);
 	(void)hipFree(b->d_shade_items);
 	(void)hipFree(b->d_blend_items);
+	(void)hipFree(b->d_sort_items);
 	(void)hipFree(b->d_ctl);
 	if(b->h_ring) (void)hipHostFree(b->h_ring);
 	for(auto& e : b->ring_ev)
@@ -288,7 +297,7 @@ ddgi_status run_batch(Batch* b, const float* orientations, uint32_t flags, hipSt
 	for(uint32_t v = 0; v < nv; ++v) {
 		Rot R;
 		std::memcpy(R.r, orientations + size_t(v) * 9, sizeof(R.r));
-		fill_volume(*b->vols[v], R, ring[v]);
+		fill_volume(*b->vols[v], R, b->cfg.trace_block * b->cfg.trace_item_blocks, ring[v]);
 	}
 	BHIP_TRY(hipMemcpyAsync(b->d_vols, ring, sizeof(BatchVolume) * nv, hipMemcpyHostToDevice, s));
 	BHIP_TRY(hipEventRecord(b->ring_ev[b->ring_pos], s));

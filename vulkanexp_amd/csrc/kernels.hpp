@@ -101,8 +101,8 @@ struct SlotBoxArgs {
 // 0xFFFFFFFF = miss (t = -1).
 // List counters, each on its own 128-byte line (device-scope atomics on one line serialise): the
 // primary pass appends its front-face hits to kShadeSegments segments of the shade list, segment s
-// counted at [kCounterStride * s] (workgroup b appends to segment b % kShadeSegments, so each XCD
-// has its own counter); the miss list is counted at [kMissCountSlot]; the key sort stores the
+// counted at [kCounterStride * s] (workgroup b of an update appends to segment b % kShadeSegments, so each
+// XCD has its own counter; item i of a batched volume to segment i % kShadeSegments); the miss list is counted at [kMissCountSlot]; the key sort stores the
 // ordered list's length at [kShadeTotalSlot], which the shading reads.
 constexpr uint32_t kShadeSegments = 8;
 constexpr uint32_t kCounterStride = 32;
@@ -137,7 +137,7 @@ struct TraceFrameArgs {
 	// (cell coordinates shifted right by key_shift, so that they stay below 64 and keys below 2^18)
 	uint32_t* shade_keys;
 	uint32_t key_shift;
-	// > 0: the shade list is kShadeSegments segments of seg_cap entries (k_trace_primary); 0: one list
+	// the shade list is kShadeSegments segments of seg_cap entries
 	uint32_t seg_cap;
 };
 constexpr uint32_t kShadeSortCounts = 1024 * 128 + 1024;  // (list tile, coarse digit) counters + digit totals
@@ -237,10 +237,13 @@ struct SortJob {
 };
 // The sort kernels' argument: one job, or (many != nullptr) job y of workgroup (x, y) at
 // many + y * stride.
+struct BatchItem;
+constexpr uint32_t kFineChunk = 4096;  // list entries per workgroup of the sort's last pass
 struct SortJobs {
 	SortJob one;
 	const char* many;
 	uint32_t stride;
+	const BatchItem* chunks;  // (job, chunk of kFineChunk entries) per workgroup of a batch's last pass
 };
 uint32_t sort_fine_bits(uint32_t key_bits);
 
@@ -307,6 +310,7 @@ constexpr uint32_t kBlendFP16 = 2;
 
 // ---- batched update of many probe volumes (one graph launch per update) ----
 constexpr uint32_t kMaxBatchVolumes = 256;
+constexpr uint32_t kMaxItemThreads = 256 * 64;  // most traversal threads of a batch's work item
 constexpr uint32_t kMfmaProbes = 64;   // probes per MFMA blend workgroup (BF16 / FP16)
 
 // Everything the kernels of one volume read during a batched update.
@@ -328,7 +332,7 @@ struct BatchVolume {
 
 struct BatchItem {
 	uint32_t volume;
-	uint32_t first;  // first traversal thread (trace items) or first slot (blend items)
+	uint32_t first;  // first traversal thread (trace items), slot (blend items), or the chunk (sort items)
 };
 
 struct BatchControl {
@@ -351,14 +355,15 @@ struct BatchLaunch {
 	uint32_t blend_mode;
 	const BatchItem* shade_items;  // one workgroup of kShadeBlock shade-list entries each
 	uint32_t shade_item_count;
+	const BatchItem* sort_items;   // every kFineChunk entries that the volumes' shade lists can hold
+	uint32_t sort_item_count;
 };
 
 hipError_t launch_batch_begin(const BatchLaunch& b, hipStream_t s);
 hipError_t launch_batch_weights(const BatchLaunch& b, hipStream_t s);
 hipError_t launch_batch_trace(const BatchLaunch& b, uint32_t block, uint32_t grid, hipStream_t s);
-// Orders the shade list of every volume (BatchVolume::sort) in one set of launches; max_capacity
-// = the largest list capacity.
-hipError_t launch_batch_sort(const BatchLaunch& b, uint64_t max_capacity, hipStream_t s);
+// Orders the shade list of every volume (BatchVolume::sort) in one set of launches.
+hipError_t launch_batch_sort(const BatchLaunch& b, hipStream_t s);
 // Shades every volume's ordered shade list: one workgroup per shade item, one thread per entry.
 hipError_t launch_batch_shade(const BatchLaunch& b, hipStream_t s);
 hipError_t launch_batch_blend(const BatchLaunch& b, hipStream_t s);

@@ -133,13 +133,12 @@ __device__ __forceinline__ uint32_t cell_key(const GridConst& g, float px, float
 // Result of the ray at position ri (= slot * n + k, thread order): its hit record, and either its
 // final ray record (miss, back face) or a shade-list entry (front-face hit).
 __device__ __forceinline__ void finish_primary_ray(const TraceFrameArgs& a, uint32_t ri, const HitResult& h,
-												   uint32_t key) {
+												   uint32_t key, uint32_t seg) {
 	const float4 packed = pack_hit(h);
 	a.hits[ri] = packed;
 	const uint32_t code = __float_as_uint(packed.y);
 	const bool front = code != 0xFFFFFFFFu && !(code & 0x80000000u);
-	// front-face hits are queued for shading, in this workgroup's segment of the list
-	const uint32_t seg = a.seg_cap ? blockIdx.x % kShadeSegments : 0u;
+	// front-face hits are queued for shading, in segment `seg` of the list
 	const size_t base = size_t(seg) * a.seg_cap;
 	const uint32_t pos = wave_append(a.shade_count + kCounterStride * seg, front);
 	if(front) {
@@ -157,9 +156,9 @@ __device__ __forceinline__ void finish_primary_ray(const TraceFrameArgs& a, uint
 }
 
 // Traversal thread `gtid` = slot * n + j traces ray perm[j] of the probe in `slot`; `stack` is the
-// thread's column of an LDS stack with `stride` columns.
+// thread's column of an LDS stack with STRIDE columns, `seg` the shade-list segment its hit goes to.
 template <int STACK, int STRIDE, bool COUNT>
-__device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint32_t gtid, uint32_t* stack) {
+__device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint32_t gtid, uint32_t* stack, uint32_t seg) {
 	const uint32_t n = a.grid.n;
 	const uint32_t slot = gtid / n, j = gtid - slot * n;
 	if(slot >= *a.count) return;
@@ -174,7 +173,7 @@ __device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint3
 															  DDGI_MASK_STATIC | DDGI_MASK_DYNAMIC, stack, nn, nt);
 	const uint32_t key = a.shade_keys ? cell_key(a.grid, o[0] + h.t * d.x, o[1] + h.t * d.y, o[2] + h.t * d.z, a.key_shift)
 									  : 0u;
-	finish_primary_ray(a, slot * n + j, h, key);  // thread order: coalesced stores
+	finish_primary_ray(a, slot * n + j, h, key, seg);  // thread order: coalesced stores
 	if(COUNT) {
 		atomicAdd(&a.visit_counters[0], (unsigned long long)nn);
 		atomicAdd(&a.visit_counters[1], (unsigned long long)nt);
@@ -186,7 +185,7 @@ template <int STACK, bool COUNT>
 __global__ __launch_bounds__(kPrimaryBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_primary(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kPrimaryBlock];
 	trace_primary_ray<STACK, kPrimaryBlock, COUNT>(a, xcd_remap(blockIdx.x, gridDim.x) * kPrimaryBlock + threadIdx.x,
-												   stack + threadIdx.x);
+												   stack + threadIdx.x, blockIdx.x % kShadeSegments);
 }
 
 // ---- closest-hit shading + shadow ray (closesthit.glsl:143-289) ----
@@ -348,14 +347,14 @@ __device__ __forceinline__ void sort_tile(const SortJob& j, uint32_t b, size_t& 
 	hi = min(count, lo + per);
 }
 
-// The list workgroup (x, y) works on: the single job, or job y of a batch's array.
-__device__ __forceinline__ SortJob sort_job(const SortJobs& J) {
+// The single job, or job y of a batch's array.
+__device__ __forceinline__ SortJob sort_job(const SortJobs& J, uint32_t y) {
 	if(!J.many) return J.one;
-	return *reinterpret_cast<const SortJob*>(J.many + size_t(blockIdx.y) * J.stride);
+	return *reinterpret_cast<const SortJob*>(J.many + size_t(y) * J.stride);
 }
 
 __global__ __launch_bounds__(1024) void k_sort_count(SortJobs J) {
-	const SortJob j = sort_job(J);
+	const SortJob j = sort_job(J, blockIdx.y);
 	const uint32_t* __restrict__ keys = j.keys;
 	const uint32_t fine_bits = j.fine_bits;
 	uint32_t* __restrict__ counts = j.counts;
@@ -384,7 +383,7 @@ __global__ __launch_bounds__(1024) void k_sort_count(SortJobs J) {
 // Column prefix sums: workgroup g takes digits 64 g .. 64 g + 63 (one per lane); wave q of the
 // workgroup walks tiles 32 q .. 32 q + 31 of them (loads coalesced over the lanes, all in flight).
 __global__ __launch_bounds__(256) void k_sort_columns(SortJobs J) {
-	const SortJob j = sort_job(J);
+	const SortJob j = sort_job(J, blockIdx.y);
 	uint32_t* __restrict__ counts = j.counts;
 	uint32_t* __restrict__ totals = j.counts + kSortTiles * kSortDigits;
 	if(j.total && blockIdx.x == 0 && threadIdx.x == 0) {  // the ordered list's length, for the shading
@@ -413,7 +412,7 @@ __global__ __launch_bounds__(256) void k_sort_columns(SortJobs J) {
 }
 
 __global__ __launch_bounds__(1024) void k_sort_bucket(SortJobs J) {
-	const SortJob j = sort_job(J);
+	const SortJob j = sort_job(J, blockIdx.y);
 	const uint32_t* __restrict__ keys = j.keys;
 	const uint32_t* __restrict__ list = j.list;
 	const uint32_t fine_bits = j.fine_bits;
@@ -453,9 +452,11 @@ __global__ __launch_bounds__(1024) void k_sort_bucket(SortJobs J) {
 // however the keys are spread): a chunk is ordered in LDS by its local key = (coarse digit - the
 // chunk's first coarse digit, fine digit), local keys from 1023 up sharing the last counter.  A
 // chunk inside one bucket is ordered by the fine digit; one spanning buckets keeps their order.
-constexpr uint32_t kFineChunk = 4096;
 __global__ __launch_bounds__(1024) void k_sort_fine(SortJobs J) {
-	const SortJob j = sort_job(J);
+	// workgroup -> (job, chunk): the single job's chunks, or a batch's chunk items (a grid of jobs x the
+	// longest list's chunks is mostly workgroups with nothing to do: 117 us for 20 volumes)
+	const uint32_t chunk = J.many ? __builtin_amdgcn_readfirstlane(J.chunks[blockIdx.x].first) : blockIdx.x;
+	const SortJob j = sort_job(J, J.many ? __builtin_amdgcn_readfirstlane(J.chunks[blockIdx.x].volume) : 0u);
 	const uint32_t* __restrict__ bucket_keys = j.bucket_keys;
 	const uint32_t* __restrict__ bucket_list = j.bucket_list;
 	const uint32_t fine_bits = j.fine_bits;
@@ -464,8 +465,8 @@ __global__ __launch_bounds__(1024) void k_sort_fine(SortJobs J) {
 	__shared__ uint32_t s_cnt[1024];
 	__shared__ uint32_t s_wave[16];
 	const uint32_t t = threadIdx.x;
-	const uint32_t count = job_length(j);
-	const uint32_t c0 = blockIdx.x * kFineChunk;
+	const uint32_t count = j.total ? __builtin_amdgcn_readfirstlane(*j.total) : job_length(j);
+	const uint32_t c0 = chunk * kFineChunk;
 	if(c0 >= count) return;  // uniform over the workgroup
 	const uint32_t c1 = min(count, c0 + kFineChunk);
 	const uint32_t first = bucket_keys[c0] >> fine_bits, mask = (1u << fine_bits) - 1u;
@@ -593,7 +594,8 @@ __global__ __launch_bounds__(kMaxRays) void k_batch_begin(BatchLaunch b) {
 		y = d.y;
 	}
 	frame_order_block(y, n, s_key, v.perm);
-	if(threadIdx.x == 0) v.trace.shade_count[0] = v.trace.shade_count[kMissCountSlot] = 0u;
+	if(threadIdx.x < kShadeSegments) v.trace.shade_count[kCounterStride * threadIdx.x] = 0u;
+	if(threadIdx.x == 0) v.trace.shade_count[kMissCountSlot] = 0u;
 	if(blockIdx.x == 0) {
 		if(threadIdx.x < 4) b.ctl->next[threadIdx.x] = 0u;
 		for(uint32_t k = threadIdx.x; k < kMaxBatchVolumes; k += 512) b.ctl->done[k] = 0ull;
@@ -604,7 +606,7 @@ __global__ __launch_bounds__(kMaxRays) void k_batch_begin(BatchLaunch b) {
 // Persistent primary traversal over the work items of all volumes: each workgroup takes the next
 // item (a run of consecutive traversal threads of one volume) from a queue until the queue is
 // empty.  Every workgroup leaves once the head passes the item count, so the grid always drains.
-// seven waves per SIMD (72 VGPRs): 2.79 ms for 21.9 M rays of 20 volumes, against 2.88 at 5, 2.82 at 6, 2.90 at 8
+// seven waves per SIMD (72 VGPRs): fastest of 5 to 8
 template <int STACK, int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_batch_trace(BatchLaunch b) {
 	__shared__ uint32_t stack[STACK * BLOCK];
@@ -620,9 +622,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 7))) v
 		const uint32_t vol = __builtin_amdgcn_readfirstlane(b.trace_items[it].volume);
 		const uint32_t first = __builtin_amdgcn_readfirstlane(b.trace_items[it].first);
 		const BatchVolume& v = b.vols[vol];
+		// a volume's items share out its list's segments, so that its hits are counted on eight lines (on
+		// one line per volume the appends' atomics serialise: 2.79 ms against 1.47 for 21.9 M rays)
+		const uint32_t seg = (first / b.trace_item_threads) % kShadeSegments;
 		const uint32_t end = min(first + b.trace_item_threads, v.threads);
 		for(uint32_t g = first + threadIdx.x; g < end; g += BLOCK)
-			trace_primary_ray<STACK, BLOCK, false>(v.trace, g, stack + threadIdx.x);
+			trace_primary_ray<STACK, BLOCK, false>(v.trace, g, stack + threadIdx.x, seg);
 	}
 }
 
@@ -1356,13 +1361,12 @@ hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint
 	return hipGetLastError();
 }
 
-static hipError_t launch_sort_jobs(const SortJobs& J, uint32_t jobs, uint64_t capacity, hipStream_t s) {
-	if(capacity == 0 || jobs == 0) return hipSuccess;
-	const uint32_t chunks = uint32_t((capacity + kFineChunk - 1) / kFineChunk);
+static hipError_t launch_sort_jobs(const SortJobs& J, uint32_t jobs, uint32_t chunks, hipStream_t s) {
+	if(chunks == 0 || jobs == 0) return hipSuccess;
 	hipLaunchKernelGGL(k_sort_count, dim3(kSortTiles, jobs), dim3(1024), 0, s, J);
 	hipLaunchKernelGGL(k_sort_columns, dim3(kSortDigits / 64u, jobs), dim3(256), 0, s, J);
 	hipLaunchKernelGGL(k_sort_bucket, dim3(kSortTiles, jobs), dim3(1024), 0, s, J);
-	hipLaunchKernelGGL(k_sort_fine, dim3(chunks, jobs), dim3(1024), 0, s, J);
+	hipLaunchKernelGGL(k_sort_fine, dim3(chunks), dim3(1024), 0, s, J);
 	return hipGetLastError();
 }
 
@@ -1375,17 +1379,17 @@ hipError_t launch_key_sort(SortJob job, uint64_t capacity, uint32_t key_bits, hi
 	job.fine_bits = sort_fine_bits(key_bits);
 	SortJobs J{};
 	J.one = job;
-	return launch_sort_jobs(J, 1, capacity, s);
+	return launch_sort_jobs(J, 1, uint32_t((capacity + kFineChunk - 1) / kFineChunk), s);
 }
 
 static_assert(std::is_standard_layout<BatchVolume>::value, "the batched sort finds each volume's job by offsetof");
 
-hipError_t launch_batch_sort(const BatchLaunch& b, uint64_t max_capacity, hipStream_t s) {
-	if(max_capacity > 0xFFFFFFFFull) return hipErrorInvalidValue;
+hipError_t launch_batch_sort(const BatchLaunch& b, hipStream_t s) {
 	SortJobs J{};
 	J.many = reinterpret_cast<const char*>(b.vols) + offsetof(BatchVolume, sort);
 	J.stride = uint32_t(sizeof(BatchVolume));
-	return launch_sort_jobs(J, b.volume_count, max_capacity, s);
+	J.chunks = b.sort_items;
+	return launch_sort_jobs(J, b.volume_count, b.sort_item_count, s);
 }
 
 void shade_key_layout(const GridConst& g, uint32_t* shift, uint32_t* bits_per_axis) {
