@@ -386,8 +386,7 @@ ddgi_status enqueue_blend_and_publish(Handle* h, const Rot* R, const float4* ray
 	b.irr_out = h->irr[nxt];
 	b.dep_out = h->dep[nxt];
 	b.max_slots = max_slots;
-	// the FP32 blend in 64-probe workgroups once they fill the device, else in 16-probe blocks
-	HIP_TRY(h, launch_blend(b, mode, s, h->cus > 0 && max_slots >= 64u * h->cus));
+	HIP_TRY(h, launch_blend(b, mode, h->cus, s));
 	h->cur = nxt;  // publish (reference: vkCmdCopyImage work -> exposed, src/IrradianceProbes.cpp:530-576)
 	return DDGI_OK;
 }
@@ -1215,7 +1214,7 @@ ddgi_status ddgi_diff_forward(void* handle, const float* albedo, const float* su
 	b.dep_out = nullptr;
 	b.max_slots = d.slots;
 	b.flags = kBlendIrradianceOnly;
-	HIP_TRY(h, launch_blend(b, kBlendFP32, s));
+	HIP_TRY(h, launch_blend(b, kBlendFP32, h->cus, s));
 	HIP_TRY(h, diff_gather_forward(d, s));
 	h->last_stream = s;
 	return DDGI_OK;

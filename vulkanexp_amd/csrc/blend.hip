@@ -434,8 +434,8 @@ struct MfmaTypes<kBlendFP32> {
 };
 
 // ---------------------------------------------------------------------------------------------
-// MFMA blend, transposed and pipelined (BF16 / FP16 modes, and FP32 on grids whose 64-probe
-// workgroups fill the device: there v_mfma_f32_16x16x4_f32 runs 8 per accumulator and K step on
+// MFMA blend, transposed and pipelined, for launches whose 64-probe workgroups fill the device
+// (launch_blend holds the rule; FP32: v_mfma_f32_16x16x4_f32 runs 8 per accumulator and K step on
 // the unconverted ray data, pairing rays as blend_fp32_tile does).  Per channel the blend of a group of 16
 // probes is C^T [16 probes x texels] = X^T [16 probes x n rays] W^T [n x texels]: the ray data is
 // the A operand, read by each lane straight from HBM (row = one of the group's probes, 8 rays per
@@ -788,6 +788,214 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 	blend_mfma_wide<MODE, STEPS>(a, blockIdx.x * kWideProbes, lds);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Blend of a 16-probe tile by eight waves, for launches whose 64-probe workgroups would leave CUs idle
+// (launch_blend holds the rule).  Such a launch is bound by the latency of one workgroup's chain of K
+// steps, so a step does as little as it can: the same products per output element in the same order as
+// the wide blend (bit-identical sums), but split over the texels.  Wave w takes texel tiles 2 w and
+// 2 w + 1 (three irradiance, thirteen depth), one thread per (probe, ray) of a 32-ray K step loads and
+// converts that ray, and the A fragments pass through LDS (double-buffered, one barrier per step), while
+// the weights, which only this wave needs, come from L2 straight into registers.  256 probes of 512 rays,
+// FP16: 48 us on four wide workgroups, 16 here; 1024 probes of 256 rays, FP32: 29 us in 4-wave blocks, 21 here;
+// 256 probes of 128 rays, FP32: 17 and 12.6.
+constexpr int kTileProbes = 16;
+constexpr int kTileThreads = 512;
+constexpr int kTileStride = kKStep + 4;  // FP32: floats per staged (channel, probe) row
+// staged K step: 16-bit, [channel][part][lane] x 16 bytes; FP32, [channel][probe][kTileStride] floats
+constexpr int kTileStageBytes = 5 * 16 * kTileStride * 4;
+static_assert(kTileStageBytes >= 5 * 2 * 64 * 16, "one stage size for all modes");
+constexpr int kTileSumBytes = kTileProbes * (kIrrStride + kDepStride) * 4;
+constexpr int kTileLdsBytes = 2 * kTileStageBytes > kTileSumBytes ? 2 * kTileStageBytes : kTileSumBytes;
+
+template <uint32_t MODE>
+__device__ __forceinline__ void blend_wave_tile(const BlendArgs& a, uint32_t slot0, uint32_t n_pad, unsigned char* smem,
+												 uint32_t* s_small) {
+	typedef MfmaTypes<MODE> M;
+	typedef typename M::T T;
+	typedef typename M::V V;
+	constexpr int P = M::kParts;
+	constexpr bool kF32 = MODE == kBlendFP32;
+	uint32_t* s_oor = s_small;
+	uint32_t* s_maxc = s_small + kTileProbes;
+	uint32_t* s_idx = s_small + 2 * kTileProbes;
+	const uint32_t count = __builtin_amdgcn_readfirstlane(*a.count);  // uniform: see blend_fp32_tile
+	if(slot0 >= count) return;
+	const uint32_t np = min(uint32_t(kTileProbes), count - slot0);
+	const uint32_t n = __builtin_amdgcn_readfirstlane(a.grid.n);
+	const uint32_t steps = __builtin_amdgcn_readfirstlane(n_pad) / kKStep;
+	const float cell_len = a.grid.cell_len;
+	const bool irr_only = (a.flags & kBlendIrradianceOnly) != 0u;
+	const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+	const int lrow = lane & 15, lgrp = lane >> 4;
+	if(t < kTileProbes) s_idx[t] = uint32_t(t) < np ? a.indices[slot0 + t] : 0u;
+	// this thread's ray of every K step: probe t / 32, ray t % 32 of the step
+	const uint32_t my_p = uint32_t(t) >> 5, my_k = uint32_t(t) & 31u;
+	const float4* my_rays = a.rays + size_t(slot0 + (my_p < np ? my_p : 0u)) * n;
+	uint32_t my_oor = 0;
+	auto load_ray = [&](uint32_t s) {
+		const uint32_t k = s * kKStep + my_k;
+		return my_p < np && k < n ? my_rays[k] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	};
+	auto stage = [&](const float4& r, unsigned char* buf) {
+		if(r.w < 0.0f || r.w > cell_len) ++my_oor;  // rays that do not exist are 0: in range
+		float dc = fminf(cell_len, r.w);
+		if(dc < 0.0f) dc = cell_len;
+		float d2 = dc * dc;
+		// FP16: rounded to FP32 first, as in the wide blend (no fused mixed multiply); BF16 keeps the fused residual
+		if constexpr(P == 1) __asm__ volatile("" : "+v"(d2));
+		const float v[6] = {r.x, r.y, r.z, dc, d2, 0.0f};
+		if constexpr(kF32) {
+#pragma unroll
+			for(int c = 0; c < 5; ++c) reinterpret_cast<float*>(buf)[(c * 16 + my_p) * kTileStride + my_k] = v[c];
+		} else {
+			// element of ray 4 j + g: lane 16 g + probe's j-th value
+			unsigned char* dst = buf + ((my_k & 3u) * 16 + my_p) * 16 + (my_k >> 2) * 2;
+#pragma unroll
+			for(int c = 0; c < 6; c += 2) {
+				// two channels at a time, rounded as the wide blend rounds them
+				uint32_t part[2];
+				if constexpr(P == 2) {
+					split_bf16x2(v[c], v[c + 1], part[0], part[1]);
+				} else {
+					typedef float f32x2 __attribute__((ext_vector_type(2)));
+					typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+					part[0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[c], v[c + 1]}, f16x2));
+				}
+#pragma unroll
+				for(int p = 0; p < P; ++p) {
+					*reinterpret_cast<uint16_t*>(dst + (c * P + p) * 1024) = uint16_t(part[p]);
+					if(c < 4) *reinterpret_cast<uint16_t*>(dst + ((c + 1) * P + p) * 1024) = uint16_t(part[p] >> 16);
+				}
+			}
+		}
+	};
+	const T* __restrict__ wsrc[2] = {static_cast<const T*>(kF32 ? static_cast<const void*>(a.wt) : a.w_hi16),
+									  static_cast<const T*>(a.w_lo16)};
+	typedef float float4_v __attribute__((ext_vector_type(4)));
+	floatx4_t acc[2][3];
+#pragma unroll
+	for(int q = 0; q < 2; ++q)
+#pragma unroll
+		for(int c = 0; c < 3; ++c) acc[q][c] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+	const int tile0 = 2 * wave;
+	// weights of K step s: per tile, 16 bytes per part (16-bit) or per 16-ray half (FP32)
+	auto load_weights = [&](uint32_t s, float4_v (&w)[2][P]) {
+#pragma unroll
+		for(int q = 0; q < 2; ++q)
+#pragma unroll
+			for(int p = 0; p < P; ++p) {
+				const T* src = kF32 ? wsrc[0] + size_t(16 * (tile0 + q) + lrow) * n_pad + s * kKStep + p * 16 + lgrp * 4
+									: wsrc[p] + size_t(16 * (tile0 + q) + lrow) * n_pad + s * kKStep + lgrp * 8;
+				w[q][p] = *reinterpret_cast<const float4_v*>(src);
+			}
+	};
+	auto products = [&](const unsigned char* buf, const float4_v (&w)[2][P]) {
+#pragma unroll
+		for(int q = 0; q < 2; ++q) {
+			const bool irr = tile0 + q < 3;  // wave-uniform
+			if(!irr && irr_only) continue;
+			const int c0 = irr ? 0 : 3;
+			if constexpr(kF32) {
+				float4_v x[3][2];
+#pragma unroll
+				for(int c = 0; c < 3; ++c) {
+					if(c == 2 && !irr) continue;
+					const float* row = reinterpret_cast<const float*>(buf) + ((c0 + c) * 16 + lrow) * kTileStride + 4 * lgrp;
+					x[c][0] = *reinterpret_cast<const float4_v*>(row);
+					x[c][1] = *reinterpret_cast<const float4_v*>(row + 16);
+				}
+#pragma unroll
+				for(int j = 0; j < 8; ++j)
+#pragma unroll
+					for(int c = 0; c < 3; ++c) {
+						if(c == 2 && !irr) continue;
+						acc[q][c] = M::mma(x[c][j >> 2][j & 3], w[q][j >> 2][j & 3], acc[q][c]);
+					}
+			} else {
+				V A[3][P];
+#pragma unroll
+				for(int c = 0; c < 3; ++c) {
+					if(c == 2 && !irr) continue;
+#pragma unroll
+					for(int p = 0; p < P; ++p)
+						A[c][p] = *reinterpret_cast<const V*>(buf + ((c0 + c) * P + p) * 1024 + lane * 16);
+				}
+				V B[P];
+#pragma unroll
+				for(int p = 0; p < P; ++p) B[p] = __builtin_bit_cast(V, w[q][p]);
+				// hi x hi, lo x hi, hi x lo, as in the wide blend
+#pragma unroll
+				for(int c = 0; c < 3; ++c)
+					if(c < 2 || irr) acc[q][c] = M::mma(A[c][0], B[0], acc[q][c]);
+				if constexpr(P == 2) {
+#pragma unroll
+					for(int c = 0; c < 3; ++c)
+						if(c < 2 || irr) acc[q][c] = M::mma(A[c][1], B[0], acc[q][c]);
+#pragma unroll
+					for(int c = 0; c < 3; ++c)
+						if(c < 2 || irr) acc[q][c] = M::mma(A[c][0], B[1], acc[q][c]);
+				}
+			}
+		}
+	};
+	float4 r = load_ray(0);
+	float4_v w[2][P], wn[2][P];
+	load_weights(0, w);
+	for(uint32_t s = 0; s < steps; ++s) {
+		unsigned char* buf = smem + (s & 1u) * kTileStageBytes;
+		stage(r, buf);
+		if(s + 1 < steps) {
+			r = load_ray(s + 1);
+			load_weights(s + 1, wn);
+		}
+		// LDS only: the loads of the next step stay in flight.  A wave that passes this barrier has finished
+		// reading the other buffer (its products of step s - 1 precede it), so the next step may fill it.
+		lds_barrier();
+		products(buf, w);
+#pragma unroll
+		for(int q = 0; q < 2; ++q)
+#pragma unroll
+			for(int p = 0; p < P; ++p) w[q][p] = wn[q][p];
+	}
+	for(int off = 16; off > 0; off >>= 1) my_oor += __shfl_xor(my_oor, off);  // the probe's 32 threads
+	if(my_k == 0) s_oor[my_p] = my_oor;
+	// one pass of the epilogue: 16 probes over eight waves; its exposed-atlas loads need the indices only
+	const EpiLane el = epilogue_lane(a);
+	EpiPrev<2> pre;
+	epilogue_load(a, el, s_idx, np, uint32_t(wave), irr_only, pre);
+	__syncthreads();  // every wave is done with the staged rays: the sums take their place
+	float* s_irr = reinterpret_cast<float*>(smem);
+	float* s_dep = s_irr + kTileProbes * kIrrStride;
+#pragma unroll
+	for(int q = 0; q < 2; ++q) {
+		const int tile = tile0 + q, tex = 16 * (tile < 3 ? tile : tile - 3) + lrow;
+#pragma unroll
+		for(int k = 0; k < 4; ++k) {
+			const int slot = 4 * lgrp + k;
+			if(tile < 3) {
+				if(tex < int(kIrrTexels)) {
+#pragma unroll
+					for(int c = 0; c < 3; ++c) s_irr[slot * kIrrStride + tex * 4 + c] = acc[q][c][k];
+				}
+			} else if(tex < int(kDepTexels)) {
+				s_dep[slot * kDepStride + tex * 2 + 0] = acc[q][0][k];
+				s_dep[slot * kDepStride + tex * 2 + 1] = acc[q][1][k];
+			}
+		}
+	}
+	__syncthreads();
+	epilogue_store(a, el, s_idx, np, uint32_t(wave), s_irr, s_dep, s_maxc, irr_only, pre);
+	__syncthreads();
+	if(uint32_t(t) < np && !irr_only) update_state(a.states, s_idx[t], __uint_as_float(s_maxc[t]), s_oor[t], n);
+}
+
+template <uint32_t MODE>
+__global__ __launch_bounds__(kTileThreads) void k_blend_tile(BlendArgs a, uint32_t n_pad) {
+	__shared__ __attribute__((aligned(16))) unsigned char smem[kTileLdsBytes];
+	__shared__ uint32_t s_small[3 * kTileProbes];
+	blend_wave_tile<MODE>(a, blockIdx.x * kTileProbes, n_pad, smem, s_small);
+}
+
 // ---- batched update ----
 // Weight rows of every volume: grid (256 rows, volumes).
 __global__ __launch_bounds__(256) void k_batch_weights(BatchLaunch b) {
@@ -875,10 +1083,31 @@ hipError_t launch_blend_weights(const GridConst& g, const float4* dirs, const ui
 	return hipGetLastError();
 }
 
-hipError_t launch_blend(const BlendArgs& a, uint32_t mode, hipStream_t s, bool fp32_wide) {
+// One round of workgroups holds 32 probes per CU of the 16-probe tiles (two resident) and 64 of the wide
+// blend, and costs the tiles about 0.7 of the wide blend's (0.45 in FP16).  So the tiles are taken where
+// they need one round against one or three against two; the wide blend with its shared weights elsewhere.
+// ddgi_blend_rays with 256 rays, tiles / wide, us on 256 CUs:
+//   probes     256 (512 rays)  4096        8192        9216        13440       20480        25344
+//   BF16       33 / 67         28 / 46     40 / 47     49 / 47     59 / 50     72 / 83      97 / 87
+//   FP16       27 / 59         25 / 42     31 / 42     38 / 42     43 / 45     58 / 72      77 / 75
+//   FP32       45 / 107        34 / 67     48 / 68     70 / 68     77 / 71     106 / 121    129 / 126
+// FP32 has a third form, the 4-wave blocks (three per CU: 48 probes a round): 42, 53, 65, 82 at 4096,
+// 8192, 9216, 13440, the best between one round of tiles and 48 probes per CU.  Irradiance-only blends
+// (which the wide kernel does not do) take the tiles for one round (1024 probes, 64 rays: 10.6 us, blocks
+// 18.8) and the blocks beyond.
+hipError_t launch_blend(const BlendArgs& a, uint32_t mode, uint32_t cus, hipStream_t s) {
 	if(a.max_slots == 0) return hipSuccess;
 	const uint32_t n_pad = (a.grid.n + kMfmaChunk - 1) & ~uint32_t(kMfmaChunk - 1);
-	if(mode == kBlendFP32 && (!fp32_wide || (a.flags & kBlendIrradianceOnly))) {
+	const bool irr_only = (a.flags & kBlendIrradianceOnly) != 0u;
+	const uint32_t round = 32u * (cus ? cus : 256u);  // probes of one round of tiles
+	if(a.max_slots <= round || (!irr_only && a.max_slots > 2u * round && a.max_slots <= 3u * round)) {
+		const dim3 grid((a.max_slots + kTileProbes - 1) / kTileProbes), block(kTileThreads);
+		if(mode == kBlendFP32) hipLaunchKernelGGL(k_blend_tile<kBlendFP32>, grid, block, 0, s, a, n_pad);
+		else if(mode == kBlendBF16) hipLaunchKernelGGL(k_blend_tile<kBlendBF16>, grid, block, 0, s, a, n_pad);
+		else hipLaunchKernelGGL(k_blend_tile<kBlendFP16>, grid, block, 0, s, a, n_pad);
+		return hipGetLastError();
+	}
+	if(mode == kBlendFP32 && (irr_only || a.max_slots <= round + round / 2u)) {
 		hipLaunchKernelGGL(k_blend_fp32, dim3((a.max_slots + kProbesPerBlock - 1) / kProbesPerBlock), dim3(256), 0, s, a, n_pad);
 		return hipGetLastError();
 	}
