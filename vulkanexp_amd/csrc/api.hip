@@ -969,7 +969,7 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 		HIP_TRY(h, hipMemsetAsync(h->visit, 0, 8 * sizeof(unsigned long long), s));
 		a.visit_counters = h->visit;
 	}
-	a.shade_keys = h->shade_keys;
+	a.shade_keys = uint64_t(max_slots) * g.n >= kShadeSortRays ? h->shade_keys : nullptr;
 	a.key_shift = key_shift;
 	{  // segment s of the shade list takes the front-face hits of workgroups b with b % 8 == s
 		const uint32_t blocks = uint32_t((uint64_t(max_slots) * g.n + kPrimaryBlock - 1) / kPrimaryBlock);
@@ -977,10 +977,10 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	}
 	HIP_TRY(h, launch_trace_primary(a, s));
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
-	// shade the front-face hits ordered by the grid cell they lie in
-	HIP_TRY(h, launch_key_sort(SortJob{h->shade_keys, h->shade_list, h->shade_count, h->sort_counts, h->sort_keys,
-									   h->sort_list, h->shade_count + kShadeTotalSlot, 0u, kShadeSegments, a.seg_cap, 0u},
-							   uint64_t(max_slots) * g.n, 3 * key_bits, s));
+	if(a.shade_keys)  // shade the front-face hits ordered by the grid cell they lie in
+		HIP_TRY(h, launch_key_sort(SortJob{h->shade_keys, h->shade_list, h->shade_count, h->sort_counts, h->sort_keys,
+										   h->sort_list, h->shade_count + kShadeTotalSlot, 0u, kShadeSegments, a.seg_cap, 0u},
+								   uint64_t(max_slots) * g.n, 3 * key_bits, s));
 	HIP_TRY(h, launch_shade(a, s));
 	if(h->light.sky_model == DDGI_SKY_ATMOSPHERE) HIP_TRY(h, launch_sky(a, s));
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));

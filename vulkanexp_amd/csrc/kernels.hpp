@@ -109,6 +109,12 @@ constexpr uint32_t kCounterStride = 32;
 constexpr uint32_t kMissCountSlot = kCounterStride * kShadeSegments;
 constexpr uint32_t kShadeTotalSlot = kMissCountSlot + kCounterStride;
 constexpr uint32_t kListCounterBytes = (kShadeTotalSlot + kCounterStride) * 4;
+// An update orders its shade list from this many rays (slots x rays per probe) up.  The ordering's four
+// launches cost 25 to 60 us; it shortens the shading by less than that while the hits' probe tiles and BVH
+// nodes fit the caches anyway.  Whole update without / with the ordering, us, instances of the scene 24, 80, 256:
+//   rays   32768                        524288                       1048576                      2097152
+//          122 / 145 144 / 170 168 / 192  186 / 213 228 / 245 266 / 285  245 / 250 324 / 300 385 / 372  391 / 358 550 / 477 689 / 591
+constexpr uint64_t kShadeSortRays = 640u * 1024u;
 
 struct TraceFrameArgs {
 	SceneDev scene;
@@ -134,7 +140,8 @@ struct TraceFrameArgs {
 	// (c0, material bits), (A, lit bits), (B, 0), (C, 0); material 0xFFFFFFFF for misses/back faces
 	float4* factors;
 	// optional (shade-list ordering): the primary pass stores the cell key of each shade-list entry
-	// (cell coordinates shifted right by key_shift, so that they stay below 64 and keys below 2^18)
+	// (cell coordinates shifted right by key_shift, so that they stay below 64 and keys below 2^18);
+	// null: the segments are shaded as they were appended
 	uint32_t* shade_keys;
 	uint32_t key_shift;
 	// the shade list is kShadeSegments segments of seg_cap entries

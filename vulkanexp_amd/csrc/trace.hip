@@ -286,7 +286,7 @@ __device__ __forceinline__ SurfaceShade shade_surface(const SceneDev& sc, const 
 // wherever one probe's rays ended.  Sorting the list by the Morton code of the probe-grid half-cell
 // holding the hit point (cell_key) gives consecutive waves hits that share cage probes (the same
 // atlas tiles) and cast shadow rays from nearby origins along the same direction (the same BVH
-// nodes), which the caches then serve.  Each entry's shading depends on its own record only, so
+// nodes), which the caches then serve.  Updates of fewer than kShadeSortRays rays do without.  Each entry's shading depends on its own record only, so
 // the order changes no output, and entries with equal keys may come in any order.
 //
 // Keys of up to 18 bits = a coarse digit (the high 10 bits) and a fine digit (the rest):
@@ -502,8 +502,7 @@ __global__ __launch_bounds__(1024) void k_sort_fine(SortJobs J) {
 // every lane of a wave shades and casts a shadow ray.  Each ray's result depends only on its own
 // record: the order of the list does not change any output.
 template <int STACK, bool COUNT>
-__device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, uint32_t* stack) {
-	if(k >= a.shade_count[kShadeTotalSlot]) return;
+__device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, size_t k, uint32_t* stack) {
 	const uint32_t n = a.grid.n;
 	const uint32_t ri = a.shade_list[k];  // hits and rays are stored in thread (ray_order) order
 	const uint32_t slot = ri / n, j = ri - slot * n;
@@ -540,8 +539,8 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, u
 	}
 }
 
-// One thread per entry of the ordered shade list, over a grid sized for the list's capacity (its
-// length is known only on the device; workgroups past it end at once).  The hardware refills a CU
+// One thread per entry of the shade list (ordered, or in its segments as appended), over a grid sized for the
+// list's capacity (its length is known only on the device; workgroups past it end at once).  The hardware refills a CU
 // as soon as one of its workgroups ends, so the CUs stay busy to the end of the list, which a
 // resident grid striding over the list does not do.  Bound by vector instructions (91 % of the SIMDs'
 // issue cycles) and the loads' data return (85 %).  Four waves per SIMD: sampling along two normals at
@@ -550,8 +549,14 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, uint32_t k, u
 template <int STACK, bool COUNT>
 __global__ __launch_bounds__(kShadeBlock, 4) void k_shade(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
-	const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
-	if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x);
+	if(a.shade_keys) {
+		const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
+		if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x);
+	} else {  // the list as it was appended: workgroup b takes entries of segment b % kShadeSegments
+		const uint32_t seg = blockIdx.x % kShadeSegments;
+		const uint32_t k = blockIdx.x / kShadeSegments * kShadeBlock + threadIdx.x;
+		if(k < a.shade_count[kCounterStride * seg]) shade_ray<STACK, COUNT>(a, size_t(seg) * a.seg_cap + k, stack + threadIdx.x);
+	}
 }
 
 // ---- misses under the atmospheric sky (miss.rmiss:17-23 with sky.glsl:60-127) ----
@@ -639,7 +644,8 @@ __global__ __launch_bounds__(kShadeBlock, 4) void k_batch_shade(BatchLaunch b) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
 	const uint32_t vol = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].volume);
 	const uint32_t first = __builtin_amdgcn_readfirstlane(b.shade_items[blockIdx.x].first);
-	shade_ray<STACK, false>(b.vols[vol].trace, first + threadIdx.x, stack + threadIdx.x);
+	const TraceFrameArgs& a = b.vols[vol].trace;
+	if(first + threadIdx.x < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, false>(a, first + threadIdx.x, stack + threadIdx.x);
 }
 
 // ---- arbitrary ray queries (public ddgi_hit records) ----
@@ -1425,7 +1431,8 @@ hipError_t launch_sky(const TraceFrameArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_shade(const TraceFrameArgs& a, hipStream_t s) {
-	const uint64_t threads = uint64_t(a.max_slots) * a.grid.n;  // upper bound of the shade list
+	// upper bound of the shade list: its entries in order, or every segment's capacity
+	const uint64_t threads = a.shade_keys ? uint64_t(a.max_slots) * a.grid.n : uint64_t(kShadeSegments) * a.seg_cap;
 	if(threads == 0) return hipSuccess;
 	const bool cnt = a.visit_counters != nullptr;
 	const void* f = cnt ? reinterpret_cast<const void*>(&k_shade<kLdsStack, true>)
