@@ -356,15 +356,33 @@ void destroy_handle(Handle* h) {
 	delete h;
 }
 
-// `order`: the ray order of the `rays` records (the traversal's thread order for ddgi_update,
-// nullptr = natural order for caller-provided buffers).
-// `R` is null when h->dirs already holds this frame's directions (the update wrote them for its trace).
-ddgi_status enqueue_blend_and_publish(Handle* h, const Rot* R, const float4* rays, const uint16_t* order,
-									  uint32_t max_slots, bool all, uint32_t flags, hipStream_t s) {
+uint32_t blend_mode(uint32_t flags) {
+	return (flags & DDGI_UPDATE_BLEND_BF16) ? kBlendBF16 : ((flags & DDGI_UPDATE_BLEND_FP16) ? kBlendFP16 : kBlendFP32);
+}
+
+// The frame's part of an update or blend, without the list of probes.  `order`: the ray order of the ray
+// records (the traversal's thread order for ddgi_update, null = natural order for caller-provided buffers).
+FrameBegin frame_begin(Handle* h, const Rot& R, uint16_t* order, uint32_t mode) {
+	FrameBegin a{};
+	a.R = R;
+	a.grid = make_grid_const(*h);
+	a.fib = h->fib;
+	a.dirs = h->dirs;
+	a.order = order;
+	a.wt = h->wt;
+	a.inv_sum = h->inv_sum;
+	a.w_hi = h->w_hi;
+	a.w_lo = h->w_lo;
+	a.sel = h->sel;
+	a.indices = h->indices;
+	a.mode = mode;
+	return a;
+}
+
+// Blends `rays` with the weights that launch_frame_begin has written for the same flags.
+ddgi_status enqueue_blend_and_publish(Handle* h, const float4* rays, uint32_t max_slots, bool all, uint32_t flags, hipStream_t s) {
 	const GridConst g = make_grid_const(*h);
-	const uint32_t mode = (flags & DDGI_UPDATE_BLEND_BF16) ? kBlendBF16 : ((flags & DDGI_UPDATE_BLEND_FP16) ? kBlendFP16 : kBlendFP32);
-	if(R) HIP_TRY(h, launch_frame_dirs(*R, h->fib, h->dirs, g.n, s));
-	HIP_TRY(h, launch_blend_weights(g, h->dirs, order, h->wt, h->inv_sum, h->w_hi, h->w_lo, mode, s));
+	const uint32_t mode = blend_mode(flags);
 	const int nxt = h->cur ^ 1;
 	if(!all) {
 		// probes that are not updated keep their tiles: start the next atlas as a copy
@@ -922,15 +940,20 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	const bool all = (flags & DDGI_UPDATE_ALL_PROBES) != 0;
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[0], s));
 	uint32_t max_slots = h->P;
+	FrameBegin begin = frame_begin(h, R, h->perm, blend_mode(flags));
+	begin.counters = h->shade_count;
+	begin.count = h->P;
 	if(all) {
-		if(!h->indices_are_iota) HIP_TRY(h, launch_iota(h->indices, h->P, h->sel, s));
-		else HIP_TRY(h, launch_set_count(h->sel, h->P, s));
-		h->indices_are_iota = true;
+		begin.list = h->indices_are_iota ? kListKeep : kListIota;
 	} else {
-		HIP_TRY(h, launch_select(h->states, h->P, h->opts.probes_per_update, h->sel, h->indices, s));
-		h->indices_are_iota = false;
+		begin.list = kListSelect;
+		begin.states = h->states;
+		begin.probe_count = h->P;
+		begin.count = h->opts.probes_per_update;
 		if(h->opts.probes_per_update) max_slots = std::min(max_slots, h->opts.probes_per_update);
 	}
+	HIP_TRY(h, launch_frame_begin(begin, s));
+	h->indices_are_iota = all;
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[1], s));
 	if(flags & DDGI_UPDATE_HYSTERESIS_RAMP) {
 		uint32_t cnt = h->P;
@@ -945,7 +968,6 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	const GridConst g = make_grid_const(*h);
 	uint32_t key_shift = 0, key_bits = 0;  // shade-list ordering keys
 	shade_key_layout(g, &key_shift, &key_bits);
-	HIP_TRY(h, launch_frame_dirs_order(R, h->fib, h->dirs, g.n, h->perm, s, h->shade_count));
 	TraceFrameArgs a{};
 	a.scene = h->sd;
 	a.grid = g;
@@ -984,7 +1006,7 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	HIP_TRY(h, launch_shade(a, s));
 	if(h->light.sky_model == DDGI_SKY_ATMOSPHERE) HIP_TRY(h, launch_sky(a, s));
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
-	if((st = enqueue_blend_and_publish(h, nullptr, h->rays, h->perm, max_slots, all, flags, s)) != DDGI_OK) return st;
+	if((st = enqueue_blend_and_publish(h, h->rays, max_slots, all, flags, s)) != DDGI_OK) return st;
 	if(timing) {
 		HIP_TRY(h, hipEventRecord(h->ev[4], s));
 		HIP_TRY(h, hipEventRecord(h->ev[5], s));
@@ -1011,14 +1033,16 @@ ddgi_status ddgi_blend_rays(void* handle, const void* rays, const void* probe_in
 	const bool timing = !(flags & DDGI_UPDATE_NO_TIMING);
 	if(timing)
 		for(int k = 0; k < 4; ++k) HIP_TRY(h, hipEventRecord(h->ev[k], s));
-	HIP_TRY(h, hipMemcpyAsync(h->indices, probe_indices, size_t(count) * 4, hipMemcpyDeviceToDevice, s));
-	HIP_TRY(h, launch_set_count(h->sel, count, s));
+	FrameBegin begin = frame_begin(h, R, nullptr, blend_mode(flags));
+	begin.list = kListCopy;
+	begin.listed = static_cast<const uint32_t*>(probe_indices);
+	begin.count = count;
+	HIP_TRY(h, launch_frame_begin(begin, s));
 	h->indices_are_iota = false;
 	// the listed probes may not cover the grid: the next atlas starts as a copy of the exposed one,
 	// unless the caller states that they are every probe
 	const bool all = (flags & DDGI_UPDATE_ALL_PROBES) && count == h->P;
-	if((st = enqueue_blend_and_publish(h, &R, static_cast<const float4*>(rays), nullptr, count, all, flags, s)) != DDGI_OK)
-		return st;
+	if((st = enqueue_blend_and_publish(h, static_cast<const float4*>(rays), count, all, flags, s)) != DDGI_OK) return st;
 	if(timing) {
 		HIP_TRY(h, hipEventRecord(h->ev[4], s));
 		HIP_TRY(h, hipEventRecord(h->ev[5], s));
@@ -1132,8 +1156,14 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	HIP_TRY(h, hipMemcpyAsync(dep, h->dep[h->cur], P * 256 * sizeof(float2), hipMemcpyDeviceToDevice, s));
 	HIP_TRY(h, hipMemcpyAsync(states, h->states, P * 4, hipMemcpyDeviceToDevice, s));
 	const GridConst g = make_grid_const(*h);
-	HIP_TRY(h, launch_frame_dirs(R, h->fib, D.dirs, g.n, s));
-	HIP_TRY(h, launch_blend_weights(g, D.dirs, h->perm, D.wt, D.inv_sum, h->w_hi, h->w_lo, kBlendFP32, s));
+	{  // directions and weights kept for the context, in the order of the update's ray records
+		FrameBegin keep = frame_begin(h, R, h->perm, kBlendFP32);
+		keep.dirs = D.dirs;
+		keep.wt = D.wt;
+		keep.inv_sum = D.inv_sum;
+		keep.sel = nullptr;
+		HIP_TRY(h, launch_frame_begin(keep, s));
+	}
 	{
 		std::vector<uint32_t> iota(P);
 		std::iota(iota.begin(), iota.end(), 0u);

@@ -21,6 +21,7 @@ namespace ddgi {
 namespace {
 
 constexpr int kProbesPerBlock = 16;
+constexpr int kWRows = 256;  // padded weight rows: irr 0..47, depth 48..255
 
 // Column of ray i in the 16-bit weight rows, which only the wide MFMA blend reads: inside each
 // block of 32 rays, ray 4 j + g is stored at 8 g + j, so that the 8 consecutive weights a lane
@@ -28,13 +29,15 @@ constexpr int kProbesPerBlock = 16;
 // of each of 16 probes per instruction).
 __device__ __forceinline__ uint32_t wide_column(uint32_t i) { return (i & ~31u) | ((i & 3u) << 3) | ((i & 31u) >> 2); }
 
-// One block per padded weight row: the weight of every ray and their sum, stored in [row][n_pad]
+// One padded weight row by 256 threads (`lane`; red: 256 floats of LDS, and every thread of the workgroup
+// calls this with the same n_pad): the weight of every ray and their sum, stored in [row][n_pad]
 // layout as FP32, or as 16-bit copies (BF16: hi/lo split; FP16: one copy) in wide_column order.
-__device__ __forceinline__ void blend_weight_row(const GridConst& g, const float4* __restrict__ dirs,
-												 const uint16_t* __restrict__ order, float* __restrict__ wt,
+// dir_of(i): the direction of the ray that column i belongs to.
+template <class Direction>
+__device__ __forceinline__ void blend_weight_row(const GridConst& g, const Direction& dir_of, float* __restrict__ wt,
 												 float* __restrict__ inv_sum, void* __restrict__ w_hi_v,
-												 void* __restrict__ w_lo_v, uint32_t mode, uint32_t n_pad, uint32_t row) {
-	__shared__ float red[256];
+												 void* __restrict__ w_lo_v, uint32_t mode, uint32_t n_pad, uint32_t row,
+												 uint32_t lane, float* red) {
 	const bool irr_row = row < kIrrTexels;
 	const bool dep_row = row >= 48u && row < 48u + kDepTexels;
 	const bool valid = irr_row || dep_row;
@@ -45,10 +48,10 @@ __device__ __forceinline__ void blend_weight_row(const GridConst& g, const float
 	__bf16* w_lo = static_cast<__bf16*>(w_lo_v);
 	_Float16* w_h = static_cast<_Float16*>(w_hi_v);
 	float sum = 0.0f;
-	for(uint32_t i = threadIdx.x; i < n_pad; i += 256) {
+	for(uint32_t i = lane; i < n_pad; i += 256) {
 		float w = 0.0f;
 		if(valid && i < g.n) {
-			const float4 d = dirs[order ? order[i] : i];
+			const float4 d = dir_of(i);
 			w = fmaxf(0.0f, tx * d.x + ty * d.y + tz * d.z);
 			if(dep_row) w = powf(w, g.sharpness);
 		}
@@ -69,20 +72,169 @@ __device__ __forceinline__ void blend_weight_row(const GridConst& g, const float
 		}
 		sum += w;
 	}
-	red[threadIdx.x] = sum;
+	red[lane] = sum;
 	__syncthreads();
 	for(int o = 128; o > 0; o >>= 1) {
-		if(int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
+		if(int(lane) < o) red[lane] += red[lane + o];
 		__syncthreads();
 	}
-	if(threadIdx.x == 0 && valid) inv_sum[t] = red[0] > 1e-3f ? 1.0f / red[0] : 1.0f;
+	if(lane == 0 && valid) inv_sum[t] = red[0] > 1e-3f ? 1.0f / red[0] : 1.0f;
 }
 
-__global__ __launch_bounds__(256) void k_blend_weights(GridConst g, const float4* __restrict__ dirs,
-													   const uint16_t* __restrict__ order, float* __restrict__ wt,
-													   float* __restrict__ inv_sum, void* __restrict__ w_hi_v,
-													   void* __restrict__ w_lo_v, uint32_t mode, uint32_t n_pad) {
-	blend_weight_row(g, dirs, order, wt, inv_sum, w_hi_v, w_lo_v, mode, n_pad, blockIdx.x);
+// ---- device-side selectProbesToUpdate: one block of 1024 threads scans the round-robin order ----
+constexpr int kSelectBlock = 1024;
+
+__device__ __forceinline__ void select_probes(const uint32_t* __restrict__ states, uint32_t P, uint32_t cap,
+											  SelectState* st, uint32_t* __restrict__ out) {
+	__shared__ uint32_t wave_sums[kSelectBlock / 64];
+	__shared__ uint32_t s_base, s_stop_q, s_done;
+	const uint32_t off = st->last_offset, loop = st->loop_index;
+	if(threadIdx.x == 0) {
+		s_base = 0;
+		s_stop_q = 0xFFFFFFFFu;
+		s_done = 0;
+	}
+	__syncthreads();
+	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+	for(uint32_t chunk = 0; chunk < P; chunk += kSelectBlock) {
+		const uint32_t q = chunk + threadIdx.x;
+		bool pred = false;
+		uint32_t idx = 0;
+		if(q < P) {
+			idx = off + q;
+			uint32_t L = loop;
+			if(idx >= P) {
+				idx -= P;
+				L += 1u;
+			}
+			const uint32_t s = states[idx];
+			pred = (s != 0u) && ((idx + L) % s) == 0u;
+		}
+		// block-wide exclusive scan of pred
+		const uint64_t ballot = __ballot(pred);
+		const uint32_t in_wave = __popcll(ballot & ((uint64_t(1) << lane) - 1u));
+		if(lane == 0) wave_sums[wave] = __popcll(ballot);
+		__syncthreads();
+		uint32_t wave_off = 0;
+		for(uint32_t w = 0; w < wave; ++w) wave_off += wave_sums[w];
+		const uint32_t pos = s_base + wave_off + in_wave;
+		if(pred && (cap == 0u || pos < cap)) {
+			out[pos] = idx;
+			if(cap != 0u && pos == cap - 1u) s_stop_q = q;  // exactly one thread
+		}
+		__syncthreads();
+		if(threadIdx.x == 0) {
+			uint32_t tot = 0;
+			for(uint32_t w = 0; w < kSelectBlock / 64; ++w) tot += wave_sums[w];
+			s_base += tot;
+			if(cap != 0u && s_base >= cap) s_done = 1;
+		}
+		__syncthreads();
+		if(s_done) break;
+	}
+	if(threadIdx.x == 0) {
+		uint32_t cnt = s_base;
+		if(cap != 0u && cnt > cap) cnt = cap;
+		st->count = cnt;
+		if(s_stop_q != 0xFFFFFFFFu) {
+			const uint32_t next = off + s_stop_q + 1u;
+			st->last_offset = next >= P ? next - P : next;
+			st->loop_index = loop + (next >= P ? 1u : 0u);
+		} else {
+			st->last_offset = off;
+			st->loop_index = loop + 1u;
+		}
+	}
+}
+
+// ---- start of an update or of a blend: everything that depends on the orientation alone ----
+// One launch for what were up to four: the frame's ray directions, their thread order, the blend weights
+// and the list of probes.  Each is a few microseconds of latency and no work to speak of, so a small update
+// is bound by their number: with 256 probes of 128 rays, directions and order 5.0, count 3.5, weights 4.3 us
+// and the gaps between them, against 5.2 us here (1024 probes of 256 rays selected of 16384: 8.6, was 8.3 +
+// 7.3 + 5.0).  Every workgroup derives the directions and the order in LDS (the rank of a ray: 2 to 8 threads
+// share its comparisons) and then computes four weight rows; workgroup 0 stores directions and order, and
+// one more workgroup selects the probes of a partial update meanwhile.
+constexpr uint32_t kBeginThreads = 1024;
+constexpr uint32_t kBeginRows = kBeginThreads / 256;
+static_assert(kBeginThreads == kSelectBlock && kBeginThreads >= 2 * kMaxRays, "one block size for both jobs");
+
+// frame_dir of the trace kernels, bit for bit: products and sums rounded one by one, in a file whose
+// multiplications and additions the compiler otherwise fuses
+__device__ __forceinline__ float4 frame_dir_unfused(const Rot& R, const float4& f) {
+	float d[3];
+#pragma unroll
+	for(int k = 0; k < 3; ++k) {
+		float x = R.r[k * 3 + 0] * f.x, y = R.r[k * 3 + 1] * f.y, z = R.r[k * 3 + 2] * f.z;
+		__asm__ volatile("" : "+v"(x), "+v"(y), "+v"(z));
+		d[k] = x + y + z;
+	}
+	return make_float4(d[0], d[1], d[2], 0.0f);
+}
+
+__global__ __launch_bounds__(kBeginThreads) void k_frame_begin(FrameBegin a) {
+	__shared__ __attribute__((aligned(16))) float s_key[kMaxRays];
+	__shared__ uint32_t s_rank[kMaxRays];
+	__shared__ float4 s_dir[kMaxRays];  // in thread order
+	__shared__ float s_red[kBeginThreads];
+	const uint32_t t = threadIdx.x, n = a.grid.n;
+	if(blockIdx.x == kWRows / kBeginRows) {  // only launched for kListSelect
+		select_probes(a.states, a.probe_count, a.count, a.sel, a.indices);
+		return;
+	}
+	const uint32_t id = blockIdx.x * kBeginThreads + t, all = kWRows / kBeginRows * kBeginThreads;
+	if(a.list == kListIota)
+		for(uint32_t i = id; i < a.count; i += all) a.indices[i] = i;
+	if(a.list == kListCopy)
+		for(uint32_t i = id; i < a.count; i += all) a.indices[i] = a.listed[i];
+	float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	if(t < n) d = frame_dir_unfused(a.R, a.fib[t]);
+	if(a.order) {
+		// rays sorted by the elevation of their world direction, ties by ray index; keys past n are +infinity,
+		// which no finite key counts.  Thread t counts for ray t % m the smaller keys of part t / m of the
+		// four-key groups (wave-uniform parts: every lane of a wave reads the same address)
+		const uint32_t m = n > 256u ? 512u : n > 128u ? 256u : 128u, parts = kBeginThreads / m;
+		if(t < kMaxRays) {
+			s_key[t] = t < n ? d.y : __int_as_float(0x7f800000);
+			s_rank[t] = 0u;
+		}
+		__syncthreads();
+		const uint32_t i = t & (m - 1u), part = __builtin_amdgcn_readfirstlane(t / m);
+		if(i < n) {
+			const float y = s_key[i];
+			const uint32_t groups = (n + 3u) / 4u, per = (groups + parts - 1u) / parts;
+			const uint32_t g1 = min(groups, (part + 1u) * per);
+			uint32_t rank = 0;
+			const float4* k4 = reinterpret_cast<const float4*>(s_key);
+#pragma unroll 4
+			for(uint32_t j = part * per; j < g1; ++j) {
+				const float4 k = k4[j];
+				const uint32_t j0 = 4u * j;
+				rank += (k.x < y || (k.x == y && j0 < i)) ? 1u : 0u;
+				rank += (k.y < y || (k.y == y && j0 + 1u < i)) ? 1u : 0u;
+				rank += (k.z < y || (k.z == y && j0 + 2u < i)) ? 1u : 0u;
+				rank += (k.w < y || (k.w == y && j0 + 3u < i)) ? 1u : 0u;
+			}
+			atomicAdd(&s_rank[i], rank);
+		}
+		__syncthreads();
+	}
+	if(t < n) {
+		const uint32_t pos = a.order ? s_rank[t] : t;
+		s_dir[pos] = d;
+		if(blockIdx.x == 0) {
+			a.dirs[t] = d;
+			if(a.order) a.order[pos] = uint16_t(t);
+		}
+	}
+	if(blockIdx.x == 0) {
+		if(a.counters && t < kShadeSegments) a.counters[kCounterStride * t] = 0u;
+		if(a.counters && t == 0) a.counters[kMissCountSlot] = 0u;
+		if(a.sel && a.list != kListSelect && t == 0) a.sel->count = a.count;
+	}
+	__syncthreads();
+	blend_weight_row(a.grid, [&](uint32_t i) { return s_dir[i]; }, a.wt, a.inv_sum, a.w_hi, a.w_lo, a.mode, a.n_pad,
+					 blockIdx.x * kBeginRows + __builtin_amdgcn_readfirstlane(t >> 8), t & 255u, s_red + (t & ~255u));
 }
 
 // The interior texel whose blended value texel (x, y) of an R x R tile holds after the border copy:
@@ -264,7 +416,6 @@ __device__ __forceinline__ void update_state(uint32_t* states, uint32_t probe, f
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kMfmaChunk = 64;              // rays staged per LDS chunk
-constexpr int kWRows = 256;                 // padded weight rows: irr 0..47, depth 48..255
 constexpr int kDepRow0 = 48;
 
 template <int NP>
@@ -999,8 +1150,12 @@ __global__ __launch_bounds__(kTileThreads) void k_blend_tile(BlendArgs a, uint32
 // ---- batched update ----
 // Weight rows of every volume: grid (256 rows, volumes).
 __global__ __launch_bounds__(256) void k_batch_weights(BatchLaunch b) {
+	__shared__ float red[256];
 	const BatchVolume& v = b.vols[blockIdx.y];
-	blend_weight_row(v.blend.grid, v.dirs, v.perm, v.wt, v.inv_sum, v.w_hi, v.w_lo, b.blend_mode, v.n_pad, blockIdx.x);
+	const float4* __restrict__ dirs = v.dirs;
+	const uint16_t* __restrict__ order = v.perm;
+	blend_weight_row(v.blend.grid, [&](uint32_t i) { return dirs[order[i]]; }, v.wt, v.inv_sum, v.w_hi, v.w_lo, b.blend_mode,
+					 v.n_pad, blockIdx.x, threadIdx.x, red);
 }
 
 // Blend over the tiles of all volumes: one workgroup per blend item (a tile of one volume's probe
@@ -1075,11 +1230,10 @@ const void* batch_blend_kernel(uint32_t mode, uint32_t probes) {
 
 }  // namespace
 
-hipError_t launch_blend_weights(const GridConst& g, const float4* dirs, const uint16_t* order, float* wt, float* inv_sum,
-								void* w_hi16, void* w_lo16, uint32_t mode, hipStream_t s) {
-	const uint32_t n_pad = (g.n + kMfmaChunk - 1) & ~uint32_t(kMfmaChunk - 1);
-	hipLaunchKernelGGL(k_blend_weights, dim3(kWRows), dim3(256), 0, s, g, dirs, order, wt, inv_sum, w_hi16, w_lo16, mode,
-					   n_pad);
+hipError_t launch_frame_begin(FrameBegin a, hipStream_t s) {
+	if(a.grid.n == 0 || a.grid.n > kMaxRays) return hipErrorInvalidValue;
+	a.n_pad = (a.grid.n + kMfmaChunk - 1) & ~uint32_t(kMfmaChunk - 1);
+	hipLaunchKernelGGL(k_frame_begin, dim3(kWRows / kBeginRows + (a.list == kListSelect ? 1 : 0)), dim3(kBeginThreads), 0, s, a);
 	return hipGetLastError();
 }
 

@@ -255,13 +255,7 @@ struct SortJobs {
 uint32_t sort_fine_bits(uint32_t key_bits);
 
 // ---- launchers (return hipGetLastError of the launch) ----
-// The frame's directions (as launch_frame_dirs) and thread -> ray order (kMaxRays entries; the first
-// n sorted by the world elevation of the directions, ties by ray index, the rest unchanged).
-hipError_t launch_frame_dirs_order(const Rot& R, const float4* fib, float4* dirs, uint32_t n, uint16_t* perm,
-								   hipStream_t s, uint32_t* zero = nullptr);
-// zero (optional): a counter cleared by the same launch
-hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint32_t count, hipStream_t s,
-							 uint32_t* zero = nullptr);
+hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint32_t count, hipStream_t s);
 // Orders job.list (keys job.keys of key_bits <= 18 bits; input in job.segments segments, output
 // contiguous, at most `capacity` entries) in place: by the keys' high 10 bits over the whole list,
 // and by the whole key inside each fixed chunk of 4096 entries (a bucket of equal high bits longer
@@ -293,17 +287,41 @@ hipError_t launch_reflection_trace(const ReflectionArgs& a, hipStream_t s);
 hipError_t launch_reflection_shade(const ReflectionArgs& a, hipStream_t s);
 hipError_t launch_init_probes(const SceneDev& sc, const GridConst& g, const float4* dirs512, uint32_t* states,
 							  uint32_t* backface_counts, hipStream_t s);
-hipError_t launch_select(const uint32_t* states, uint32_t P, uint32_t cap, SelectState* st, uint32_t* indices,
-						 hipStream_t s);
 hipError_t launch_iota(uint32_t* indices, uint32_t P, SelectState* st, hipStream_t s);
-hipError_t launch_set_count(SelectState* st, uint32_t count, hipStream_t s);
 hipError_t launch_sample(const GridConst& g, const uint32_t* states, const float4* irr, const float2* dep,
 						 const float* pos, const float* nrm, const float* tocam, uint64_t count, float* out,
 						 hipStream_t s);
-// Weight row k uses direction dirs[order[k]] (order = nullptr: identity), so that the blend can
-// consume ray records stored in the traversal's thread order.
-hipError_t launch_blend_weights(const GridConst& g, const float4* dirs, const uint16_t* order, float* wt, float* inv_sum,
-								void* w_hi16, void* w_lo16, uint32_t mode, hipStream_t s);
+// The start of an update or a blend: the frame's directions fib * R, the thread -> ray order (the first n
+// entries: rays sorted by the elevation of their world direction, ties by ray index), the weight rows of the
+// blend (column k: ray order[k], so that the blend can consume ray records stored in that order) and the list of probes.
+enum : uint32_t {
+	kListKeep,    // the list stays; sel->count = count
+	kListIota,    // 0 .. count - 1
+	kListCopy,    // `count` entries of `listed`
+	kListSelect,  // the due probes of probe_count by their states, at most `count` (0: no bound)
+};
+struct FrameBegin {
+	Rot R;
+	GridConst grid;
+	const float4* fib;
+	float4* dirs;
+	uint16_t* order;         // null: natural order
+	uint32_t* counters;      // optional: the shade-list counters, cleared
+	float* wt;
+	float* inv_sum;
+	void* w_hi;
+	void* w_lo;
+	SelectState* sel;        // optional with kListKeep
+	uint32_t* indices;
+	const uint32_t* listed;
+	const uint32_t* states;
+	uint32_t mode;           // blend mode
+	uint32_t list;           // kList...
+	uint32_t count;
+	uint32_t probe_count;
+	uint32_t n_pad;          // set by the launcher
+};
+hipError_t launch_frame_begin(FrameBegin a, hipStream_t s);
 // Picks the workgroup shape by the number of slots and of the device's compute units (0: unknown); every
 // shape gives the same sums (the same MFMAs per output element, in the same order).
 hipError_t launch_blend(const BlendArgs& a, uint32_t mode, uint32_t cus, hipStream_t s);

@@ -37,18 +37,13 @@ __device__ __forceinline__ float4 frame_dir(const Rot& R, float4 f) {
 	return make_float4(d[0], d[1], d[2], 0.0f);
 }
 
-// `zero` (optional): two counters the next kernels start from (the shade- and miss-list lengths),
-// cleared here so that no separate memset is needed.
 __global__ void k_clear(uint32_t* __restrict__ words, uint32_t n) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if(i < n) words[i] = 0u;
 }
 
-__global__ void k_frame_dirs(Rot R, const float4* __restrict__ fib, float4* __restrict__ dirs, uint32_t count,
-							 uint32_t* zero) {
+__global__ void k_frame_dirs(Rot R, const float4* __restrict__ fib, float4* __restrict__ dirs, uint32_t count) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if(zero && i < kShadeSegments) zero[kCounterStride * i] = 0u;
-	if(zero && i == 0) zero[kMissCountSlot] = 0u;
 	if(i >= count) return;
 	dirs[i] = frame_dir(R, fib[i]);
 }
@@ -79,24 +74,6 @@ __device__ __forceinline__ void frame_order_block(float y, uint32_t n, float* s_
 		}
 		perm[rank] = uint16_t(i);
 	}
-}
-
-// The update's frame directions and thread -> ray order in one workgroup of kMaxRays threads
-// (thread i: ray i); `zero` as in k_frame_dirs.
-__global__ __launch_bounds__(kMaxRays) void k_frame_dirs_order(Rot R, const float4* __restrict__ fib,
-															   float4* __restrict__ dirs, uint32_t n, uint16_t* perm,
-															   uint32_t* zero) {
-	__shared__ __attribute__((aligned(16))) float s_key[kMaxRays];
-	const uint32_t i = threadIdx.x;
-	if(zero && i < kShadeSegments) zero[kCounterStride * i] = 0u;
-	if(zero && i == 0) zero[kMissCountSlot] = 0u;
-	float y = 0.0f;
-	if(i < n) {
-		const float4 d = frame_dir(R, fib[i]);
-		dirs[i] = d;
-		y = d.y;
-	}
-	frame_order_block(y, n, s_key, perm);
 }
 
 // Ray records of rays that need no shading: misses.rmiss (sky radiance, depth -1) and back faces
@@ -1260,76 +1237,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_init_probes(SceneDev sc, GridCo
 	}
 }
 
-// ---- device-side selectProbesToUpdate: one block of 1024 threads scans the round-robin order ----
-constexpr int kSelectBlock = 1024;
-
-__global__ __launch_bounds__(kSelectBlock) void k_select(const uint32_t* __restrict__ states, uint32_t P, uint32_t cap,
-														 SelectState* st, uint32_t* __restrict__ out) {
-	__shared__ uint32_t wave_sums[kSelectBlock / 64];
-	__shared__ uint32_t s_base, s_stop_q, s_done;
-	const uint32_t off = st->last_offset, loop = st->loop_index;
-	if(threadIdx.x == 0) {
-		s_base = 0;
-		s_stop_q = 0xFFFFFFFFu;
-		s_done = 0;
-	}
-	__syncthreads();
-	const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-	for(uint32_t chunk = 0; chunk < P; chunk += kSelectBlock) {
-		const uint32_t q = chunk + threadIdx.x;
-		bool pred = false;
-		uint32_t idx = 0;
-		if(q < P) {
-			idx = off + q;
-			uint32_t L = loop;
-			if(idx >= P) {
-				idx -= P;
-				L += 1u;
-			}
-			const uint32_t s = states[idx];
-			pred = (s != 0u) && ((idx + L) % s) == 0u;
-		}
-		// block-wide exclusive scan of pred
-		const uint64_t ballot = __ballot(pred);
-		const uint32_t in_wave = __popcll(ballot & ((uint64_t(1) << lane) - 1u));
-		if(lane == 0) wave_sums[wave] = __popcll(ballot);
-		__syncthreads();
-		uint32_t wave_off = 0;
-		for(uint32_t w = 0; w < wave; ++w) wave_off += wave_sums[w];
-		const uint32_t pos = s_base + wave_off + in_wave;
-		if(pred && (cap == 0u || pos < cap)) {
-			out[pos] = idx;
-			if(cap != 0u && pos == cap - 1u) s_stop_q = q;  // exactly one thread
-		}
-		__syncthreads();
-		if(threadIdx.x == 0) {
-			uint32_t tot = 0;
-			for(uint32_t w = 0; w < kSelectBlock / 64; ++w) tot += wave_sums[w];
-			s_base += tot;
-			if(cap != 0u && s_base >= cap) s_done = 1;
-		}
-		__syncthreads();
-		if(s_done) break;
-	}
-	if(threadIdx.x == 0) {
-		uint32_t cnt = s_base;
-		if(cap != 0u && cnt > cap) cnt = cap;
-		st->count = cnt;
-		if(s_stop_q != 0xFFFFFFFFu) {
-			const uint32_t next = off + s_stop_q + 1u;
-			st->last_offset = next >= P ? next - P : next;
-			st->loop_index = loop + (next >= P ? 1u : 0u);
-		} else {
-			st->last_offset = off;
-			st->loop_index = loop + 1u;
-		}
-	}
-}
-
-__global__ void k_set_count(SelectState* st, uint32_t c) {
-	if(blockIdx.x == 0 && threadIdx.x == 0) st->count = c;
-}
-
 __global__ void k_iota(uint32_t* __restrict__ out, uint32_t P, SelectState* st) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if(i < P) out[i] = i;
@@ -1353,17 +1260,8 @@ inline uint32_t blocks_for(uint64_t n, uint32_t b) { return uint32_t((n + b - 1)
 
 }  // namespace
 
-hipError_t launch_frame_dirs_order(const Rot& R, const float4* fib, float4* dirs, uint32_t n, uint16_t* perm,
-								   hipStream_t s, uint32_t* zero) {
-	static_assert(kShadeSegments <= kMaxRays, "one thread clears each shade-list counter");
-	if(n == 0 || n > kMaxRays) return hipErrorInvalidValue;
-	hipLaunchKernelGGL(k_frame_dirs_order, dim3(1), dim3(kMaxRays), 0, s, R, fib, dirs, n, perm, zero);
-	return hipGetLastError();
-}
-
-hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint32_t count, hipStream_t s,
-							 uint32_t* zero) {
-	hipLaunchKernelGGL(k_frame_dirs, dim3(blocks_for(count, 256)), dim3(256), 0, s, R, fib, dirs, count, zero);
+hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint32_t count, hipStream_t s) {
+	hipLaunchKernelGGL(k_frame_dirs, dim3(blocks_for(count, 256)), dim3(256), 0, s, R, fib, dirs, count);
 	return hipGetLastError();
 }
 
@@ -1511,17 +1409,6 @@ hipError_t launch_init_probes(const SceneDev& sc, const GridConst& g, const floa
 							  uint32_t* backface_counts, hipStream_t s) {
 	if(g.probe_count == 0) return hipSuccess;
 	hipLaunchKernelGGL(k_init_probes<kLdsStack>, dim3(g.probe_count), dim3(kTraceBlock), 0, s, sc, g, dirs512, states, backface_counts);
-	return hipGetLastError();
-}
-
-hipError_t launch_select(const uint32_t* states, uint32_t P, uint32_t cap, SelectState* st, uint32_t* indices,
-						 hipStream_t s) {
-	hipLaunchKernelGGL(k_select, dim3(1), dim3(kSelectBlock), 0, s, states, P, cap, st, indices);
-	return hipGetLastError();
-}
-
-hipError_t launch_set_count(SelectState* st, uint32_t count, hipStream_t s) {
-	hipLaunchKernelGGL(k_set_count, dim3(1), dim3(64), 0, s, st, count);
 	return hipGetLastError();
 }
 
