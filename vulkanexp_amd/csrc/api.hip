@@ -353,6 +353,8 @@ void destroy_handle(Handle* h) {
 	for(auto& e : h->ev)
 		if(e) (void)hipEventDestroy(e);
 	if(h->move_done) (void)hipEventDestroy(h->move_done);
+	if(h->selected_ready) (void)hipEventDestroy(h->selected_ready);
+	if(h->selected) (void)hipHostFree(h->selected);
 	delete h;
 }
 
@@ -379,12 +381,14 @@ FrameBegin frame_begin(Handle* h, const Rot& R, uint16_t* order, uint32_t mode) 
 	return a;
 }
 
-// Blends `rays` with the weights that launch_frame_begin has written for the same flags.
-ddgi_status enqueue_blend_and_publish(Handle* h, const float4* rays, uint32_t max_slots, bool all, uint32_t flags, hipStream_t s) {
+// Blends `rays` with the weights that launch_frame_begin has written for the same flags; `copied`: the next
+// atlas holds the exposed one already, or every tile of it is written.
+ddgi_status enqueue_blend_and_publish(Handle* h, const float4* rays, uint32_t max_slots, bool copied, uint32_t flags,
+									  hipStream_t s) {
 	const GridConst g = make_grid_const(*h);
 	const uint32_t mode = blend_mode(flags);
 	const int nxt = h->cur ^ 1;
-	if(!all) {
+	if(!copied) {
 		// probes that are not updated keep their tiles: start the next atlas as a copy
 		HIP_TRY(h, hipMemcpyAsync(h->irr[nxt], h->irr[h->cur], size_t(h->P) * 64 * sizeof(float4), hipMemcpyDeviceToDevice, s));
 		HIP_TRY(h, hipMemcpyAsync(h->dep[nxt], h->dep[h->cur], size_t(h->P) * 256 * sizeof(float2), hipMemcpyDeviceToDevice, s));
@@ -620,7 +624,13 @@ ddgi_status ddgi_create(const ddgi_grid_params* params, const ddgi_options* opti
 		std::vector<uint32_t> ones(P, 1u);
 		e = hipMemcpy(h->states, ones.data(), P * 4, hipMemcpyHostToDevice);
 	}
-	for(int i = 0; i < 6 && e == hipSuccess; ++i) e = hipEventCreate(&h->ev[i]);
+	for(int i = 0; i < 5 && e == hipSuccess; ++i) e = hipEventCreate(&h->ev[i]);
+	if(e == hipSuccess) e = hipEventCreateWithFlags(&h->selected_ready, hipEventDisableTiming);
+	if(e == hipSuccess) {
+		void* p = nullptr;
+		e = hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocDefault);
+		h->selected = static_cast<uint32_t*>(p);
+	}
 	if(e != hipSuccess) {
 		h->err = std::string("initialisation failed: ") + hipGetErrorString(e);
 		return cleanup_fail(DDGI_ERROR_HIP);
@@ -952,19 +962,21 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 		begin.count = h->opts.probes_per_update;
 		if(h->opts.probes_per_update) max_slots = std::min(max_slots, h->opts.probes_per_update);
 	}
+	// The ramp moves by the number of updated probes, which the selection leaves on the device: the host waits
+	// for it only when it has enqueued the tracing, so that the device does not wait for the host.
+	const bool ramp = (flags & DDGI_UPDATE_HYSTERESIS_RAMP) != 0, late_count = ramp && !all;
+	if(late_count) {
+		hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+		HIP_TRY(h, hipStreamIsCapturing(s, &capture));
+		if(capture != hipStreamCaptureStatusNone)
+			return fail(h, DDGI_ERROR_HIP, "the hysteresis ramp of a partial update reads the device and cannot be captured");
+		begin.host_count = h->selected;
+	}
 	HIP_TRY(h, launch_frame_begin(begin, s));
 	h->indices_are_iota = all;
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[1], s));
-	if(flags & DDGI_UPDATE_HYSTERESIS_RAMP) {
-		uint32_t cnt = h->P;
-		if(!all) {
-			SelectState ss;
-			HIP_TRY(h, hipMemcpyAsync(&ss, h->sel, sizeof(ss), hipMemcpyDeviceToHost, s));
-			HIP_TRY(h, hipStreamSynchronize(s));
-			cnt = ss.count;
-		}
-		advance_hysteresis(h, cnt);
-	}
+	const hipEvent_t counted = timing ? h->ev[1] : h->selected_ready;
+	if(late_count && !timing) HIP_TRY(h, hipEventRecord(counted, s));
 	const GridConst g = make_grid_const(*h);
 	uint32_t key_shift = 0, key_bits = 0;  // shade-list ordering keys
 	shade_key_layout(g, &key_shift, &key_bits);
@@ -1003,14 +1015,26 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 		HIP_TRY(h, launch_key_sort(SortJob{h->shade_keys, h->shade_list, h->shade_count, h->sort_counts, h->sort_keys,
 										   h->sort_list, h->shade_count + kShadeTotalSlot, 0u, kShadeSegments, a.seg_cap, 0u},
 								   uint64_t(max_slots) * g.n, 3 * key_bits, s));
+	const bool beside = !all && h->P < (1u << 24);
+	if(beside) {  // probes that are not updated keep their tiles: the next atlas starts as a copy, made beside the shading
+		const int nxt = h->cur ^ 1;
+		a.copy_src[0] = h->irr[h->cur];
+		a.copy_dst[0] = h->irr[nxt];
+		a.copy_n[0] = h->P * 64u;
+		a.copy_src[1] = reinterpret_cast<const float4*>(h->dep[h->cur]);
+		a.copy_dst[1] = reinterpret_cast<float4*>(h->dep[nxt]);
+		a.copy_n[1] = h->P * 128u;
+	}
 	HIP_TRY(h, launch_shade(a, s));
 	if(h->light.sky_model == DDGI_SKY_ATMOSPHERE) HIP_TRY(h, launch_sky(a, s));
 	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
-	if((st = enqueue_blend_and_publish(h, h->rays, max_slots, all, flags, s)) != DDGI_OK) return st;
+	if(late_count) HIP_TRY(h, hipEventSynchronize(counted));
+	if(ramp) advance_hysteresis(h, all ? h->P : *h->selected);
+	if((st = enqueue_blend_and_publish(h, h->rays, max_slots, all || beside, flags, s)) != DDGI_OK) return st;
 	if(timing) {
 		HIP_TRY(h, hipEventRecord(h->ev[4], s));
-		HIP_TRY(h, hipEventRecord(h->ev[5], s));
 		h->timing_pending = true;
+		h->timing_from = 0;
 	}
 	h->last_count = all ? h->P : 0xFFFFFFFFu;
 	h->last_stream = s;
@@ -1031,8 +1055,7 @@ ddgi_status ddgi_blend_rays(void* handle, const void* rays, const void* probe_in
 	if(st != DDGI_OK || (st = ensure_fib(h)) != DDGI_OK) return st;
 	hipStream_t s = static_cast<hipStream_t>(stream);
 	const bool timing = !(flags & DDGI_UPDATE_NO_TIMING);
-	if(timing)
-		for(int k = 0; k < 4; ++k) HIP_TRY(h, hipEventRecord(h->ev[k], s));
+	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
 	FrameBegin begin = frame_begin(h, R, nullptr, blend_mode(flags));
 	begin.list = kListCopy;
 	begin.listed = static_cast<const uint32_t*>(probe_indices);
@@ -1045,8 +1068,8 @@ ddgi_status ddgi_blend_rays(void* handle, const void* rays, const void* probe_in
 	if((st = enqueue_blend_and_publish(h, static_cast<const float4*>(rays), count, all, flags, s)) != DDGI_OK) return st;
 	if(timing) {
 		HIP_TRY(h, hipEventRecord(h->ev[4], s));
-		HIP_TRY(h, hipEventRecord(h->ev[5], s));
 		h->timing_pending = true;
+		h->timing_from = 3;
 	}
 	h->last_count = count;
 	h->last_stream = s;
@@ -1505,9 +1528,9 @@ ddgi_status ddgi_get_timings(void* handle, ddgi_timings* out) {
 	ddgi_status st = set_device(h);
 	if(st != DDGI_OK) return st;
 	if(h->timing_pending) {
-		HIP_TRY(h, hipEventSynchronize(h->ev[5]));
-		float ms[5] = {};
-		for(int i = 0; i < 5; ++i) HIP_TRY(h, hipEventElapsedTime(&ms[i], h->ev[i], h->ev[i + 1]));
+		HIP_TRY(h, hipEventSynchronize(h->ev[4]));
+		float ms[4] = {};
+		for(int i = h->timing_from; i < 4; ++i) HIP_TRY(h, hipEventElapsedTime(&ms[i], h->ev[i], h->ev[i + 1]));
 		h->last.select_ms = ms[0];
 		h->last.primary_ms = ms[1];
 		h->last.shade_ms = ms[2];
@@ -1515,7 +1538,7 @@ ddgi_status ddgi_get_timings(void* handle, ddgi_timings* out) {
 		h->last.blend_ms = ms[3];
 		h->last.border_ms = 0.0f;
 		h->last.copy_ms = 0.0f;
-		HIP_TRY(h, hipEventElapsedTime(&h->last.total_ms, h->ev[0], h->ev[5]));
+		HIP_TRY(h, hipEventElapsedTime(&h->last.total_ms, h->ev[h->timing_from], h->ev[4]));
 		uint32_t cnt = h->last_count;
 		if(cnt == 0xFFFFFFFFu) {
 			SelectState ss;

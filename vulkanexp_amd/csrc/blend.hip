@@ -180,6 +180,7 @@ __global__ __launch_bounds__(kBeginThreads) void k_frame_begin(FrameBegin a) {
 	const uint32_t t = threadIdx.x, n = a.grid.n;
 	if(blockIdx.x == kWRows / kBeginRows) {  // only launched for kListSelect
 		select_probes(a.states, a.probe_count, a.count, a.sel, a.indices);
+		if(a.host_count && t == 0) *a.host_count = a.sel->count;  // thread 0 stored it
 		return;
 	}
 	const uint32_t id = blockIdx.x * kBeginThreads + t, all = kWRows / kBeginRows * kBeginThreads;

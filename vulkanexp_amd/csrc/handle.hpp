@@ -82,8 +82,11 @@ struct Handle {
 	bool move_pending = false;
 	LightConst light{};
 	// timing
-	hipEvent_t ev[6] = {};
+	hipEvent_t ev[5] = {};  // start, list and weights ready, primary rays, shading, end
 	bool timing_pending = false;
+	int timing_from = 0;           // first event of the pending timings (3: a blend alone)
+	uint32_t* selected = nullptr;  // pinned: probes of the last partial update under the ramp
+	hipEvent_t selected_ready = nullptr;
 	ddgi_timings last{};
 	uint32_t last_count = 0xFFFFFFFFu;
 	uint32_t updated_probes = 0;  // hysteresis ramp bookkeeping (src/IrradianceProbes.cpp:463)

@@ -146,6 +146,11 @@ struct TraceFrameArgs {
 	uint32_t key_shift;
 	// the shade list is kShadeSegments segments of seg_cap entries
 	uint32_t seg_cap;
+	// optional (launch_shade): arrays copied by workgroups that follow the shading ones, counted in float4
+	const float4* copy_src[2];
+	float4* copy_dst[2];
+	uint32_t copy_n[2];
+	uint32_t shade_blocks;  // set by launch_shade
 };
 constexpr uint32_t kShadeSortCounts = 1024 * 128 + 1024;  // (list tile, coarse digit) counters + digit totals
 
@@ -320,6 +325,7 @@ struct FrameBegin {
 	uint32_t count;
 	uint32_t probe_count;
 	uint32_t n_pad;          // set by the launcher
+	uint32_t* host_count;    // optional with kListSelect: pinned host memory that receives the count
 };
 hipError_t launch_frame_begin(FrameBegin a, hipStream_t s);
 // Picks the workgroup shape by the number of slots and of the device's compute units (0: unknown); every

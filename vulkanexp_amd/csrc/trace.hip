@@ -516,6 +516,26 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, size_t k, uin
 	}
 }
 
+// Copies of a partial update (the next atlases start as the exposed ones): 64 x 16 float4 per workgroup,
+// all loads in flight.  They ride along with the shading, which leaves the memory idle: 50 MB took two
+// copies of 20 us each by themselves, and 10 us more of shading here.
+constexpr uint32_t kCopyPerBlock = kShadeBlock * 16u;
+__device__ __forceinline__ void copy_block(const TraceFrameArgs& a, uint32_t b) {
+	const uint32_t first = (a.copy_n[0] + kCopyPerBlock - 1u) / kCopyPerBlock;
+	const uint32_t which = b >= first ? 1u : 0u;
+	const uint32_t i0 = (b - (which ? first : 0u)) * kCopyPerBlock + threadIdx.x;
+	const uint32_t n = which ? a.copy_n[1] : a.copy_n[0];
+	const float4* __restrict__ src = which ? a.copy_src[1] : a.copy_src[0];
+	float4* __restrict__ dst = which ? a.copy_dst[1] : a.copy_dst[0];
+	float4 v[16];
+#pragma unroll
+	for(uint32_t u = 0; u < 16u; ++u)
+		if(i0 + kShadeBlock * u < n) v[u] = src[i0 + kShadeBlock * u];
+#pragma unroll
+	for(uint32_t u = 0; u < 16u; ++u)
+		if(i0 + kShadeBlock * u < n) dst[i0 + kShadeBlock * u] = v[u];
+}
+
 // One thread per entry of the shade list (ordered, or in its segments as appended), over a grid sized for the
 // list's capacity (its length is known only on the device; workgroups past it end at once).  The hardware refills a CU
 // as soon as one of its workgroups ends, so the CUs stay busy to the end of the list, which a
@@ -526,6 +546,10 @@ __device__ __forceinline__ void shade_ray(const TraceFrameArgs& a, size_t k, uin
 template <int STACK, bool COUNT>
 __global__ __launch_bounds__(kShadeBlock, 4) void k_shade(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
+	if(blockIdx.x >= a.shade_blocks) {
+		copy_block(a, blockIdx.x - a.shade_blocks);
+		return;
+	}
 	if(a.shade_keys) {
 		const uint32_t k = blockIdx.x * kShadeBlock + threadIdx.x;
 		if(k < a.shade_count[kShadeTotalSlot]) shade_ray<STACK, COUNT>(a, k, stack + threadIdx.x);
@@ -1335,8 +1359,9 @@ hipError_t launch_shade(const TraceFrameArgs& a, hipStream_t s) {
 	const bool cnt = a.visit_counters != nullptr;
 	const void* f = cnt ? reinterpret_cast<const void*>(&k_shade<kLdsStack, true>)
 						: reinterpret_cast<const void*>(&k_shade<kLdsStack, false>);
-	const dim3 grid(blocks_for(threads, kShadeBlock));  // one thread per entry the list can hold
 	TraceFrameArgs arg = a;
+	arg.shade_blocks = blocks_for(threads, kShadeBlock);  // one thread per entry the list can hold
+	const dim3 grid(arg.shade_blocks + blocks_for(a.copy_n[0], kCopyPerBlock) + blocks_for(a.copy_n[1], kCopyPerBlock));
 	void* args[] = {&arg};
 	return hipLaunchKernel(f, grid, dim3(kShadeBlock), args, 0, s);
 }
