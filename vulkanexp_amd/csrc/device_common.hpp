@@ -622,9 +622,11 @@ __device__ __forceinline__ bool make_cage(const GridConst& g, Vec3 position, Cag
 __device__ __forceinline__ bool cage_corner(const GridConst& g, const uint32_t* __restrict__ states, const Cage& c,
 											Vec3 position, int i, uint32_t& lin, Vec3& pp, Vec3& dtp, float& trw) {
 	const int o0 = i & 1, o1 = (i >> 1) & 1, o2 = (i >> 2) & 1;
-	const int p0i = c.f[0] + o0, p1i = c.f[1] + o1, p2i = c.f[2] + o2;
-	if(p0i > g.res[0] - 1 || p1i > g.res[1] - 1 || p2i > g.res[2] - 1) return false;
-	lin = uint32_t(p0i) + uint32_t(g.res[0]) * (uint32_t(p1i) + uint32_t(g.res[1]) * uint32_t(p2i));
+	// unsigned: a position 2^31 cells away has the largest int as its cell, whose upper corner would wrap to a
+	// negative one and pass for on-grid
+	const uint32_t p0i = uint32_t(c.f[0]) + o0, p1i = uint32_t(c.f[1]) + o1, p2i = uint32_t(c.f[2]) + o2;
+	if(p0i >= uint32_t(g.res[0]) || p1i >= uint32_t(g.res[1]) || p2i >= uint32_t(g.res[2])) return false;
+	lin = p0i + uint32_t(g.res[0]) * (p1i + uint32_t(g.res[1]) * p2i);
 	if(states[lin] == 0u) return false;
 	pp = v3(float(p0i) * g.cell[0] + g.emin[0], float(p1i) * g.cell[1] + g.emin[1], float(p2i) * g.cell[2] + g.emin[2]);
 	dtp = normalize_rn(pp - position);
@@ -665,6 +667,31 @@ __device__ __forceinline__ void cage_weight(const float2* __restrict__ dep, uint
 	fbw *= trw;
 }
 
+// What probe `lin` of a cage adds for one normal: its irradiance (square root space) times the weight, the
+// weight, and the same with the fallback weight.
+__device__ __forceinline__ void sample_corner(const float4* __restrict__ irr, const float2* __restrict__ dep, uint32_t lin,
+											  Vec3 pp, Vec3 dtp, float trw, Vec3 normal, Vec3 biased, uint32_t tap, float wx,
+											  float wy, float (&v)[8]) {
+	float weight, fbw;
+	cage_weight(dep, lin, pp, dtp, trw, normal, biased, weight, fbw);
+	const float4* ct = irr + size_t(lin) * 64 + tap;
+	const float4 c00 = ct[0], c10 = ct[1], c01 = ct[8], c11 = ct[9];
+	const float cr = (c00.x * (1.0f - wx) + c10.x * wx) * (1.0f - wy) + (c01.x * (1.0f - wx) + c11.x * wx) * wy;
+	const float cg = (c00.y * (1.0f - wx) + c10.y * wx) * (1.0f - wy) + (c01.y * (1.0f - wx) + c11.y * wx) * wy;
+	const float cb = (c00.z * (1.0f - wx) + c10.z * wx) * (1.0f - wy) + (c01.z * (1.0f - wx) + c11.z * wx) * wy;
+	Vec3 col;
+	if(fminf(fminf(cr, cg), cb) >= 1.26217745e-29f) col = v3(sqrt_rn(cr), sqrt_rn(cg), sqrt_rn(cb));
+	else col = v3(sqrtf(cr), sqrtf(cg), sqrtf(cb));  // 0, or too small for sqrt_rn's residuals (2^-96)
+	v[0] = col.x * weight;
+	v[1] = col.y * weight;
+	v[2] = col.z * weight;
+	v[3] = weight;
+	v[4] = col.x * fbw;
+	v[5] = col.y * fbw;
+	v[6] = col.z * fbw;
+	v[7] = fbw;
+}
+
 // sampleProbes (src/shaders/irradiance.glsl:145-237) on the tiled FP32 atlases, at one position for N
 // normals, which share each probe's index, state, direction and trilinear factor.  Bound by vector
 // instructions: 395 per probe and normal as separate calls with the compiler's divisions and square roots
@@ -699,21 +726,12 @@ __device__ __forceinline__ void sample_probes(const GridConst& g, const uint32_t
 		if(!cage_corner(g, states, cage, position, i, lin, pp, dtp, trw)) continue;
 #pragma unroll
 		for(int k = 0; k < N; ++k) {
-			float weight, fbw;
-			cage_weight(dep, lin, pp, dtp, trw, normal[k], biased[k], weight, fbw);
-			const float4* ct = irr + size_t(lin) * 64 + tap[k];
-			const float4 c00 = ct[0], c10 = ct[1], c01 = ct[8], c11 = ct[9];
-			const float wx = cwx[k], wy = cwy[k];
-			const float cr = (c00.x * (1.0f - wx) + c10.x * wx) * (1.0f - wy) + (c01.x * (1.0f - wx) + c11.x * wx) * wy;
-			const float cg = (c00.y * (1.0f - wx) + c10.y * wx) * (1.0f - wy) + (c01.y * (1.0f - wx) + c11.y * wx) * wy;
-			const float cb = (c00.z * (1.0f - wx) + c10.z * wx) * (1.0f - wy) + (c01.z * (1.0f - wx) + c11.z * wx) * wy;
-			Vec3 col;
-			if(fminf(fminf(cr, cg), cb) >= 1.26217745e-29f) col = v3(sqrt_rn(cr), sqrt_rn(cg), sqrt_rn(cb));
-			else col = v3(sqrtf(cr), sqrtf(cg), sqrtf(cb));  // 0, or too small for sqrt_rn's residuals (2^-96)
-			fin[k] = fin[k] + col * weight;
-			tw[k] += weight;
-			fb[k] = fb[k] + col * fbw;
-			tfb[k] += fbw;
+			float v[8];
+			sample_corner(irr, dep, lin, pp, dtp, trw, normal[k], biased[k], tap[k], cwx[k], cwy[k], v);
+			fin[k] = fin[k] + v3(v[0], v[1], v[2]);
+			tw[k] += v[3];
+			fb[k] = fb[k] + v3(v[4], v[5], v[6]);
+			tfb[k] += v[7];
 		}
 	}
 #pragma unroll
