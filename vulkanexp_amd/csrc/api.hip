@@ -350,11 +350,10 @@ void destroy_handle(Handle* h) {
 					h->miss_list, h->shade_keys, h->sort_keys, h->sort_list, h->sort_counts, h->fib,   h->perm,       h->fib512,
 					h->dirs,   h->wt,      h->inv_sum,    h->w_hi,        h->w_lo,       h->visit};
 	for(void* b : bufs) (void)hipFree(b);
-	for(auto& e : h->ev)
-		if(e) (void)hipEventDestroy(e);
 	if(h->move_done) (void)hipEventDestroy(h->move_done);
 	if(h->selected_ready) (void)hipEventDestroy(h->selected_ready);
-	if(h->selected) (void)hipHostFree(h->selected);
+	if(h->timed_end) (void)hipEventDestroy(h->timed_end);
+	if(h->stamps.host) (void)hipHostFree(h->stamps.host);
 	delete h;
 }
 
@@ -384,7 +383,7 @@ FrameBegin frame_begin(Handle* h, const Rot& R, uint16_t* order, uint32_t mode) 
 // Blends `rays` with the weights that launch_frame_begin has written for the same flags; `copied`: the next
 // atlas holds the exposed one already, or every tile of it is written.
 ddgi_status enqueue_blend_and_publish(Handle* h, const float4* rays, uint32_t max_slots, bool copied, uint32_t flags,
-									  hipStream_t s) {
+									  const PhaseStamps& stamps, hipStream_t s) {
 	const GridConst g = make_grid_const(*h);
 	const uint32_t mode = blend_mode(flags);
 	const int nxt = h->cur ^ 1;
@@ -408,6 +407,7 @@ ddgi_status enqueue_blend_and_publish(Handle* h, const float4* rays, uint32_t ma
 	b.irr_out = h->irr[nxt];
 	b.dep_out = h->dep[nxt];
 	b.max_slots = max_slots;
+	b.stamps = stamps;
 	HIP_TRY(h, launch_blend(b, mode, h->cus, s));
 	h->cur = nxt;  // publish (reference: vkCmdCopyImage work -> exposed, src/IrradianceProbes.cpp:530-576)
 	return DDGI_OK;
@@ -620,16 +620,20 @@ ddgi_status ddgi_create(const ddgi_grid_params* params, const ddgi_options* opti
 	if(e == hipSuccess) e = hipMemset(h->sel, 0, sizeof(SelectState));
 	if(e == hipSuccess) e = hipMemset(h->rays, 0, P * R * sizeof(float4));
 	if(e == hipSuccess) e = hipMemset(h->visit, 0, 8 * sizeof(unsigned long long));
+	if(e == hipSuccess) e = hipMemset(h->shade_count, 0, kListCounterBytes);
 	if(e == hipSuccess) {
 		std::vector<uint32_t> ones(P, 1u);
 		e = hipMemcpy(h->states, ones.data(), P * 4, hipMemcpyHostToDevice);
 	}
-	for(int i = 0; i < 5 && e == hipSuccess; ++i) e = hipEventCreate(&h->ev[i]);
+	if(e == hipSuccess) e = hipEventCreateWithFlags(&h->timed_end, hipEventDisableTiming);
+	if(e == hipSuccess) e = hipDeviceGetAttribute(&h->wall_khz, hipDeviceAttributeWallClockRate, h->device);
 	if(e == hipSuccess) e = hipEventCreateWithFlags(&h->selected_ready, hipEventDisableTiming);
 	if(e == hipSuccess) {
 		void* p = nullptr;
-		e = hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocDefault);
-		h->selected = static_cast<uint32_t*>(p);
+		e = hipHostMalloc(&p, 5 * sizeof(unsigned long long) + sizeof(uint32_t), hipHostMallocDefault);
+		h->stamps.host = static_cast<unsigned long long*>(p);
+		h->stamps.done = h->shade_count + kBlendDoneSlot;
+		h->selected = p ? reinterpret_cast<uint32_t*>(h->stamps.host + 5) : nullptr;
 	}
 	if(e != hipSuccess) {
 		h->err = std::string("initialisation failed: ") + hipGetErrorString(e);
@@ -948,10 +952,11 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	ddgi_status st = DDGI_OK;
 	const bool timing = !(flags & DDGI_UPDATE_NO_TIMING);
 	const bool all = (flags & DDGI_UPDATE_ALL_PROBES) != 0;
-	if(timing) HIP_TRY(h, hipEventRecord(h->ev[0], s));
+	const PhaseStamps stamps = timing ? h->stamps : PhaseStamps{};
 	uint32_t max_slots = h->P;
 	FrameBegin begin = frame_begin(h, R, h->perm, blend_mode(flags));
 	begin.counters = h->shade_count;
+	begin.stamp = stamps.host;
 	begin.count = h->P;
 	if(all) {
 		begin.list = h->indices_are_iota ? kListKeep : kListIota;
@@ -974,9 +979,7 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	}
 	HIP_TRY(h, launch_frame_begin(begin, s));
 	h->indices_are_iota = all;
-	if(timing) HIP_TRY(h, hipEventRecord(h->ev[1], s));
-	const hipEvent_t counted = timing ? h->ev[1] : h->selected_ready;
-	if(late_count && !timing) HIP_TRY(h, hipEventRecord(counted, s));
+	if(late_count) HIP_TRY(h, hipEventRecord(h->selected_ready, s));
 	const GridConst g = make_grid_const(*h);
 	uint32_t key_shift = 0, key_bits = 0;  // shade-list ordering keys
 	shade_key_layout(g, &key_shift, &key_bits);
@@ -999,6 +1002,7 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	a.max_slots = max_slots;
 	a.visit_counters = nullptr;
 	a.factors = factors;
+	a.stamps = stamps.host;
 	if(flags & DDGI_UPDATE_COUNT_VISITS) {
 		HIP_TRY(h, hipMemsetAsync(h->visit, 0, 8 * sizeof(unsigned long long), s));
 		a.visit_counters = h->visit;
@@ -1010,11 +1014,10 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 		a.seg_cap = (blocks + kShadeSegments - 1) / kShadeSegments * kPrimaryBlock;
 	}
 	HIP_TRY(h, launch_trace_primary(a, s));
-	if(timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
 	if(a.shade_keys)  // shade the front-face hits ordered by the grid cell they lie in
 		HIP_TRY(h, launch_key_sort(SortJob{h->shade_keys, h->shade_list, h->shade_count, h->sort_counts, h->sort_keys,
 										   h->sort_list, h->shade_count + kShadeTotalSlot, 0u, kShadeSegments, a.seg_cap, 0u},
-								   uint64_t(max_slots) * g.n, 3 * key_bits, s));
+								   uint64_t(max_slots) * g.n, 3 * key_bits, s, stamps.host ? stamps.host + 2 : nullptr));
 	const bool beside = !all && h->P < (1u << 24);
 	if(beside) {  // probes that are not updated keep their tiles: the next atlas starts as a copy, made beside the shading
 		const int nxt = h->cur ^ 1;
@@ -1027,12 +1030,11 @@ static ddgi_status run_update(Handle* h, const Rot& R, uint32_t flags, hipStream
 	}
 	HIP_TRY(h, launch_shade(a, s));
 	if(h->light.sky_model == DDGI_SKY_ATMOSPHERE) HIP_TRY(h, launch_sky(a, s));
-	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
-	if(late_count) HIP_TRY(h, hipEventSynchronize(counted));
+	if(late_count) HIP_TRY(h, hipEventSynchronize(h->selected_ready));
 	if(ramp) advance_hysteresis(h, all ? h->P : *h->selected);
-	if((st = enqueue_blend_and_publish(h, h->rays, max_slots, all || beside, flags, s)) != DDGI_OK) return st;
+	if((st = enqueue_blend_and_publish(h, h->rays, max_slots, all || beside, flags, stamps, s)) != DDGI_OK) return st;
 	if(timing) {
-		HIP_TRY(h, hipEventRecord(h->ev[4], s));
+		HIP_TRY(h, hipEventRecord(h->timed_end, s));
 		h->timing_pending = true;
 		h->timing_from = 0;
 	}
@@ -1055,19 +1057,20 @@ ddgi_status ddgi_blend_rays(void* handle, const void* rays, const void* probe_in
 	if(st != DDGI_OK || (st = ensure_fib(h)) != DDGI_OK) return st;
 	hipStream_t s = static_cast<hipStream_t>(stream);
 	const bool timing = !(flags & DDGI_UPDATE_NO_TIMING);
-	if(timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
+	const PhaseStamps stamps = timing ? h->stamps : PhaseStamps{};
 	FrameBegin begin = frame_begin(h, R, nullptr, blend_mode(flags));
 	begin.list = kListCopy;
 	begin.listed = static_cast<const uint32_t*>(probe_indices);
 	begin.count = count;
+	begin.stamp = stamps.host;
 	HIP_TRY(h, launch_frame_begin(begin, s));
 	h->indices_are_iota = false;
 	// the listed probes may not cover the grid: the next atlas starts as a copy of the exposed one,
 	// unless the caller states that they are every probe
 	const bool all = (flags & DDGI_UPDATE_ALL_PROBES) && count == h->P;
-	if((st = enqueue_blend_and_publish(h, static_cast<const float4*>(rays), count, all, flags, s)) != DDGI_OK) return st;
+	if((st = enqueue_blend_and_publish(h, static_cast<const float4*>(rays), count, all, flags, stamps, s)) != DDGI_OK) return st;
 	if(timing) {
-		HIP_TRY(h, hipEventRecord(h->ev[4], s));
+		HIP_TRY(h, hipEventRecord(h->timed_end, s));
 		h->timing_pending = true;
 		h->timing_from = 3;
 	}
@@ -1528,9 +1531,14 @@ ddgi_status ddgi_get_timings(void* handle, ddgi_timings* out) {
 	ddgi_status st = set_device(h);
 	if(st != DDGI_OK) return st;
 	if(h->timing_pending) {
-		HIP_TRY(h, hipEventSynchronize(h->ev[4]));
+		HIP_TRY(h, hipEventSynchronize(h->timed_end));
 		float ms[4] = {};
-		for(int i = h->timing_from; i < 4; ++i) HIP_TRY(h, hipEventElapsedTime(&ms[i], h->ev[i], h->ev[i + 1]));
+		const unsigned long long* at = h->stamps.host;
+		auto ticks_ms = [&](int from, int to) { return at[to] > at[from] ? float(double(at[to] - at[from]) / h->wall_khz) : 0.0f; };
+		if(h->timing_from == 0)
+			for(int i = 0; i < 4; ++i) ms[i] = ticks_ms(i, i + 1);
+		else
+			ms[3] = ticks_ms(0, 4);  // a blend alone, its start included
 		h->last.select_ms = ms[0];
 		h->last.primary_ms = ms[1];
 		h->last.shade_ms = ms[2];
@@ -1538,7 +1546,7 @@ ddgi_status ddgi_get_timings(void* handle, ddgi_timings* out) {
 		h->last.blend_ms = ms[3];
 		h->last.border_ms = 0.0f;
 		h->last.copy_ms = 0.0f;
-		HIP_TRY(h, hipEventElapsedTime(&h->last.total_ms, h->ev[h->timing_from], h->ev[4]));
+		h->last.total_ms = ticks_ms(0, 4);
 		uint32_t cnt = h->last_count;
 		if(cnt == 0xFFFFFFFFu) {
 			SelectState ss;

@@ -172,12 +172,27 @@ __device__ __forceinline__ float4 frame_dir_unfused(const Rot& R, const float4& 
 	return make_float4(d[0], d[1], d[2], 0.0f);
 }
 
+// Phase stamps of a blend kernel: its start from the first workgroup, the end of the update from the last
+// one to finish.
+__device__ __forceinline__ void stamp_start(const PhaseStamps& p) {
+	if(p.host && blockIdx.x == 0 && threadIdx.x == 0) p.host[3] = wall_clock64();
+}
+__device__ __forceinline__ void stamp_end(const PhaseStamps& p) {
+	if(!p.host) return;  // uniform
+	__syncthreads();
+	if(threadIdx.x == 0 && atomicAdd(p.done, 1u) == gridDim.x - 1u) {
+		*p.done = 0u;
+		p.host[4] = wall_clock64();
+	}
+}
+
 __global__ __launch_bounds__(kBeginThreads) void k_frame_begin(FrameBegin a) {
 	__shared__ __attribute__((aligned(16))) float s_key[kMaxRays];
 	__shared__ uint32_t s_rank[kMaxRays];
 	__shared__ float4 s_dir[kMaxRays];  // in thread order
 	__shared__ float s_red[kBeginThreads];
 	const uint32_t t = threadIdx.x, n = a.grid.n;
+	if(a.stamp && blockIdx.x == 0 && t == 0) *a.stamp = wall_clock64();
 	if(blockIdx.x == kWRows / kBeginRows) {  // only launched for kListSelect
 		select_probes(a.states, a.probe_count, a.count, a.sel, a.indices);
 		if(a.host_count && t == 0) *a.host_count = a.sel->count;  // thread 0 stored it
@@ -547,7 +562,9 @@ __device__ __forceinline__ void blend_fp32_tile(const BlendArgs& a, uint32_t slo
 
 // 4 waves/SIMD: the 4 blocks of a CU that a 16-probe tiling of a large grid needs stay resident
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_blend_fp32(BlendArgs a, uint32_t n_pad) {
+	stamp_start(a.stamps);
 	blend_fp32_tile<kProbesPerBlock>(a, blockIdx.x * kProbesPerBlock, n_pad);
+	stamp_end(a.stamps);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -937,7 +954,9 @@ __device__ __forceinline__ void blend_mfma_wide(const BlendArgs& a, uint32_t slo
 template <uint32_t MODE, int STEPS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_blend_wide(BlendArgs a) {
 	DDGI_WIDE_LDS;
+	stamp_start(a.stamps);
 	blend_mfma_wide<MODE, STEPS>(a, blockIdx.x * kWideProbes, lds);
+	stamp_end(a.stamps);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1145,7 +1164,9 @@ template <uint32_t MODE>
 __global__ __launch_bounds__(kTileThreads) void k_blend_tile(BlendArgs a, uint32_t n_pad) {
 	__shared__ __attribute__((aligned(16))) unsigned char smem[kTileLdsBytes];
 	__shared__ uint32_t s_small[3 * kTileProbes];
+	stamp_start(a.stamps);
 	blend_wave_tile<MODE>(a, blockIdx.x * kTileProbes, n_pad, smem, s_small);
+	stamp_end(a.stamps);
 }
 
 // ---- batched update ----

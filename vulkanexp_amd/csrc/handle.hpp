@@ -82,9 +82,11 @@ struct Handle {
 	bool move_pending = false;
 	LightConst light{};
 	// timing
-	hipEvent_t ev[5] = {};  // start, list and weights ready, primary rays, shading, end
+	PhaseStamps stamps{};          // of the last timed update or blend
+	int wall_khz = 0;              // ticks of the stamps per ms
+	hipEvent_t timed_end = nullptr;
 	bool timing_pending = false;
-	int timing_from = 0;           // first event of the pending timings (3: a blend alone)
+	int timing_from = 0;           // first stamp of the pending timings (3: a blend alone)
 	uint32_t* selected = nullptr;  // pinned: probes of the last partial update under the ramp
 	hipEvent_t selected_ready = nullptr;
 	ddgi_timings last{};

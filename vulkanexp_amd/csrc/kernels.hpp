@@ -108,13 +108,23 @@ constexpr uint32_t kShadeSegments = 8;
 constexpr uint32_t kCounterStride = 32;
 constexpr uint32_t kMissCountSlot = kCounterStride * kShadeSegments;
 constexpr uint32_t kShadeTotalSlot = kMissCountSlot + kCounterStride;
-constexpr uint32_t kListCounterBytes = (kShadeTotalSlot + kCounterStride) * 4;
+constexpr uint32_t kBlendDoneSlot = kShadeTotalSlot + kCounterStride;  // PhaseStamps::done
+constexpr uint32_t kListCounterBytes = (kBlendDoneSlot + kCounterStride) * 4;
 // An update orders its shade list from this many rays (slots x rays per probe) up.  The ordering's four
 // launches cost 25 to 60 us; it shortens the shading by less than that while the hits' probe tiles and BVH
 // nodes fit the caches anyway.  Whole update without / with the ordering, us, instances of the scene 24, 80, 256:
 //   rays   32768                        524288                       1048576                      2097152
 //          122 / 145 144 / 170 168 / 192  186 / 213 228 / 245 266 / 285  245 / 250 324 / 300 385 / 372  391 / 358 550 / 477 689 / 591
 constexpr uint64_t kShadeSortRays = 640u * 1024u;
+
+// Phase times of an update, in ticks of the device's wall clock, in pinned host memory: [0] the start, then
+// the starts of [1] tracing, [2] ordering or shading, [3] the blend, and [4] the end, written by the blend's
+// last workgroup (`done`: device counter, 0 between launches).  Each kernel's first workgroup stores its
+// own start: an event record between two kernels holds the second back for 4 us, and there were four.
+struct PhaseStamps {
+	unsigned long long* host;  // null: no stamps
+	uint32_t* done;
+};
 
 struct TraceFrameArgs {
 	SceneDev scene;
@@ -151,6 +161,7 @@ struct TraceFrameArgs {
 	float4* copy_dst[2];
 	uint32_t copy_n[2];
 	uint32_t shade_blocks;  // set by launch_shade
+	unsigned long long* stamps;  // optional: PhaseStamps::host
 };
 constexpr uint32_t kShadeSortCounts = 1024 * 128 + 1024;  // (list tile, coarse digit) counters + digit totals
 
@@ -177,6 +188,7 @@ struct BlendArgs {
 	float2* dep_out;
 	uint32_t max_slots;
 	uint32_t flags;             // kBlendIrradianceOnly: no depth stores, no state update
+	PhaseStamps stamps;         // optional
 };
 constexpr uint32_t kBlendIrradianceOnly = 0x1;
 
@@ -255,6 +267,7 @@ struct SortJobs {
 	SortJob one;
 	const char* many;
 	uint32_t stride;
+	unsigned long long* stamp;  // optional: receives the start (PhaseStamps)
 	const BatchItem* chunks;  // (job, chunk of kFineChunk entries) per workgroup of a batch's last pass
 };
 uint32_t sort_fine_bits(uint32_t key_bits);
@@ -267,7 +280,7 @@ hipError_t launch_frame_dirs(const Rot& R, const float4* fib, float4* dirs, uint
 // than a chunk is ordered chunk by chunk); entries with equal keys come in any order.  Scratch:
 // job.counts (kShadeSortCounts), job.bucket_keys and job.bucket_list (capacity each).  The
 // caller's job.fine_bits is ignored (set from key_bits).
-hipError_t launch_key_sort(SortJob job, uint64_t capacity, uint32_t key_bits, hipStream_t s);
+hipError_t launch_key_sort(SortJob job, uint64_t capacity, uint32_t key_bits, hipStream_t s, unsigned long long* stamp = nullptr);
 // Cell-key layout of the shade ordering for a grid: coordinate shift and bits per axis.
 void shade_key_layout(const GridConst& g, uint32_t* shift, uint32_t* bits_per_axis);
 hipError_t launch_clear(uint32_t* words, uint32_t n, hipStream_t s);
@@ -325,6 +338,7 @@ struct FrameBegin {
 	uint32_t count;
 	uint32_t probe_count;
 	uint32_t n_pad;          // set by the launcher
+	unsigned long long* stamp;  // optional: receives the start (PhaseStamps)
 	uint32_t* host_count;    // optional with kListSelect: pinned host memory that receives the count
 };
 hipError_t launch_frame_begin(FrameBegin a, hipStream_t s);

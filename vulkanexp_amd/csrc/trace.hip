@@ -161,6 +161,7 @@ template <int STACK, bool COUNT>
 // eight waves per SIMD (64 VGPRs, no spills): 0.559 ms, against 0.580 at 7 and 0.617 at 6
 __global__ __launch_bounds__(kPrimaryBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_primary(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kPrimaryBlock];
+	if(a.stamps && blockIdx.x == 0 && threadIdx.x == 0) a.stamps[1] = wall_clock64();
 	trace_primary_ray<STACK, kPrimaryBlock, COUNT>(a, xcd_remap(blockIdx.x, gridDim.x) * kPrimaryBlock + threadIdx.x,
 												   stack + threadIdx.x, blockIdx.x % kShadeSegments);
 }
@@ -337,6 +338,7 @@ __global__ __launch_bounds__(1024) void k_sort_count(SortJobs J) {
 	uint32_t* __restrict__ counts = j.counts;
 	__shared__ uint32_t s_cnt[kSortDigits];
 	const uint32_t t = threadIdx.x;
+	if(J.stamp && blockIdx.x == 0 && t == 0) *J.stamp = wall_clock64();
 	s_cnt[t] = 0u;
 	__syncthreads();
 	size_t base;
@@ -546,6 +548,7 @@ __device__ __forceinline__ void copy_block(const TraceFrameArgs& a, uint32_t b) 
 template <int STACK, bool COUNT>
 __global__ __launch_bounds__(kShadeBlock, 4) void k_shade(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kShadeBlock];
+	if(a.stamps && !a.shade_keys && blockIdx.x == 0 && threadIdx.x == 0) a.stamps[2] = wall_clock64();
 	if(blockIdx.x >= a.shade_blocks) {
 		copy_block(a, blockIdx.x - a.shade_blocks);
 		return;
@@ -1359,13 +1362,14 @@ static hipError_t launch_sort_jobs(const SortJobs& J, uint32_t jobs, uint32_t ch
 
 uint32_t sort_fine_bits(uint32_t key_bits) { return key_bits > kSortCoarseBits ? key_bits - kSortCoarseBits : 0u; }
 
-hipError_t launch_key_sort(SortJob job, uint64_t capacity, uint32_t key_bits, hipStream_t s) {
+hipError_t launch_key_sort(SortJob job, uint64_t capacity, uint32_t key_bits, hipStream_t s, unsigned long long* stamp) {
 	if(key_bits > kSortCoarseBits + 8u || capacity > 0xFFFFFFFFull || job.segments == 0 ||
 	   job.segments > kShadeSegments || kSortTiles % job.segments != 0)
 		return hipErrorInvalidValue;
 	job.fine_bits = sort_fine_bits(key_bits);
 	SortJobs J{};
 	J.one = job;
+	J.stamp = stamp;
 	return launch_sort_jobs(J, 1, uint32_t((capacity + kFineChunk - 1) / kFineChunk), s);
 }
 
