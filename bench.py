@@ -6,8 +6,8 @@ updated every step.  A step is one full update: trace (primary rays + shading + 
 irradiance/depth blend with hysteresis + border copy (fused) + publish.
 
 Prints ONE JSON line (rank 0).  `value` = primary probe rays per second of whole updates, in
-Mrays/s, over `--steps` updates enqueued back to back (no timing events, no host wait between
-them); `phases_ms` come from a second pass over the same updates with per-phase HIP events.
+Mrays/s, over `--steps` updates enqueued back to back (no timings, no host wait between
+them); `phases_ms` come from a second pass over the same updates with timings on.
 `roofline` describes the kernel with the largest share of the step: its algorithmic bytes come from
 the traversal's own fetch counters (80-byte 4-wide nodes, 48-byte triangles) of an untimed
 counting update, set against the HBM peak; `traffic` (bytes leaving L2 per launch, from the
@@ -536,11 +536,11 @@ def main():
     wall = time.perf_counter() - t0
     ms_per_step = wall / args.steps * 1e3
     value = P * n / (ms_per_step * 1e-3) / 1e6
-    # per-phase HIP-event times of the same updates, in a separate untimed pass
+    # per-phase times of the same updates, in a separate untimed pass
     phase = {"select_ms": [], "primary_ms": [], "shade_ms": [], "blend_ms": [], "total_ms": []}
     for k in range(args.steps):
         probes.update(Rs[1 + args.warmup + k], flags, stream)
-        tm = probes.timings()  # waits for this update's events
+        tm = probes.timings()  # waits for this update
         for key in phase:
             phase[key].append(tm[key])
     torch.cuda.synchronize()

@@ -120,7 +120,7 @@ typedef struct ddgi_options {
 #define DDGI_UPDATE_BLEND_BF16 0x2u       /* blend on BF16 MFMA (hi/lo compensated), FP32 accumulation */
 #define DDGI_UPDATE_BLEND_FP16 0x4u       /* blend on FP16 MFMA, FP32 accumulation */
 #define DDGI_UPDATE_HYSTERESIS_RAMP 0x8u  /* reference hysteresis ramp (src/IrradianceProbes.cpp:462-476) */
-#define DDGI_UPDATE_NO_TIMING 0x10u       /* skip per-phase HIP events */
+#define DDGI_UPDATE_NO_TIMING 0x10u       /* skip the per-phase timings */
 #define DDGI_UPDATE_COUNT_VISITS 0x20u    /* count BVH node/triangle fetches (slower; statistics) */
 
 /* Atlas kinds / layouts */
@@ -167,7 +167,9 @@ typedef struct ddgi_gbuffer_texel {
 } ddgi_gbuffer_texel;
 
 /* Per-phase GPU times of the last completed update, in milliseconds (the reference's timestamp
- * split, src/IrradianceProbes.cpp:441-452). */
+ * split, src/IrradianceProbes.cpp:441-452): the times between the starts of the phases' first kernels,
+ * stored by the kernels themselves.  select_ms covers the probe list, the ray directions and the blend
+ * weights; of ddgi_blend_rays everything is blend_ms. */
 typedef struct ddgi_timings {
 	float select_ms;
 	float trace_ms;   /* primary traversal + shading + shadow rays */
