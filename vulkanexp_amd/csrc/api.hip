@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "handle.hpp"
+#include "packed_node.hpp"
 
 using namespace ddgi;
 
@@ -246,7 +247,7 @@ bool instance_dev(const ddgi_instance& in, const float* M, uint32_t prim_base, I
 }
 
 // The triangle slots (first, end) under every child of the wide tree's nodes, 4 per node (an empty child:
-// first >= end), and the nodes' child codes.  The slots are in the tree's leaf order, so a range holds
+// first >= end), and the packed nodes' child codes.  The slots are in the tree's leaf order, so a range holds
 // exactly its subtree's.
 void node_ranges(const BvhHost& bvh, std::vector<uint32_t>& range, std::vector<uint32_t>& codes) {
 	range.assign(size_t(bvh.node_count) * 8, 0u);
@@ -256,7 +257,7 @@ void node_ranges(const BvhHost& bvh, std::vector<uint32_t>& range, std::vector<u
 		for(uint32_t k = 0; k < kWide; ++k) {
 			uint32_t code;
 			std::memcpy(&code, &bvh.nodes[w * kNodeFloats + kCodeRow + k], 4);
-			codes[w * 4 + k] = code;
+			codes[w * 4 + k] = packed_code(code);
 			uint32_t first = 0xFFFFFFFFu, end = 0;
 			if(code == kEmptyChild) {
 				first = end = 0;

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "device_common.hpp"
+#include "packed_node.hpp"
 
 namespace ddgi {
 
@@ -1137,8 +1138,8 @@ __global__ void k_apply_moves(const InstanceMove* __restrict__ staged, InstanceM
 // boxes tight enough that no more nodes are visited).  A plane is origin + q * scale; the traversal's
 // distance fma(q, scale / d, (origin - o) / d) is off by at most about 2.4e-7 of the node's size (in
 // position) beside the errors relative to the distance that the far end's widening covers, so the padded
-// boxes are first grown by 1e-6 of that size.  An empty child gets an inverted box, which no ray enters; a
-// node too large for the grid gets infinite ones.
+// boxes are first grown by 1e-6 of that size.  A node too large
+// for the grid gets infinite boxes (node_grid and child_planes).
 // 32 lanes per node, eight per child: `range` holds each child's triangle slots (first, end), and lane j of
 // a child takes the j-th box of either end of its range on every level.
 __global__ __launch_bounds__(256) void k_make_nodes(BoxTree tree, const uint2* __restrict__ range,
@@ -1179,33 +1180,12 @@ __global__ __launch_bounds__(256) void k_make_nodes(BoxTree tree, const uint2* _
 		mx[a] = double(h);
 		size = fmax(size, mx[a] - mn[a]);
 	}
-	const double slack = size * 1e-6;
-	float org[3];
-	double ext = 0.0;
-#pragma unroll
-	for(int a = 0; a < 3; ++a) {
-		org[a] = float(mn[a] - slack);
-		if(double(org[a]) > mn[a] - slack) org[a] = nextafterf(org[a], -__int_as_float(0x7f800000));
-		ext = fmax(ext, mx[a] + slack - double(org[a]));
-	}
-	const bool fits = ext < 1e37;  // false for infinite extents too
-	// the smallest power of two with 2047 steps over the extent
-	uint32_t sb = __float_as_uint(float(ext * (1.000001 / 2047.0)));
-	sb = (sb + 0x007FFFFFu) & 0x7F800000u;
-	const float scale = fits ? __uint_as_float(sb) : 1.0f;
-	const double inv = 1.0 / double(scale);
+	const NodeGrid grid = node_grid(mn, mx, size);
 	float4* dst = reinterpret_cast<float4*>(reinterpret_cast<char*>(packed) + size_t(node) * kPackedNodeBytes);
 	const uint32_t base = lane & 32u;  // the node's first lane
 #pragma unroll
 	for(int a = 0; a < 3; ++a) {
-		const double l = floor((double(b.lo[a]) - slack - double(org[a])) * inv);
-		const double h = ceil((double(b.hi[a]) + slack - double(org[a])) * inv);
-		// FP16 bits: the integers, 65504 / -65504 for an empty child, -inf / inf beyond the grid
-		const auto bits = [](double q) {
-			return uint32_t(__builtin_bit_cast(unsigned short, _Float16(float(fmin(fmax(q, 0.0), 2047.0)))));
-		};
-		const uint32_t ql = empty ? 0x7BFFu : (fits ? bits(l) : 0xFC00u), qh = empty ? 0xFBFFu : (fits ? bits(h) : 0x7C00u);
-		const int q = int(ql | (qh << 16));
+		const int q = int(child_planes(grid, a, b.lo[a], b.hi[a], empty));
 		uint32_t c[4];
 #pragma unroll
 		for(int k = 0; k < 4; ++k) c[k] = uint32_t(__shfl(q, int(base) + 8 * k));
@@ -1214,7 +1194,7 @@ __global__ __launch_bounds__(256) void k_make_nodes(BoxTree tree, const uint2* _
 									 __uint_as_float((c[0] >> 16) | (c[1] & 0xFFFF0000u)),
 									 __uint_as_float((c[2] >> 16) | (c[3] & 0xFFFF0000u)));
 	}
-	if((lane & 31u) == 3u) dst[0] = fits ? make_float4(org[0], org[1], org[2], scale) : make_float4(0.0f, 0.0f, 0.0f, 1.0f);
+	if((lane & 31u) == 3u) dst[0] = make_float4(grid.org[0], grid.org[1], grid.org[2], grid.scale);
 	if((lane & 31u) == 4u) {
 		const uint4 c = codes[node];
 		dst[4] = make_float4(__uint_as_float(c.x), __uint_as_float(c.y), __uint_as_float(c.z), __uint_as_float(c.w));
