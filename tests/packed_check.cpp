@@ -4,6 +4,9 @@
 // packed nodes and through the builder's FP32 boxes, with the kernels' FP32 box tests and one
 // double-precision triangle test.  MODE says how the rays run:
 //   generic  uniform directions
+//   axis     along a coordinate axis, the other components +-0
+//   plane    one component +-0
+//   tiny     along a coordinate axis, the others of magnitude 1e-44 .. 1e-25
 //   far      from REACH away (and above) toward the scene's triangles
 // from origins inside the scene's bounds (not farther than REACH from 0) unless far.
 // Prints: rays hits mismatches-to-every-triangle packed-visits fp32-visits most-packed-visits
@@ -166,6 +169,7 @@ double trace(const BvhHost& b, const std::vector<Packed>* packed, const Ray& r, 
 	constexpr uint32_t kNone = 0xFFFFFFFFu;
 	float inv[3];
 	for(int a = 0; a < 3; ++a) inv[a] = 1.0f / r.d[a];
+	if(packed) slab_reciprocals(r.o, (*packed)[0].header, inv);
 	std::vector<uint32_t> stack{kNone, 0u};
 	double best = 1e30;
 	for(;;) {
@@ -229,12 +233,16 @@ int main(int argc, char** argv) {
 			const double lo = std::max<double>(T.bounds_min[a], -reach), hi = std::min<double>(T.bounds_max[a], reach);
 			r.o[a] = float(lo + (hi - lo) * U(rng));
 		}
+		const int axis = int(U(rng) * 3.0);
 		const double z = 2.0 * U(rng) - 1.0, ph = 2.0 * M_PI * U(rng), s = std::sqrt(1.0 - z * z);
 		const double d[3] = {std::cos(ph) * s, std::sin(ph) * s, z};
 		const float* at = &b.tris[size_t(U(rng) * b.tri_count) * 12];
 		for(int a = 0; a < 3; ++a) {
-			const double e = U(rng);
+			const double sign = U(rng) < 0.5 ? -1.0 : 1.0, e = U(rng);
 			r.d[a] = float(d[a]);
+			if(mode == "axis") r.d[a] = float(sign * (a == axis ? 1.0 : 0.0));
+			if(mode == "plane" && a == axis) r.d[a] = float(sign * 0.0);
+			if(mode == "tiny") r.d[a] = float(sign * (a == axis ? 1.0 : std::pow(10.0, -44.0 + 19.0 * e)));
 			// toward the triangle, within a tenth of the distance by which the box test widens a box's exit
 			if(mode == "far") {
 				const double to = at[a] + 1e-7 * reach * (2.0 * e - 1.0);

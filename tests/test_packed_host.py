@@ -1,6 +1,9 @@
 """The traversal's packed box test on the CPU: tests/packed_check.cpp packs a scene's nodes with the code of
 vulkanexp_amd/csrc/packed_node.hpp and traces rays through them with the kernels' FP32 operations.  Every
-ray finds the nearest of all triangles."""
+ray finds the nearest of all triangles, and it visits about as many nodes as with FP32 boxes: a plane is
+rounded outward by at most one step of a 1024th of the node's extent, so a quarter more visits is a generous
+bound (a box test that an axis no longer takes part in costs a multiple)."""
+import dataclasses
 import os
 import subprocess
 
@@ -23,6 +26,37 @@ def checker(tmp_path_factory):
     return out
 
 
+def _scaled(scene, scale):
+    v = scene.vertices.copy()
+    v["pos"] = (v["pos"].astype(np.float64) * scale).astype(np.float32)
+    return dataclasses.replace(scene, vertices=v)
+
+
+def _beyond():
+    """A room's boxes under a triangle too large for a node's grid."""
+    sb = scenes.SceneBuilder()
+    rng = np.random.Generator(np.random.PCG64(3))
+    m = sb.add_material((0.5, 0.5, 0.5))
+    for _ in range(40):
+        lo = rng.uniform(0.0, 10.0, 3)
+        p, n, t = scenes.box_mesh(lo, lo + rng.uniform(0.01, 2.0, 3))
+        sb.add_instance(sb.add_mesh(p, n, t, m))
+    p = np.array([[-2e37, 11.0, -2e37], [2e37, 11.0, -2e37], [0.0, 11.0, 2e37]], np.float32)
+    sb.add_instance(sb.add_mesh(p, np.tile(np.float32([0, -1, 0]), (3, 1)), np.array([[0, 1, 2]]), m))
+    return sb.build((0, 0, 0), (12, 12, 12))
+
+
+SCENES = {
+    "room": lambda: scenes.config_small(seed=1)[0],
+    "clustered": lambda: scenes.clustered_scene(seed=5, n_instances=24),
+    "room_1e-3": lambda: _scaled(scenes.config_small(seed=1)[0], 1e-3),
+    "room_1e6": lambda: _scaled(scenes.config_small(seed=1)[0], 1e6),
+    "room_1e14": lambda: _scaled(scenes.config_small(seed=1)[0], 1e14),
+    "room_beyond": _beyond,
+    "room_1e19": lambda: _scaled(scenes.config_small(seed=1)[0], 1e19),
+}
+
+
 def _trace(checker, tmp_path, scene, mode, rays, reach=1e30):
     path = str(tmp_path / "s.scene")
     scenes.save(scene, path)
@@ -31,6 +65,17 @@ def _trace(checker, tmp_path, scene, mode, rays, reach=1e30):
     print(mode, r.stdout.strip())
     n, hits, bad, packed, fp32, most = r.stdout.split()
     return int(n), int(hits), int(bad), float(packed), float(fp32), int(most)
+
+
+@pytest.mark.parametrize("mode", ["generic", "axis", "plane", "tiny"])
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_directions_with_components_near_zero(checker, tmp_path, name, mode):
+    n, hits, bad, packed, fp32, most = _trace(checker, tmp_path, SCENES[name](), mode, 400 if name == "clustered" else 2000,
+                                                12.0 if name == "room_beyond" else 1e30)
+    assert hits > 0.1 * n
+    assert bad == 0
+    if name not in ("room_1e19", "room_beyond"):  # too large for bounded reciprocals: boxes are kept, and hits
+        assert packed <= 1.25 * fp32
 
 
 def _details(size):

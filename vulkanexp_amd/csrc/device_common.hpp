@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "kernels.hpp"
+#include "packed_node.hpp"
 
 namespace ddgi {
 
@@ -20,7 +21,7 @@ struct RayPrep {
 	float o[3];
 	int kx, ky, kz;
 	float sx, sy, sz;
-	float inv[3];  // 1/d for the slab tests
+	float inv[3];  // 1/d
 	float okx, oky, okz;
 };
 
@@ -131,8 +132,8 @@ struct HitResult {
 // plane (distance = q * (scale / d) + (origin - o) / d), and two loads fewer are returned.  The near and
 // far plane rows are chosen by the sign of 1/d (which is the smaller distance, since the distance is
 // monotonic in the plane), so no min / max pair is needed, and the far end is widened by a few ulps
-// (robust traversal, Ize 2013).  With d = +-0 the distances are infinite or NaN; maxima and minima drop
-// the NaNs, so such a box is kept.
+// (robust traversal, Ize 2013).  A plane's two terms must be finite for that: the reciprocals of zero and
+// very small direction components are bounded per ray (slab_reciprocals), which the triangle tests are not.
 //
 // For the closest hit the children the ray enters are sorted by entry distance (a five-comparator network on registers;
 // sorting only the nearest, or leaving the middle pair, visits more and took 0.64 / 0.66 ms against
@@ -222,8 +223,12 @@ __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, 
 	uint32_t leaf = kNone;
 	uint32_t n_nodes = 0, n_tris = 0;
 	const float kInf = __int_as_float(0x7f800000);
-	const bool neg[3] = {(__float_as_uint(r.inv[0]) >> 31) != 0u, (__float_as_uint(r.inv[1]) >> 31) != 0u,
-						 (__float_as_uint(r.inv[2]) >> 31) != 0u};
+	const float4 root = nodes[0];
+	const float header[4] = {root.x, root.y, root.z, root.w};
+	float inv[3] = {r.inv[0], r.inv[1], r.inv[2]};
+	slab_reciprocals(r.o, header, inv);
+	const bool neg[3] = {(__float_as_uint(inv[0]) >> 31) != 0u, (__float_as_uint(inv[1]) >> 31) != 0u,
+						 (__float_as_uint(inv[2]) >> 31) != 0u};
 	const char* __restrict__ node_bytes = reinterpret_cast<const char*>(nodes);
 	typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 	for(;;) {
@@ -239,7 +244,7 @@ __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, 
 			for(int ax = 0; ax < 3; ++ax) {
 				const float4 pl = ax == 0 ? px : (ax == 1 ? py : pz);
 				const float org = ax == 0 ? h.x : (ax == 1 ? h.y : h.z);
-				const float A = h.w * r.inv[ax], B = (org - r.o[ax]) * r.inv[ax];
+				const float A = h.w * inv[ax], B = (org - r.o[ax]) * inv[ax];
 				const uint32_t n01 = __float_as_uint(neg[ax] ? pl.z : pl.x), n23 = __float_as_uint(neg[ax] ? pl.w : pl.y);
 				const uint32_t f01 = __float_as_uint(neg[ax] ? pl.x : pl.z), f23 = __float_as_uint(neg[ax] ? pl.y : pl.w);
 				const half2_t qn[2] = {__builtin_bit_cast(half2_t, n01), __builtin_bit_cast(half2_t, n23)};

@@ -1,6 +1,6 @@
 // The arithmetic of the traversal's packed nodes that decides whether a box test is conservative: the grid
-// of a node and the planes on it.  Shared by the kernels (k_make_nodes) and by host
-// programs, with the same FP32 and FP64 operations (no contraction) on both.
+// of a node, the planes on it and a ray's reciprocals.  Shared by the kernels (k_make_nodes, traverse) and
+// by host programs, with the same FP32 and FP64 operations (no contraction) on both.
 #pragma once
 
 #include <cmath>
@@ -22,7 +22,8 @@ constexpr uint32_t kPlaneInf = 0x7C00u, kPlaneNegInf = 0xFC00u;  // FP16 infinit
 
 // The grid of a node whose children's (padded) boxes span mn .. mx, `size` along the longest axis: origin,
 // scale (a power of two) and the growth of the boxes in position.  Not `fits`: the extent is too large for
-// it (or infinite), and the children's planes are infinite.
+// it (or infinite), and the children's planes are infinite.  The scale then only states how large the
+// node's coordinates are, as slab_reciprocals wants it.
 struct NodeGrid {
 	float org[3], scale;
 	double slack;
@@ -78,5 +79,24 @@ DDGI_HD uint32_t child_planes(const NodeGrid& g, int axis, float lo, float hi, b
 // box be entered all the same (a ray whose distances are no numbers), a triangle of the scene is tested once
 // more, which changes no hit.
 inline uint32_t packed_code(uint32_t code) { return code == kEmptyChild ? kLeafFlag : code; }
+
+// A ray's reciprocals for the box test (inv: 1 / direction on entry; `root`: the root node's header, origin
+// and scale).  A plane's distance is fma(q, scale * inv, (org - o) * inv): while |org - o| and |plane - o|
+// are at most `reach`, reciprocals up to 3e38 / reach keep both terms finite.  Larger ones (a direction
+// component of zero, or so small that the terms would overflow: to a miss, or to infinity minus infinity)
+// are replaced by that bound, which moves the ray by less than 1e-38 reach^2 / |direction|: far less than
+// the boxes' padding of 1e-6, unless the coordinates are astronomical (from about 1e16 on, for directions of
+// length one).  There the reciprocal becomes a NaN, and the axis excludes no box: the maxima and minima of
+// the box test drop its distances.
+DDGI_HD void slab_reciprocals(const float o[3], const float root[4], float inv[3]) {
+	const float reach = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fabsf(o[2])) +
+						fmaxf(fmaxf(fabsf(root[0]), fabsf(root[1])), fabsf(root[2])) + kPlaneSteps * root[3];
+	const float least = fminf(fminf(fabsf(inv[0]), fabsf(inv[1])), fabsf(inv[2]));  // of the longest component
+	const float at_least = fmaxf(reach, 1.0f);
+	const float bound = 3e38f / at_least;
+	const float cap = reach * at_least * least <= 1e32f ? bound : NAN;
+	for(int a = 0; a < 3; ++a)
+		if(!(fabsf(inv[a]) <= bound)) inv[a] = copysignf(cap, inv[a]);
+}
 
 }  // namespace ddgi
