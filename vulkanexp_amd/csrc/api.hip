@@ -1143,6 +1143,7 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	if(e == hipSuccess) e = diff_alloc(h, &D.wt, size_t(kWeightRows) * kMaxRays * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &D.inv_sum, kBlendTexels * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &D.dirs, kMaxRays * sizeof(float4));
+	if(e == hipSuccess) e = diff_alloc(h, &D.order, kMaxRays * sizeof(uint16_t));
 	if(e == hipSuccess) e = diff_alloc(h, &D.count, 4);
 	if(e == hipSuccess) e = diff_alloc(h, &pos, N * 12);
 	if(e == hipSuccess) e = diff_alloc(h, &nrm, N * 12);
@@ -1183,8 +1184,8 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	HIP_TRY(h, hipMemcpyAsync(dep, h->dep[h->cur], P * 256 * sizeof(float2), hipMemcpyDeviceToDevice, s));
 	HIP_TRY(h, hipMemcpyAsync(states, h->states, P * 4, hipMemcpyDeviceToDevice, s));
 	const GridConst g = make_grid_const(*h);
-	{  // directions and weights kept for the context, in the order of the update's ray records
-		FrameBegin keep = frame_begin(h, R, h->perm, kBlendFP32);
+	{  // directions, order and weights kept for the context; the order is that of the update's ray records
+		FrameBegin keep = frame_begin(h, R, D.order, kBlendFP32);
 		keep.dirs = D.dirs;
 		keep.wt = D.wt;
 		keep.inv_sum = D.inv_sum;
@@ -1201,7 +1202,7 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	}
 	d.grid = g;
 	d.factors = factors;
-	d.perm = h->perm;
+	d.perm = D.order;
 	d.dirs = D.dirs;
 	d.inv_sum = D.inv_sum;
 	d.states = states;

@@ -109,6 +109,7 @@ struct Handle {
 		float* wt = nullptr;        // blend weights of the prepared frame (ray_order order)
 		float* inv_sum = nullptr;
 		float4* dirs = nullptr;
+		uint16_t* order = nullptr;  // ray order of the prepared frame (the handle's changes with every update)
 		uint32_t* count = nullptr;  // = P (all probes)
 		float2* dep_scratch = nullptr;
 		uint32_t loss_parts = 0;
