@@ -6,9 +6,10 @@
 //   rad = c0 + A (.) a[m] + (B (.) a[m] + C) (.) sun
 // Forward:  rad -> irradiance blend (FP32 kernel, irradiance only) -> sampleProbes at every
 //           G-buffer texel -> shade = out (.) a[g] * 0.996 (FinalGather.frag:62-72) -> MSE.
-// Backward: hand-written adjoint.  All reductions are deterministic: partial sums are 64-bit
-//           fixed-point integers (order-independent) combined in a fixed order.  The sampling
-//           weights (visibility, trilinear) and the blend weights are recomputed, not stored.
+// Backward: hand-written adjoint.  All reductions are deterministic: the contributions are fixed-point
+//           integers and their sums exact (order-independent).  The sampling weights (visibility,
+//           trilinear) of a texel are kept in a record by the preparation, unless there are too many
+//           texels; then they are recomputed.  The blend weights are kept.
 // G-buffer texels are binned by probe cell at prepare time, so a work item (a chunk of one cell's
 // texels) scatters into only the 8 probe tiles of that cell's cage, accumulated in LDS.
 #include "device_common.hpp"
@@ -325,14 +326,15 @@ __global__ __launch_bounds__(1024) void k_loss(DiffArgs d, uint32_t parts) {
 }
 
 // ---- backward ----
-// Contributions are held in units of 2^-50, rounded to integers, in doubles: sums of these are exact,
-// hence independent of their order, while they stay below 2^53 units (8.0; the contributions of a mean
-// over the texels are far smaller), and are rounded to 53 bits above that.
+// Contributions are rounded to integers in units of 2^-50 and their sums are exact, hence independent of
+// their order.  Those below kSmallUnits are summed in doubles (an addition there is one instruction, a
+// conversion to 64-bit integers eight): kDiffChunk of them, the most that one sum takes, stay within the
+// 2^53 to which doubles hold every integer.  Larger ones go to the 64-bit integers one by one.
 constexpr float kUnits = 1125899906842624.0f;  // 2^50
+constexpr float kSmallUnits = 8796093022208.0f;  // 2^43
+static_assert(double(kSmallUnits) * kDiffChunk <= 9007199254740992.0 && kMaxRays <= kDiffChunk, "sums in doubles are exact");
 __device__ __forceinline__ float to_units(float x) { return fminf(fmaxf(x * kUnits, -9.0e18f), 9.0e18f); }
-__device__ __forceinline__ void add_units(unsigned long long* a, double v) {
-	atomicAdd(a, (unsigned long long)(long long)(fmin(fmax(v, -9.0e18), 9.0e18)));
-}
+__device__ __forceinline__ void add_units(unsigned long long* a, double v) { atomicAdd(a, (unsigned long long)(long long)v); }
 
 // One workgroup per work item: its texels share one cage of 8 probes, whose gradient tiles it sums in
 // LDS.  A wavefront evaluates 64 texels, one per lane, and then, for each channel, turns to eight texels at
@@ -340,8 +342,9 @@ __device__ __forceinline__ void add_units(unsigned long long* a, double v) {
 // eight nearly always share their four taps (and the 64 their material), so that a lane adds its
 // contributions to registers and goes to the LDS tiles only when the taps change.  Full-HD view: 531 us
 // with 96 LDS atomics per texel, most of them 64 lanes on one address; 233 us with eight lanes per texel
-// throughout, where the evaluation is done eight times over; 110 us so (178 with the texels ordered by
-// cell only, 124 with items of 2048 texels, 195 with 4096; 5 waves per SIMD spill: 157).  Bound by vector
+// throughout, where the evaluation is done eight times over; 112 us so (as multiples of it: 1.6 with the texels ordered
+// by cell only, 1.13 with items of 2048 texels, 1.8 with 4096, 1.4 with 5 waves per SIMD, which spill; 109 us
+// when contributions too large for a sum in doubles were not told apart).  Bound by vector
 // instructions: the square roots, divisions and roundings of 96 contributions per texel.
 // four waves per SIMD: 128 VGPRs
 __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 	unsigned long long* mat = lds + 8 * 192;         // [M][3]
 	__shared__ __attribute__((aligned(16))) float s_g[kBlock / 64][64 * 8];  // gradient per (texel, probe), one channel
 	__shared__ __attribute__((aligned(16))) float s_b[kBlock / 64][64 * 4];  // tap weights per texel
-	__shared__ uint32_t s_t[kBlock / 64][64];                                // first tap, kNo: no texel
+	__shared__ uint32_t s_t[kBlock / 64][64];                                // first tap (| kLarge), kNo: no texel
 	const uint32_t item = blockIdx.x;
 	if(item >= *d.n_items) return;
 	for(uint32_t k = threadIdx.x; k < 8 * 192 + d.M * 3; k += kBlock) lds[k] = 0ull;
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 	const float inv3n = 2.0f / float(3ull * d.N);
 	const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6, i = lane & 7u;
 	unsigned long long* my_tile = tile + i * 192;
-	constexpr uint32_t kNo = 0xFFFFFFFFu;
+	constexpr uint32_t kNo = 0xFFFFFFFFu, kLarge = 64u;
 	uint32_t cur_tap = kNo, cur_mat = kNo;  // wave-uniform: what the registers hold sums of
 	double acc[4][3], macc[3];
 #pragma unroll
@@ -403,21 +406,23 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 			const float o = e.fb[ch] * e.fb[ch] * (1.0f - e.k) + e.fin[ch] * e.fin[ch] * e.k;
 			const float gs = on ? (o * a[ch] * 0.996f - d.target[x * 3 + ch]) * inv3n : 0.0f;
 			go[ch] = gs * a[ch] * 0.996f;
-			const double gm = double(rintf(to_units(gs * o * 0.996f)));
-			if(one_mat) macc[ch] += gm;
-			else if(gm != 0.0) add_units(mat + size_t(m) * 3 + ch, gm);
+			const float gm = on ? rintf(to_units(gs * o * 0.996f)) : 0.0f;
+			if(one_mat && fabsf(gm) < kSmallUnits) macc[ch] += double(gm);
+			else if(gm != 0.0f) add_units(mat + size_t(m) * 3 + ch, double(gm));
 		}
 		*reinterpret_cast<float4*>(&s_b[wave][lane * 4]) = make_float4((1.0f - c.cwx) * (1.0f - c.cwy), c.cwx * (1.0f - c.cwy),
 																	  (1.0f - c.cwx) * c.cwy, c.cwx * c.cwy);
-		s_t[wave][lane] = on ? c.t00 : kNo;
 #pragma unroll
 		for(int ch = 0; ch < 3; ++ch) {
 			// d loss / d (the probe's bilinear irradiance); sqrt'(v) taken at s >= 1e-6
 			const float df = (1.0f - e.k) * 2.0f * e.fb[ch] * e.inv_fb, dw = e.k * 2.0f * e.fin[ch] * e.inv_w;
-			float g[8];
+			float g[8], most = 0.0f;
 #pragma unroll
-			for(int p = 0; p < 8; ++p)
+			for(int p = 0; p < 8; ++p) {
 				g[p] = to_units(go[ch] * (df * c.fw[p] + dw * c.w[p]) * 0.5f / fmaxf(e.s[p][ch], 1e-6f));
+				most = fmaxf(most, fabsf(g[p]));
+			}
+			s_t[wave][lane] = on ? (most < kSmallUnits ? c.t00 : c.t00 | kLarge) : kNo;
 			float4* dst = reinterpret_cast<float4*>(&s_g[wave][lane * 8]);
 			dst[0] = make_float4(g[0], g[1], g[2], g[3]);
 			dst[1] = make_float4(g[4], g[5], g[6], g[7]);
@@ -426,11 +431,11 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 			for(uint32_t h = 0; h < 64u && k0 + h < cnt; h += 8u) {
 				const uint32_t texel = h + (lane >> 3);
 				const uint32_t t00 = s_t[wave][texel];
-				const uint32_t tap0 = uint32_t(__builtin_amdgcn_readfirstlane(int(t00)));  // the first texel exists
+				const uint32_t tap0 = uint32_t(__builtin_amdgcn_readfirstlane(int(t00))) & ~kLarge;  // the first texel exists
 				const float gv = s_g[wave][texel * 8 + i];
 				const float4 b4 = *reinterpret_cast<const float4*>(&s_b[wave][texel * 4]);
 				const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-				if(__ballot(t00 != kNo && t00 != tap0) == 0u) {
+				if(__ballot(t00 != kNo && t00 != tap0) == 0u) {  // one tap, none large
 					if(tap0 != cur_tap) {
 						flush_taps();
 						cur_tap = tap0;
@@ -441,7 +446,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_gather_bwd(DiffArgs d) {
 #pragma unroll
 					for(int q = 0; q < 4; ++q) {
 						const float v = rintf(gv * b[q]);
-						if(v != 0.0f) add_units(my_tile + tap_of(t00, q) * 3 + ch, double(v));
+						if(v != 0.0f) add_units(my_tile + tap_of(t00 & ~kLarge, q) * 3 + ch, double(v));
 					}
 				}
 			}
@@ -546,7 +551,9 @@ __global__ __launch_bounds__(kBlock) void k_blend_bwd(DiffArgs d) {
 		const float Av[3] = {A.x, A.y, A.z}, Bv[3] = {B.x, B.y, B.z}, Cv[3] = {C.x, C.y, C.z};
 		for(int ch = 0; ch < 3; ++ch) {
 			atomicAdd(&mat[m * 3 + ch], (unsigned long long)to_fixed(gr[ch] * (Av[ch] + Bv[ch] * d.sun[ch])));
-			sun[ch] += double(rintf(to_units(gr[ch] * (Bv[ch] * a[ch] + Cv[ch]))));
+			const float gs = rintf(to_units(gr[ch] * (Bv[ch] * a[ch] + Cv[ch])));
+			if(fabsf(gs) < kSmallUnits) sun[ch] += double(gs);
+			else add_units(&mat[d.M * 3 + ch], double(gs));
 		}
 	}
 #pragma unroll
