@@ -1126,11 +1126,8 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	DiffArgs d{};
 	float4* factors = nullptr;
 	float *pos, *nrm, *toc, *loss_part, *g_T;
-	float4* rec = nullptr;
 	uint32_t *gmat, *states, *indices;
 	DiffBins bins{};
-	// texels of a cell ordered by their first colour tap, unless the keys' counters grow too large
-	bins.taps = P <= (uint64_t(1) << 18) ? 64u : 1u;
 	float2* dep;
 	long long *part_tile, *part_mat_pix, *part_mat_ray, *part_rows;
 	hipError_t e = diff_alloc(h, &factors, rays * 4 * sizeof(float4));
@@ -1149,13 +1146,9 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	if(e == hipSuccess) e = diff_alloc(h, &nrm, N * 12);
 	if(e == hipSuccess) e = diff_alloc(h, &toc, N * 12);
 	if(e == hipSuccess) e = diff_alloc(h, &gmat, N * 4);
-	if(e == hipSuccess && N <= kDiffRecords) e = diff_alloc(h, &rec, N * kDiffRecRows * sizeof(float4));
 	D.loss_parts = uint32_t((N + 255) / 256);
 	if(e == hipSuccess) e = diff_alloc(h, &loss_part, size_t(D.loss_parts) * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &bins.key_of, N * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &bins.key_count, P * bins.taps * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &bins.key_start, P * bins.taps * 4);
-	if(e == hipSuccess) e = diff_alloc(h, &bins.cursor, P * bins.taps * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &bins.cell_item_start, (P + 1) * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &bins.item_begin, size_t(max_items) * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &bins.item_count, size_t(max_items) * 4);
@@ -1166,6 +1159,21 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	if(e == hipSuccess) e = diff_alloc(h, &g_T, P * 108 * 4);
 	if(e == hipSuccess) e = diff_alloc(h, &part_mat_ray, P * (M * 3 + 3) * 8);
 	if(e == hipSuccess) e = diff_alloc(h, &part_rows, size_t(kDiffSumBlocks) * (M * 3 + 3) * 8);
+	DiffSpare spare{};
+	if(e == hipSuccess) {
+		spare = diff_spare_memory(N, P, [&](size_t bytes) -> void* {
+			char* p = nullptr;
+			const hipError_t a = diff_alloc(h, &p, bytes);
+			if(a == hipErrorOutOfMemory) (void)hipGetLastError();  // the launches' checks would report it
+			else if(a != hipSuccess) e = a;
+			return p;
+		});
+		if(e == hipSuccess && !spare.keys) e = hipErrorOutOfMemory;
+	}
+	bins.taps = spare.taps;
+	bins.key_count = static_cast<uint32_t*>(spare.keys);
+	bins.key_start = bins.key_count + P * bins.taps;
+	bins.cursor = bins.key_start + P * bins.taps;
 	if(e != hipSuccess) {
 		free_diff(h);
 		return fail(h, e == hipErrorOutOfMemory ? DDGI_ERROR_OUT_OF_MEMORY : DDGI_ERROR_HIP,
@@ -1231,7 +1239,8 @@ ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const fl
 	d.part_mat_ray = part_mat_ray;
 	d.part_rows = part_rows;
 	HIP_TRY(h, diff_bin(d, bins, s));
-	if(rec) {
+	if(spare.records) {
+		float4* rec = static_cast<float4*>(spare.records);
 		HIP_TRY(h, diff_records(d, rec, s));
 		d.rec = rec;
 	}

@@ -8,8 +8,8 @@
 //           G-buffer texel -> shade = out (.) a[g] * 0.996 (FinalGather.frag:62-72) -> MSE.
 // Backward: hand-written adjoint.  All reductions are deterministic: the contributions are fixed-point
 //           integers and their sums exact (order-independent).  The sampling weights (visibility,
-//           trilinear) of a texel are kept in a record by the preparation, unless there are too many
-//           texels; then they are recomputed.  The blend weights are kept.
+//           trilinear) of a texel are kept in a record by the preparation where memory allows it, and
+//           recomputed elsewhere; the blend weights are recomputed.
 // G-buffer texels are binned by probe cell at prepare time, so a work item (a chunk of one cell's
 // texels) scatters into only the 8 probe tiles of that cell's cage, accumulated in LDS.
 #include "device_common.hpp"

@@ -1,13 +1,12 @@
 // Arguments and launchers of the differentiable probe update (diff.hip).
 #pragma once
 
+#include "diff_memory.hpp"
 #include "kernels.hpp"
 
 namespace ddgi {
 
 constexpr uint32_t kDiffChunk = 1024;  // G-buffer texels per backward work item (one cell)
-constexpr uint32_t kDiffRecRows = 5;  // float4s of a texel's sampling record
-constexpr uint64_t kDiffRecords = 12u << 20;  // most texels whose records are kept (1 GiB; a 4K view has 8.3 M)
 constexpr uint32_t kDiffSumBlocks = 64;  // workgroups that add up the material partial sums
 
 struct DiffArgs {
