@@ -7,6 +7,8 @@
 //   axis     along a coordinate axis, the other components +-0
 //   plane    one component +-0
 //   tiny     along a coordinate axis, the others of magnitude 1e-44 .. 1e-25
+//   none     without a direction: all components +-0
+//   infinite from a point with one infinite coordinate, every other one along another axis
 //   far      from REACH away (and above) toward the scene's triangles
 // from origins inside the scene's bounds (not farther than REACH from 0) unless far.
 // Prints: rays hits mismatches-to-every-triangle packed-visits fp32-visits most-packed-visits
@@ -243,6 +245,9 @@ int main(int argc, char** argv) {
 			if(mode == "axis") r.d[a] = float(sign * (a == axis ? 1.0 : 0.0));
 			if(mode == "plane" && a == axis) r.d[a] = float(sign * 0.0);
 			if(mode == "tiny") r.d[a] = float(sign * (a == axis ? 1.0 : std::pow(10.0, -44.0 + 19.0 * e)));
+			if(mode == "none") r.d[a] = float(sign * 0.0);
+			if(mode == "infinite" && a == axis) r.o[a] = float(sign) * INFINITY;
+			if(mode == "infinite" && q % 2) r.d[a] = float(sign * (a == (axis + 1) % 3 ? 1.0 : 0.0));
 			// toward the triangle, within a tenth of the distance by which the box test widens a box's exit
 			if(mode == "far") {
 				const double to = at[a] + 1e-7 * reach * (2.0 * e - 1.0);

@@ -78,6 +78,14 @@ def test_directions_with_components_near_zero(checker, tmp_path, name, mode):
         assert packed <= 1.25 * fp32
 
 
+@pytest.mark.parametrize("mode", ["none", "infinite"])
+@pytest.mark.parametrize("name", ["room", "clustered"])
+def test_rays_that_hit_nothing_end_early(checker, tmp_path, name, mode):
+    n, hits, bad, packed, fp32, most = _trace(checker, tmp_path, SCENES[name](), mode, 400)
+    assert hits == 0 and bad == 0
+    assert packed <= 1.25 * fp32
+
+
 def _details(size):
     """A 200 m ground and details on it, each of seven triangles of extent `size`."""
     sb = scenes.SceneBuilder()

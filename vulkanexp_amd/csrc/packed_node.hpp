@@ -87,14 +87,18 @@ inline uint32_t packed_code(uint32_t code) { return code == kEmptyChild ? kLeafF
 // are replaced by that bound, which moves the ray by less than 1e-38 reach^2 / |direction|: far less than
 // the boxes' padding of 1e-6, unless the coordinates are astronomical (from about 1e16 on, for directions of
 // length one).  There the reciprocal becomes a NaN, and the axis excludes no box: the maxima and minima of
-// the box test drop its distances.
+// the box test drop its distances.  A ray without a direction (all reciprocals infinite) hits nothing; it
+// keeps the bound, and so only the boxes around its origin.  A ray from infinity enters no box with any
+// finite reciprocal.
 DDGI_HD void slab_reciprocals(const float o[3], const float root[4], float inv[3]) {
-	const float reach = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fabsf(o[2])) +
+	const float from = fmaxf(fmaxf(fabsf(o[0]), fabsf(o[1])), fabsf(o[2]));
+	const float reach = (from < INFINITY ? from : 0.0f) +
 						fmaxf(fmaxf(fabsf(root[0]), fabsf(root[1])), fabsf(root[2])) + kPlaneSteps * root[3];
-	const float least = fminf(fminf(fabsf(inv[0]), fabsf(inv[1])), fabsf(inv[2]));  // of the longest component
 	const float at_least = fmaxf(reach, 1.0f);
+	if(fmaxf(fmaxf(fabsf(inv[0]), fabsf(inv[1])), fabsf(inv[2])) * at_least <= 3e38f) return;  // nearly every ray
+	const float least = fminf(fminf(fabsf(inv[0]), fabsf(inv[1])), fabsf(inv[2]));  // of the longest component
 	const float bound = 3e38f / at_least;
-	const float cap = reach * at_least * least <= 1e32f ? bound : NAN;
+	const float cap = reach * at_least * least <= 1e32f || least == INFINITY ? bound : NAN;
 	for(int a = 0; a < 3; ++a)
 		if(!(fabsf(inv[a]) <= bound)) inv[a] = copysignf(cap, inv[a]);
 }
