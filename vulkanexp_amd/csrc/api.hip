@@ -822,7 +822,7 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	sd.instance_count = uint32_t(instance_count);
 	sd.stack_depth = 3 * bvh.wide_depth;  // entries the traversal can hold at once
 	h->sd = sd;
-	h->bvh_bytes = bvh.nodes.size() * 4 + bvh.tris.size() * 4;
+	h->bvh_bytes = size_t(bvh.node_count) * kPackedNodeBytes + bvh.tris.size() * 4;
 	bvh.nodes.clear();
 	bvh.tris.clear();
 	bvh.obj_tris.clear();
