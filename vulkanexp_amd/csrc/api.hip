@@ -252,8 +252,7 @@ bool instance_dev(const ddgi_instance& in, const float* M, uint32_t prim_base, I
 void node_ranges(const BvhHost& bvh, std::vector<uint32_t>& range, std::vector<uint32_t>& codes) {
 	range.assign(size_t(bvh.node_count) * 8, 0u);
 	codes.resize(size_t(bvh.node_count) * 4);
-	for(size_t q = bvh.level_nodes.size(); q-- > 0;) {  // deepest level first
-		const size_t w = bvh.level_nodes[q];
+	for(size_t w = bvh.node_count; w-- > 0;) {  // children have higher indices than their parent
 		for(uint32_t k = 0; k < kWide; ++k) {
 			uint32_t code;
 			std::memcpy(&code, &bvh.nodes[w * kNodeFloats + kCodeRow + k], 4);
@@ -820,7 +819,6 @@ ddgi_status ddgi_set_scene(void* handle, const ddgi_vertex* vertices, size_t ver
 	sd.tri_count = bvh.tri_count;
 	sd.node_count = bvh.node_count;
 	sd.instance_count = uint32_t(instance_count);
-	sd.stack_depth = 3 * bvh.wide_depth;  // entries the traversal can hold at once
 	h->sd = sd;
 	h->bvh_bytes = size_t(bvh.node_count) * kPackedNodeBytes + bvh.tris.size() * 4;
 	bvh.nodes.clear();

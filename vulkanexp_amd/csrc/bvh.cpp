@@ -538,7 +538,7 @@ static void emit_tree(const std::vector<float>& world, const std::vector<float>&
 		uint32_t depth;
 		int32_t kids[kWide];  // binary child nodes, -1 = empty slot
 	};
-	// depth first: the children of a node get consecutive indices, then each child's subtree in turn
+	// depth first: the children of a node get consecutive indices above its own, then each child's subtree in turn
 	Wide root{0, 1, {}};
 	for(uint32_t k = 0; k < kWide; ++k) root.kids[k] = -1;
 	std::vector<Wide> wide{root};
@@ -592,15 +592,6 @@ static void emit_tree(const std::vector<float>& world, const std::vector<float>&
 		}
 	}
 	out.node_count = uint32_t(wide.size());
-	// nodes by level, for bottom-up refits
-	out.level_offsets.assign(wide_depth + 1, 0);
-	for(const Wide& w : wide) ++out.level_offsets[w.depth];
-	for(uint32_t d = 1; d <= wide_depth; ++d) out.level_offsets[d] += out.level_offsets[d - 1];
-	out.level_nodes.resize(wide.size());
-	{
-		std::vector<uint32_t> fill(out.level_offsets.begin(), out.level_offsets.end() - 1);
-		for(size_t w = 0; w < wide.size(); ++w) out.level_nodes[fill[wide[w].depth - 1]++] = uint32_t(w);
-	}
 	// SAH cost of the emitted tree (for reporting)
 	double cost = 0.0;
 	const double root_area = std::max(b.nodes[0].box.half_area(), 1e-30);

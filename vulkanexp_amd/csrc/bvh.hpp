@@ -2,7 +2,7 @@
 // (src/Renderer.cpp:272-449, :525-642).  Instances are flattened into world space at build time,
 // so traversal is single-level.
 //
-// Device layout (all float4 / 16-byte aligned, accessed 16 bytes at a time):
+// Layout (all float4 / 16-byte aligned):
 //   node k  : kNodeFloats floats, a kWide-wide node collapsed from the binary SAH tree, holding the
 //             boxes of its (up to) kWide children side by side so that one node fetch tests all of
 //             them, in rows of kWide floats (one float4 per 4 children):
@@ -10,14 +10,15 @@
 //               row 3 = hi.y                          row 4 = lo.z   row 5 = hi.z
 //               row 6 = child codes as int bits: inner node index, or
 //                       leaf = 0x80000000 | first_triangle << 3 | (count - 1), or kEmptyChild
-//             then padding (4-wide: 128 bytes, 8-wide: 256 bytes)
+//             then padding (128 bytes); a child's index is above its parent's
 //   triangle: 3 float4 = 48 bytes, leaf order (a slot; a triangle cut by spatial splits fills one
 //             slot per piece, each a full copy of the triangle whose leaf box bounds only its piece):
 //               [0] = (v0.xyz, global triangle id)   global id = instance-major flattened index
 //               [1] = (v1.xyz, instance index)
 //               [2] = (v2.xyz, mask | flip_facing << 8)
-// The traversal reads the nodes in a packed form made on the device from the slots' boxes (k_make_nodes,
-// kPackedNodeBytes each, the same node indices and child codes).
+// The device holds the triangles as they are, and of the nodes a packed form, made there from the slots'
+// boxes (k_make_nodes, kPackedNodeBytes each, the same node indices): of these records it uses the codes.
+// The boxes here are the reference that the packed ones are checked against.
 // Node boxes are inflated by a few ulps so that FP32 slab tests stay conservative; an empty child
 // slot has the code kEmptyChild and a point box far outside any scene.
 #pragma once
@@ -35,10 +36,10 @@ constexpr uint32_t kMaxLeafSize = 8;
 // children per node: 4 (8-wide nodes visit 26 % fewer nodes per probe ray but trace slower: the
 // wider fetch, slab tests and sorting network cost registers and occupancy)
 constexpr uint32_t kWide = 4;
-constexpr uint32_t kNodeFloats = kWide == 4 ? 32 : 64;  // 6 box rows + 1 code row of kWide, padded
+constexpr uint32_t kNodeFloats = 32;     // 6 box rows + 1 code row of kWide, padded
 constexpr uint32_t kCodeRow = 6 * kWide;               // float offset of the child codes
 constexpr uint32_t kMaxWideDepth = 32;   // traversal stack: kWide - 1 entries per level
-static_assert(kWide == 4 || kWide == 8, "nodes are 4- or 8-wide");
+static_assert(kWide == 4, "the traversal and its packed nodes are 4-wide");
 constexpr uint32_t kPackedNodeBytes = 80;  // the traversal's form of a 4-wide node (trace.hip, k_make_nodes)
 
 struct BvhHost {
@@ -50,16 +51,12 @@ struct BvhHost {
 	uint32_t max_depth = 0;       // binary tree
 	uint32_t wide_depth = 0;      // levels of the wide tree
 	double sah_cost = 0.0;
-	// for refits after instance moves: object-space vertices of each triangle slot (9 floats, leaf
-	// order) and the wide nodes grouped by depth (level d = nodes level_nodes[level_offsets[d-1] ..
-	// level_offsets[d]), root at level 1)
+	// for refits after instance moves: object-space vertices of each triangle slot (9 floats, leaf order)
 	std::vector<float> obj_tris;
 	// per slot the bounds of the part of its triangle that the slot holds (the whole triangle, or
 	// the piece a spatial split left there; 6 floats: lo xyz, hi xyz), which a refit keeps for
 	// instances that have not moved
 	std::vector<float> slot_box;
-	std::vector<uint32_t> level_nodes;
-	std::vector<uint32_t> level_offsets;
 };
 
 // Box padding of the device layout: the float just below v - (|v| 1e-6 + 1e-6) and just above

@@ -185,7 +185,6 @@ template <bool ANY, int STACK, int STRIDE, bool COUNT = false, bool CULL = false
 __device__ __forceinline__ HitResult traverse(const float4* __restrict__ nodes, const float4* __restrict__ tris,
 											  const RayPrep& r, float tmin, float tmax, uint32_t mask,
 											  uint32_t* stack, uint32_t& n_nodes_out, uint32_t& n_tris_out) {
-	static_assert(kWide == 4, "packed nodes are 4-wide");
 	HitResult best;
 	best.t = tmax;
 	best.slot = 0xFFFFFFFFu;

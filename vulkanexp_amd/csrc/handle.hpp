@@ -37,10 +37,10 @@ struct Handle {
 	bool indices_are_iota = false;
 	float4* rays = nullptr;
 	float4* hits = nullptr;
-	uint32_t* shade_list = nullptr;   // P * max_rays entries
-	uint32_t* shade_count = nullptr;  // [0] shade list, [kMissCountSlot] miss list
+	uint32_t* shade_list = nullptr;   // kShadeSegments segments, P * max_rays + kShadeSegments * kMaxItemThreads entries
+	uint32_t* shade_count = nullptr;  // kListCounterBytes: the segments' counters, miss list, ordered length, blend's done
 	uint32_t* miss_list = nullptr;    // P * max_rays entries, allocated with the atmospheric sky
-	uint32_t* shade_keys = nullptr;   // P * max_rays: cell key of each shade-list entry
+	uint32_t* shade_keys = nullptr;   // as shade_list: cell key of each entry
 	uint32_t* sort_keys = nullptr;    // P * max_rays: keys / entries bucketed by coarse digit
 	uint32_t* sort_list = nullptr;
 	uint32_t* sort_counts = nullptr;  // kShadeSortCounts
@@ -111,7 +111,6 @@ struct Handle {
 		float4* dirs = nullptr;
 		uint16_t* order = nullptr;  // ray order of the prepared frame (the handle's changes with every update)
 		uint32_t* count = nullptr;  // = P (all probes)
-		float2* dep_scratch = nullptr;
 		uint32_t loss_parts = 0;
 	} diff;
 };

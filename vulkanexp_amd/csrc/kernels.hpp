@@ -66,7 +66,6 @@ struct SceneDev {
 	uint32_t tri_count;
 	uint32_t node_count;
 	uint32_t instance_count;
-	uint32_t stack_depth;      // most stack entries a traversal needs (3 per level of the 4-wide tree)
 };
 
 // One moved instance: its transform, its motion since the BVH was built (both row-major 3x4), the triangle

@@ -159,7 +159,8 @@ __device__ __forceinline__ void trace_primary_ray(const TraceFrameArgs& a, uint3
 }
 
 template <int STACK, bool COUNT>
-// eight waves per SIMD (64 VGPRs, no spills): 0.559 ms, against 0.580 at 7 and 0.617 at 6
+// eight waves per SIMD (64 VGPRs; five values spill outside the loop over nodes): 0.559 ms, against 0.580 at 7
+// and 0.617 at 6
 __global__ __launch_bounds__(kPrimaryBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_trace_primary(TraceFrameArgs a) {
 	__shared__ uint32_t stack[STACK * kPrimaryBlock];
 	if(a.stamps && blockIdx.x == 0 && threadIdx.x == 0) a.stamps[1] = wall_clock64();
