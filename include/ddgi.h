@@ -387,13 +387,13 @@ ddgi_status ddgi_reflection_noalloc(void* handle, const ddgi_gbuffer_texel* gbuf
  *   DDGI_UPDATE_ALL_PROBES) and keeps what the parameters do not change: ray hits and shading
  *   factors, the irradiance atlas before the update, the depth atlas and the probe states after
  *   it, and the G-buffer (device arrays: position/normal/to_camera float[3*count], material
- *   uint32[count], copied).  Requires non-metallic materials (radiance is then affine in albedo
- *   and sun); material_count (<= 1024) albedo slots, every material id < material_count.
+ *   uint32[count], copied).  Updates of the handle afterwards do not change the context.  Requires
+ *   non-metallic materials (radiance is then affine in albedo and sun); material_count (<= 1024) albedo slots, every material id < material_count.
  * ddgi_diff_forward: device albedo float[3*material_count], sun float[3], target float[3*count]
  *   -> shade_out float[3*count], loss_out float[1].
  * ddgi_diff_backward: differentiates the most recent ddgi_diff_forward of the handle (same albedo,
  *   sun, target); grad_loss float[1] is d(total)/d(loss); writes grad_albedo float[3*material_count]
- *   and grad_sun float[3].  Deterministic (fixed-point reductions). */
+ *   and grad_sun float[3].  Deterministic (exact fixed-point sums, independent of the texels' order). */
 ddgi_status ddgi_diff_prepare(void* handle, const float orientation[9], const float* gbuf_position,
 							  const float* gbuf_normal, const float* gbuf_to_camera, const uint32_t* gbuf_material,
 							  uint64_t texel_count, uint32_t material_count, void* stream);

@@ -1139,8 +1139,8 @@ __global__ void k_apply_moves(const InstanceMove* __restrict__ staged, InstanceM
 // boxes tight enough that no more nodes are visited).  A plane is origin + q * scale; the traversal's
 // distance fma(q, scale / d, (origin - o) / d) is off by at most about 2.4e-7 of the node's size (in
 // position) beside the errors relative to the distance that the far end's widening covers, so the padded
-// boxes are first grown by 1e-6 of that size.  A node too large
-// for the grid gets infinite boxes (node_grid and child_planes).
+// boxes are first grown by 1e-6 of that size.  A node too large for the grid gets infinite boxes (node_grid
+// and child_planes).  The planes are bounds only: no result is computed from them.
 // 32 lanes per node, eight per child: `range` holds each child's triangle slots (first, end), and lane j of
 // a child takes the j-th box of either end of its range on every level.
 __global__ __launch_bounds__(256) void k_make_nodes(BoxTree tree, const uint2* __restrict__ range,
