@@ -388,7 +388,8 @@ ddgi_status ddgi_reflection_noalloc(void* handle, const ddgi_gbuffer_texel* gbuf
  *   factors, the irradiance atlas before the update, the depth atlas and the probe states after
  *   it, and the G-buffer (device arrays: position/normal/to_camera float[3*count], material
  *   uint32[count], copied).  Updates of the handle afterwards do not change the context.  Requires
- *   non-metallic materials (radiance is then affine in albedo and sun); material_count (<= 1024) albedo slots, every material id < material_count.
+ *   non-metallic materials (radiance is then affine in albedo and sun); material_count (<= 1024)
+ *   albedo slots, every material id < material_count.
  * ddgi_diff_forward: device albedo float[3*material_count], sun float[3], target float[3*count]
  *   -> shade_out float[3*count], loss_out float[1].
  * ddgi_diff_backward: differentiates the most recent ddgi_diff_forward of the handle (same albedo,
